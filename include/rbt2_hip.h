@@ -80,7 +80,10 @@ int rbt_hip_set_router_order(rbt_hip *h, int order);
  *                         weights: (token, slot) pairs dispatched into per-expert lists and the
  *                         expert FFN run as grouped GEMMs on the matrix cores, each expert's weights
  *                         read once per call. Smaller T runs one GEMV per pair. Routing is the same
- *                         either way; outputs agree within the parity tolerance.
+ *                         either way; outputs agree within the parity tolerance. f32 weights, and bf16
+ *                         weights whose dims the bf16 tiles do not divide, have a grouped form of their
+ *                         own at full f32 activation precision; it is taken where it is faster (by
+ *                         size), or from this many tokens (and at least 2) on once the option is set.
  *   "prefill_layout"      1 (default): the grouped GEMMs read a layer's tiled expert copy where the
  *                         caller made one with rbt_hip_prefill_layout (none exists otherwise: by
  *                         default every kernel reads the .rbt2 blobs); 0: the blobs only.
@@ -156,7 +159,8 @@ int rbt_hip_reserve(rbt_hip *h, const rbt_moe_layer *L, int max_tokens);
 
 /* rbt_hip_moe_dev that allocates nothing (no counterpart in the reference; for callers that cannot
  * allocate device memory: code under HIP graph capture, tight serving loops, hosts that forbid it).
- * Same arguments, kernels and results as rbt_hip_moe_dev, but the workspace is a fixed 64 MiB scratch
+ * Same arguments, kernels and results as rbt_hip_moe_dev (except that where the full-precision grouped
+ * form's buffers do not fit, the per-pair GEMVs run instead), but the workspace is a fixed 64 MiB scratch
  * array the library holds on each GPU until the process ends, instead of the handle's workspace: calls
  * whose workspace would exceed it fail with a message (a 512-token call at the OLMoE layer shape needs
  * 52.2 MiB). No profiling events are taken. Every call on one GPU shares that GPU's array, so calls

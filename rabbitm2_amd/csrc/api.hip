@@ -132,6 +132,7 @@ struct rbt_hip {
     Sampling sampling;     // rbt_hip_set_sampling: how rbt_hip_generate* pick tokens
     uint64_t seed = 0;
     int prefill_min_tokens = kPrefillMinTokensDefault;  // option "prefill_min_tokens"
+    bool prefill_min_set = false;                        // the caller chose it
     int prefill_tile_rows = 0;  // option "prefill_tile_rows": rows per grouped-GEMM tile, 0 = by batch
     bool prefill_wide = true;   // option "prefill_wide": 128-row tiles 512 weight rows wide
     int gen_timed_from = 1;     // option "generate_timed_from": first generated step of ms_out[1]
@@ -363,6 +364,7 @@ void ws_release(Workspace &w) {
 // Grows the workspace to hold T tokens of this shape (never shrinks). Allocation happens only here.
 int ws_reserve(rbt_hip *h, int T, int E, int K, int H) {
     Workspace &w = h->ws;
+    H = full_h_stride(H);  // the h rows of the full-precision grouped form are padded
     if (T <= w.tokens && E <= w.E && K <= w.K && H <= w.H) return 1;
     const int nT = T > w.tokens ? T : w.tokens, nE = E > w.E ? E : w.E, nK = K > w.K ? K : w.K,
               nH = H > w.H ? H : w.H;
@@ -870,10 +872,18 @@ int capture_step(rbt_hip *h, bool final, hipGraphExec_t *exec) {
     return 1;
 }
 
+// Whether T tokens take the full-precision grouped form by size: where it beats the per-pair GEMVs, or from
+// the caller's own "prefill_min_tokens" on.
+bool full_from(const rbt_hip *h, int dtype, int T, int E, int K, int D, int H, const void *experts, uint64_t stride,
+               const float *xb) {
+    if (h->prefill_min_set) return T >= h->prefill_min_tokens;
+    return full_pays(experts_decode_supported(dtype, T, K, D, H, experts, stride, xb, xb), dtype, T, E, K, D, H);
+}
+
 // The form the MoE block takes for a call: the batch-1 kernels with the top-k inside gate/up, the
-// grouped GEMM path, or the per-pair GEMVs. (Both workspaces give the h buffer 256-byte alignment, so
-// the decode kernels' alignment test sees xb's, which it also checks.)
-enum MoeForm { kMoeFastDecode, kMoeGrouped, kMoeGeneral };
+// grouped GEMM path, its full-precision form, or the per-pair GEMVs. (Both workspaces give the h buffer
+// 256-byte alignment, so the decode kernels' alignment test sees xb's, which it also checks.)
+enum MoeForm { kMoeFastDecode, kMoeGrouped, kMoeGroupedFull, kMoeGeneral };
 MoeForm moe_form(const rbt_hip *h, const rbt_moe_layer *L, int T, const float *xb) {
     if (T == 1 && h->fused_decode && L->n_experts <= kTopkInGateupMaxE &&
         experts_decode_supported(L->dtype, T, L->top_k, L->dim, L->expert_hidden, L->experts, L->expert_stride, xb,
@@ -882,28 +892,37 @@ MoeForm moe_form(const rbt_hip *h, const rbt_moe_layer *L, int T, const float *x
     if (prefill_supported(L->dtype, T, h->prefill_min_tokens, L->n_experts, L->top_k, L->dim, L->expert_hidden,
                           L->experts, L->expert_stride, xb))
         return kMoeGrouped;
+    if (T > 1 && full_from(h, L->dtype, T, L->n_experts, L->top_k, L->dim, L->expert_hidden, L->experts, L->expert_stride,
+                           xb) &&
+        full_supported(L->dtype, T, L->n_experts, L->top_k, L->dim, L->expert_hidden, L->experts, L->expert_stride, xb))
+        return kMoeGroupedFull;
     return kMoeGeneral;
+}
+
+// Bytes of the grouped lists and buffers (Workspace::pre) that a form needs.
+size_t pre_bytes_of(MoeForm form, int T, int E, int K, int D) {
+    return form == kMoeGrouped ? prefill_workspace_bytes(T, E, K, D)
+                               : form == kMoeGroupedFull ? full_workspace_bytes(T, E, K, D) : 0;
 }
 
 size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
-// Scratch bytes of one MoE call: probs [T][E], routing and weights [T][K], hbuf [T*K][H], and the
-// grouped path's lists, down outputs and activation planes.
-size_t moe_scratch_bytes(int T, int E, int K, int H, int D, bool grouped) {
-    const size_t t = (size_t)T;
-    return up256(4 * t * E) + 2 * up256(4 * t * K) + up256(4 * t * K * H) +
-           (grouped ? prefill_workspace_bytes(T, E, K, D) : 0);
+// Scratch bytes of one MoE call: probs [T][E], routing and weights [T][K], hbuf [T*K][H] (rows padded in
+// the full-precision grouped form), and the grouped forms' lists, down outputs and activation planes.
+size_t moe_scratch_bytes(int T, int E, int K, int H, int D, MoeForm form) {
+    const size_t t = (size_t)T, hs = (size_t)(form == kMoeGroupedFull ? full_h_stride(H) : H);
+    return up256(4 * t * E) + 2 * up256(4 * t * K) + up256(4 * t * K * hs) + pre_bytes_of(form, T, E, K, D);
 }
 
 // A workspace view of the scratch array (device address `base`), in moe_scratch_bytes' order.
-Workspace scratch_view(void *base, int T, int E, int K, int H, int D, bool grouped) {
+Workspace scratch_view(void *base, int T, int E, int K, int H, int D, MoeForm form) {
     uint8_t *p = static_cast<uint8_t *>(base);
-    const size_t t = (size_t)T;
+    const size_t t = (size_t)T, hs = (size_t)(form == kMoeGroupedFull ? full_h_stride(H) : H);
     Workspace w;
     w.tokens = T;
     w.E = E;
     w.K = K;
-    w.H = H;
+    w.H = (int)hs;
     w.probs = reinterpret_cast<float *>(p);
     p += up256(4 * t * E);
     w.routing = reinterpret_cast<int32_t *>(p);
@@ -911,9 +930,9 @@ Workspace scratch_view(void *base, int T, int E, int K, int H, int D, bool group
     w.weights = reinterpret_cast<float *>(p);
     p += up256(4 * t * K);
     w.hbuf = reinterpret_cast<float *>(p);
-    p += up256(4 * t * K * H);
-    w.pre = grouped ? p : nullptr;
-    w.pre_bytes = grouped ? prefill_workspace_bytes(T, E, K, D) : 0;
+    p += up256(4 * t * K * hs);
+    w.pre_bytes = pre_bytes_of(form, T, E, K, D);
+    w.pre = w.pre_bytes ? p : nullptr;
     return w;
 }
 
@@ -976,6 +995,14 @@ int moe_block(rbt_hip *h, const rbt_moe_layer *L, const float *xb_dev, int T, fl
     HIP_OK(h, launch_router(lc(h, kProfRouter), lc(h, kProfTopk), h->order, L->dtype, xb_dev, L->router,
                             L->router_bias, T, L->n_experts, L->dim, L->top_k, L->norm_topk, w.probs, routing,
                             weights));
+    if (form == kMoeGroupedFull) {
+        int32_t *counts = nullptr;
+        HIP_OK(h, launch_grouped_full(lc(h, kProfDispatch), lc(h, kProfGateup), lc(h, kProfDown), lc(h, kProfCombine),
+                                      L->dtype, L->experts, L->expert_stride, xb_dev, T, L->n_experts, L->top_k, L->dim,
+                                      L->expert_hidden, routing, weights, w.hbuf, w.pre, x_dev, moe_dev, &counts));
+        h->expert_counts = counts;
+        return done();
+    }
     if (decode_kernels) {
         HIP_OK(h, launch_experts_decode(lc(h, kProfGateup), lc(h, kProfDown), L->dtype, L->experts, L->expert_stride,
                                         routing, weights, xb_dev, w.hbuf, T, L->top_k, L->dim, L->expert_hidden, x_dev,
@@ -1272,7 +1299,9 @@ int rbt_hip_reserve(rbt_hip *h, const rbt_moe_layer *L, int max_tokens) {
     if (max_tokens < 0) return fail(h, "reserve: negative token count");
     const int T = max_tokens > 0 ? max_tokens : 1;
     if (!ws_reserve(h, T, L->n_experts, L->top_k, L->expert_hidden)) return 0;
-    if (T >= h->prefill_min_tokens)
+    // the larger of the two grouped forms' (it adds the activation planes), for any alignment of the rows
+    if (T >= h->prefill_min_tokens ||
+        full_from(h, L->dtype, T, L->n_experts, L->top_k, L->dim, L->expert_hidden, L->experts, 1, nullptr))
         return pre_reserve(h, prefill_workspace_bytes(T, L->n_experts, L->top_k, L->dim));
     return 1;
 }
@@ -1287,7 +1316,7 @@ int rbt_hip_moe_dev(rbt_hip *h, const rbt_moe_layer *L, const float *xb_dev, int
     if (!set_device(h)) return 0;
     if (!ws_reserve(h, T, L->n_experts, L->top_k, L->expert_hidden)) return 0;
     const MoeForm form = moe_form(h, L, T, xb_dev);
-    if (form == kMoeGrouped && !pre_reserve(h, prefill_workspace_bytes(T, L->n_experts, L->top_k, L->dim))) return 0;
+    if (!pre_reserve(h, pre_bytes_of(form, T, L->n_experts, L->top_k, L->dim))) return 0;
     return moe_block(h, L, xb_dev, T, x_dev, moe_dev, routing_dev, weights_dev, h->ws, form, true);
 }
 
@@ -1299,13 +1328,17 @@ int rbt_hip_moe_dev_noalloc(rbt_hip *h, const rbt_moe_layer *L, const float *xb_
     if (T == 0) return 1;
     if (!xb_dev) return fail(h, "moe_noalloc: xb is NULL");
     if (!h->scratch) return fail(h, "moe_noalloc: no scratch address for device %d", h->device);
-    const MoeForm form = moe_form(h, L, T, xb_dev);
-    const size_t need = moe_scratch_bytes(T, L->n_experts, L->top_k, L->expert_hidden, L->dim, form == kMoeGrouped);
+    MoeForm form = moe_form(h, L, T, xb_dev);
+    size_t need = moe_scratch_bytes(T, L->n_experts, L->top_k, L->expert_hidden, L->dim, form);
+    if (form == kMoeGroupedFull && need > kScratchBytes) {  // the GEMVs need less, and run wherever they did
+        form = kMoeGeneral;
+        need = moe_scratch_bytes(T, L->n_experts, L->top_k, L->expert_hidden, L->dim, form);
+    }
     if (need > kScratchBytes)
         return fail(h, "moe_noalloc: %d tokens of this layer need %zu bytes of scratch, above its %zu bytes", T, need,
                     (size_t)kScratchBytes);
     if (!set_device(h)) return 0;
-    Workspace w = scratch_view(h->scratch, T, L->n_experts, L->top_k, L->expert_hidden, L->dim, form == kMoeGrouped);
+    Workspace w = scratch_view(h->scratch, T, L->n_experts, L->top_k, L->expert_hidden, L->dim, form);
     return moe_block(h, L, xb_dev, T, x_dev, moe_dev, routing_dev, weights_dev, w, form, false);
 }
 
@@ -1462,6 +1495,7 @@ int rbt_hip_set_option(rbt_hip *h, const char *name, int64_t value) {
     } else if (strcmp(name, "prefill_min_tokens") == 0) {
         if (value < 1 || value > 65536) return fail(h, "set_option: prefill_min_tokens must be in [1, 65536]");
         h->prefill_min_tokens = (int)value;
+        h->prefill_min_set = true;
     } else if (strcmp(name, "prefill_tile_rows") == 0) {
         if (value != 0 && value != 32 && value != 64 && value != 128)
             return fail(h, "set_option: prefill_tile_rows must be 0, 32, 64 or 128");

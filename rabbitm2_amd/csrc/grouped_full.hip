@@ -1,0 +1,440 @@
+// The expert FFN of many tokens at full f32 activation precision: the grouped form for f32 weights, and
+// for bf16 weights of dims that the tiles of prefill.hip do not divide. (Those would otherwise run one
+// GEMV per (token, slot) pair, reading an expert's weights once per pair instead of once per call.)
+//
+// Reference semantics: rabbit2/src/rabbit2.c:531-542 for every token: h = silu(W1 xb) * (W3 xb),
+// tmp = W2 h, moe += w_k * tmp in selection order, x += moe; blobs w1[H][D] | w3[H][D] | w2[D][H] (:173).
+//
+// The lists, their order and the combine are prefill.hip's; the two GEMMs are grouped_full_kernel's.
+#include <math.h>
+
+#include <type_traits>
+
+#include "rbt2_internal.h"
+
+namespace rbt {
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kFullWaves = 4, kFullAhead = 3;  // waves per block; k-steps of weights in flight ahead
+constexpr int kFullWin = 128;                  // bytes of a weight row per k-step
+
+struct FullArgs {
+    const uint8_t *experts;
+    uint64_t stride, w_off, w3_off;
+    int N, Kd;             // output columns, reduction length
+    const float *act;      // activation rows, act_stride floats apart, zeros from Kd to the next multiple of 4
+    int act_stride, gather;
+    const int32_t *perm;
+    int topk;
+    const int32_t *counts, *offsets, *m_off, *choice;  // choice: the dispatch's plan (bit 1: column-major slots)
+    int E;
+    float *out;            // output rows in list order, out_stride floats apart
+    int out_stride;
+};
+
+// x = hi + mid + lo exactly, each part a bf16 (its upper 16 bits): 8 + 8 + 8 bits of the significand by
+// truncation. A non-finite x is its own hi part (a NaN made quiet, so that truncation keeps it one).
+__device__ __forceinline__ void split3(float x, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
+    const uint32_t u = __float_as_uint(x);
+    const bool fin = (u & 0x7F800000u) != 0x7F800000u;
+    hi = x != x ? (u | 0x00400000u) & 0xFFFF0000u : u & 0xFFFF0000u;
+    const float r1 = fin ? x - __uint_as_float(hi) : 0.0f;
+    mid = __float_as_uint(r1) & 0xFFFF0000u;
+    lo = __float_as_uint(r1 - __uint_as_float(mid)) & 0xFFFF0000u;
+}
+__device__ __forceinline__ uint32_t pack_hi16(uint32_t a, uint32_t b) { return (a >> 16) | (b & 0xFFFF0000u); }
+
+// One tile: 16 RG list rows x 16 columns of W1 and of W3 per wave (MATS = 2: h = silu(W1 a) * (W3 a), 64
+// columns per block) or 32 columns of W2 (MATS = 1: y = W2 a, 128 columns per block).
+//
+// Weights go from HBM into registers in the operands' order (blob_operands: whole 128-byte lines of the
+// row-major blobs), kFullAhead k-steps of 128 bytes per row ahead, each weight byte once per tile. The f32
+// activation rows are loaded four steps ahead (buffer loads: rows past the list and columns past the row
+// read as zeros without a request) and pass through a two-stage LDS ring that all waves read. Products:
+//   bf16 weights: the activation as three bf16 parts that carry all 24 bits (split on the way into LDS),
+//     three v_mfma_f32_16x16x32_bf16 per 32 columns; every product is exact in the f32 accumulator;
+//   f32 weights: v_mfma_f32_16x16x4_f32.
+// The sums are no further from 64 bits than the GEMVs' lanes and trees: bf16, a step's products are summed
+// from zero (the small parts first), eight steps' sums are added up, and those to the running sums; f32,
+// 16 columns' products are summed from zero and added to the running sums, which carry their rounding
+// errors along. The tile order and the rotation of the k-steps by weight tile are
+// prefill.hip's (the row tiles of a weight tile run together on one XCD and stay in step).
+// Bound: short lists by the weight stream (dim 2048, 64 experts, top-8, hidden 1024, f32: 12 tokens, about
+// 51 experts, 161 + 86 us, 5.2 TB/s; 200 tokens, two row groups per tile, 309 + 160 us against 3936 + 1939
+// us of per-pair GEMVs, of which the compensated sums take 58 + 26); long ones by the wave's own chain of
+// LDS reads and products (bf16, dim 1600, 40 experts of 150 rows, hidden 800: 210 + 120 us, 440 TFLOP/s
+// issued). Four waves per block, two blocks per CU: with eight-wave blocks (one per CU) every wave waits at
+// each step's barrier, 22 + 27 against 17 + 17 us at dim 1000, hidden 330, 50 tokens; activations one step
+// ahead instead of four: 26 + 31 us; tiles of 128 rows and eight waves: 307 against 217 us on the 150-row
+// lists (spills).
+// GR: bytes per weight load, from the rows' alignment (16, 4 or 2); the last k-step of a row may be
+// partial: its loads are clamped into the row and the parts past the end set to zero.
+template <int DT, int MATS, int RG, int GR>
+__global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const FullArgs a) {
+    constexpr int ESZ = DT == RBT_DT_BF16 ? 2 : 4, KW = kFullWin / ESZ;  // columns per k-step
+    constexpr int ROWS = 16 * RG, NT = 64 * kFullWaves, NCOL = (MATS == 2 ? 16 : 32) * kFullWaves;
+    constexpr int PARTS = DT == RBT_DT_BF16 ? 3 : 1;
+    constexpr int ABYTES = ROWS * kFullWin, STAGE = PARTS * ABYTES;  // LDS bytes of a part, of a k-step
+    constexpr int UNITS = ROWS * 8, AU = (UNITS + NT - 1) / NT;     // activation units of KW / 8 columns
+    constexpr int UL = KW / 32;                                      // 16-byte loads per unit
+    constexpr int SLOTS = kFullAhead + 1;  // register sets of weights
+    constexpr int AS = AU * UL > 2 ? 2 : SLOTS;  // register sets of activations (two where a set is large)
+    __shared__ __align__(1024) uint8_t ring[2 * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63, W = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ntiles_n = (a.N + NCOL - 1) / NCOL;
+    const int total = a.m_off[a.E] * ntiles_n, range = (total + 7) >> 3;
+    const int slot = (int)(blockIdx.x >> 3), tau = (int)(blockIdx.x & 7) * range + slot;
+    if (slot >= range || tau >= total) return;
+    int e, jt, il;
+    tile_of(tau, a.m_off, a.E, ntiles_n, (__builtin_amdgcn_readfirstlane(*a.choice) >> 1) & 1, &e, &jt, &il);
+    const int row0 = a.offsets[e] + il * ROWS;
+    const int rows = __builtin_amdgcn_readfirstlane(min(ROWS, a.counts[e] - il * ROWS));
+    const int n0 = jt * NCOL;
+    const int rowb = a.Kd * ESZ;  // bytes per weight row
+    const int nch = (rowb + kFullWin - 1) / kFullWin;
+    const bool tail = rowb % kFullWin != 0;
+    const int rot = (e + jt * max(1, nch / ntiles_n)) % nch;
+    auto cidx = [&](int c) { return c + rot < nch ? c + rot : c + rot - nch; };
+
+    // weight rows of this lane: column group g, half s2 (rows 8 s2 .. 8 s2 + 7 of the group's 16)
+    const uint8_t *wp[2][2];
+    const int woff = 16 * blob_chunk(lane);
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2) {
+            const int n = n0 + (MATS == 2 ? 16 * W : 32 * W + 16 * g) + 8 * s2 + (lane & 7);
+            wp[g][s2] = a.experts + (size_t)e * a.stride + (MATS == 2 && g ? a.w3_off : a.w_off) +
+                        (size_t)min(n, a.N - 1) * (size_t)rowb;
+        }
+    // activation units of this thread: row u / 8, granule u % 8 of the step's KW columns
+    const size_t base_row = a.gather ? 0 : (size_t)row0;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(a.act) + base_row * (size_t)a.act_stride, 0, kWrBufRecords, kBufConfig);
+    uint32_t aoff[AU], adst[AU];
+    int acol[AU];
+#pragma unroll
+    for (int i = 0; i < AU; ++i) {
+        const int u = tid + NT * i, r = u >> 3, g = u & 7;
+        const int lr = row0 + (r < rows ? r : 0);
+        const size_t arow = a.gather ? (size_t)(a.perm[lr] / a.topk) : (size_t)lr;
+        acol[i] = (KW / 8) * g;
+        aoff[i] = r < rows ? (uint32_t)((arow - base_row) * a.act_stride + acol[i]) * 4u : (uint32_t)kWrBufRecords;
+        adst[i] = (uint32_t)(r * kFullWin + 16 * (g ^ ((r >> 1) & 7)));
+    }
+
+    u32x4 aset[AS][AU][UL];
+    u32x4 wv[SLOTS][2][2];
+    auto load_a = [&](u32x4 (&av)[AU][UL], int c) {
+        const int cc = cidx(c);
+#pragma unroll
+        for (int i = 0; i < AU; ++i)
+#pragma unroll
+            for (int j = 0; j < UL; ++j) {
+                uint32_t off = aoff[i] + (uint32_t)(KW * cc + 4 * j) * 4u;
+                if (KW * cc + acol[i] + 4 * j >= a.Kd) off = (uint32_t)kWrBufRecords;  // past the row: zeros
+                av[i][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0);
+            }
+    };
+    auto store_a = [&](const u32x4 (&av)[AU][UL], int buf) {
+        uint8_t *st = ring + buf * STAGE;
+#pragma unroll
+        for (int i = 0; i < AU; ++i) {
+            if (UNITS % NT != 0 && tid + NT * i >= UNITS) continue;
+            if constexpr (PARTS == 1) {
+                *reinterpret_cast<u32x4 *>(st + adst[i]) = av[i][0];
+            } else {
+                u32x4 p[3];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    uint32_t x0[3], x1[3];
+                    split3(__uint_as_float(av[i][j >> 1][2 * (j & 1)]), x0[0], x0[1], x0[2]);
+                    split3(__uint_as_float(av[i][j >> 1][2 * (j & 1) + 1]), x1[0], x1[1], x1[2]);
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) p[q][j] = pack_hi16(x0[q], x1[q]);
+                }
+#pragma unroll
+                for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4 *>(st + q * ABYTES + adst[i]) = p[q];
+            }
+        }
+    };
+    auto load_w = [&](u32x4 (&dst)[2][2], int c) {
+        const int off = cidx(c) * kFullWin + woff;
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2) {
+                const uint8_t *p = wp[g][s2];
+                if constexpr (GR == 16) {
+                    dst[g][s2] = ld_stream_u4(p + min(off, rowb - 16));
+                } else if constexpr (GR == 4) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        dst[g][s2][j] = __builtin_nontemporal_load(
+                            reinterpret_cast<const uint32_t *>(p + min(off + 4 * j, rowb - 4)));
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const uint16_t w0 = __builtin_nontemporal_load(
+                            reinterpret_cast<const uint16_t *>(p + min(off + 4 * j, rowb - 2)));
+                        const uint16_t w1 = __builtin_nontemporal_load(
+                            reinterpret_cast<const uint16_t *>(p + min(off + 4 * j + 2, rowb - 2)));
+                        dst[g][s2][j] = (uint32_t)w0 | ((uint32_t)w1 << 16);
+                    }
+                }
+            }
+    };
+    // the loads of a row's last, partial k-step past the row's end become zeros
+    auto mask_w = [&](u32x4 (&w)[2][2], int c) {
+        const int off = (nch - 1) * kFullWin + woff;
+        if (!tail || cidx(c) != nch - 1) return;
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    uint32_t v = off + 4 * j < rowb ? w[g][s2][j] : 0u;
+                    if (GR == 2 && off + 4 * j + 2 >= rowb) v &= 0xFFFFu;
+                    w[g][s2][j] = v;
+                }
+    };
+
+    // bf16: mid holds the sums of the last steps, acc of everything before them; f32: the sums, and what
+    // their adds rounded away
+    f32x4 acc[RG][2], mid[RG][2];
+#pragma unroll
+    for (int q = 0; q < RG; ++q) acc[q][0] = acc[q][1] = mid[q][0] = mid[q][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto flush = [&]() {
+#pragma unroll
+        for (int q = 0; q < RG; ++q)
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                acc[q][g] += mid[q][g];
+                mid[q][g] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+    };
+
+    // k-step c, its operands in slot J = c % SLOTS. Loads return in issue order and a wait covers every older
+    // load, so a step issues activations (AS steps ahead, stored to LDS one step ahead) before weights
+    // (kFullAhead steps ahead): the LDS store waits for activations issued AS - 1 steps ago and not for
+    // the weights behind them. FULL: every load of the step exists (no branches, so the waits stay exact).
+    auto step = [&](auto jc, auto fullc, int c) {
+        constexpr int J = decltype(jc)::value;
+        constexpr bool FULL = decltype(fullc)::value;
+        if (FULL || c + 1 < nch) store_a(aset[(J + 1) % AS], (c + 1) & 1);  // the buffer that step c - 1 read
+        if (FULL || c + AS < nch) load_a(aset[J % AS], c + AS);
+        if (FULL || c + kFullAhead < nch) load_w(wv[(J + kFullAhead) % SLOTS], c + kFullAhead);
+        const uint8_t *st = ring + (c & 1) * STAGE;
+        mask_w(wv[J], c);
+        blob_operands(wv[J][0][0], wv[J][0][1]);
+        blob_operands(wv[J][1][0], wv[J][1][1]);
+#pragma unroll
+        for (int q = 0; q < RG; ++q) {
+            if (16 * q < rows) {  // wave-uniform: the row group holds list entries
+                const int r = 16 * q + (lane & 15);
+                f32x4 t[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+                const uint8_t *ap[2];
+#pragma unroll
+                for (int s2 = 0; s2 < 2; ++s2) ap[s2] = st + r * kFullWin + 16 * ((4 * s2 + (lane >> 4)) ^ ((r >> 1) & 7));
+                if constexpr (DT == RBT_DT_BF16) {
+#pragma unroll
+                    for (int p = PARTS - 1; p >= 0; --p)  // the small parts first
+#pragma unroll
+                        for (int s2 = 0; s2 < 2; ++s2) {
+                            const bf16x8 x = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(ap[s2] + p * ABYTES));
+#pragma unroll
+                            for (int g = 0; g < 2; ++g)
+                                t[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, __builtin_bit_cast(bf16x8, wv[J][g][s2]),
+                                                                               t[g], 0, 0, 0);
+                        }
+                } else {
+#pragma unroll
+                    for (int s2 = 0; s2 < 2; ++s2) {
+                        const u32x4 x = *reinterpret_cast<const u32x4 *>(ap[s2]);
+                        t[0] = t[1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+#pragma unroll
+                            for (int g = 0; g < 2; ++g)
+                                t[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(x[i]),
+                                                                            __uint_as_float(wv[J][g][s2][i]), t[g], 0, 0, 0);
+#pragma unroll
+                        for (int g = 0; g < 2; ++g) {
+#pragma clang fp reassociate(off)
+                            const f32x4 was = acc[q][g];
+                            acc[q][g] = was + t[g];
+                            mid[q][g] += t[g] - (acc[q][g] - was);  // what the sum rounded away
+                        }
+                    }
+                }
+                if constexpr (DT == RBT_DT_BF16) {
+                    mid[q][0] += t[0];
+                    mid[q][1] += t[1];
+                }
+            }
+        }
+        __syncthreads();
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    static_assert(SLOTS == 4 && kFullAhead == 3, "one step call per slot below");
+    // prologue, in the steady state's order
+#pragma unroll
+    for (int p = 0; p < SLOTS; ++p) {
+        if (p < AS && p < nch) load_a(aset[p % AS], p);
+        if (p < kFullAhead && p < nch) load_w(wv[p], p);
+    }
+    store_a(aset[0], 0);
+    __syncthreads();
+    int c = 0;
+    for (; c + 2 * SLOTS <= nch; c += SLOTS) {
+        step(I0{}, std::true_type{}, c);
+        step(I1{}, std::true_type{}, c + 1);
+        step(I2{}, std::true_type{}, c + 2);
+        step(I3{}, std::true_type{}, c + 3);
+        if (DT == RBT_DT_BF16 && (c & SLOTS)) flush();
+    }
+    for (; c < nch; c += SLOTS) {
+        step(I0{}, std::false_type{}, c);
+        if (c + 1 < nch) step(I1{}, std::false_type{}, c + 1);
+        if (c + 2 < nch) step(I2{}, std::false_type{}, c + 2);
+        if (c + 3 < nch) step(I3{}, std::false_type{}, c + 3);
+    }
+    flush();
+
+    // acc[q][g] lane holds column (lane % 16) of group g for list rows 16 q + 4 (lane / 16) + i
+#pragma unroll
+    for (int q = 0; q < RG; ++q) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = 16 * q + 4 * (lane >> 4) + i;
+            if (r >= rows) continue;
+            float *orow = a.out + (size_t)(row0 + r) * a.out_stride;
+            if constexpr (MATS == 2) {
+                const int n = n0 + 16 * W + (lane & 15);
+                const float g = acc[q][0][i], u = acc[q][1][i];
+                // silu(g) * u, rabbit2.c:535-537; the columns that pad the row are zeros
+                if (n < a.out_stride) orow[n] = n < a.N ? (g / (1.0f + expf(-g))) * u : 0.0f;
+            } else {
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    const int n = n0 + 32 * W + 16 * g + (lane & 15);
+                    if (n < a.N) orow[n] = acc[q][g][i];
+                }
+            }
+        }
+    }
+}
+
+// Bytes per weight load that the rows of Kd elements from `base` on (rows and experts `step` apart) allow.
+int load_granule(uint64_t base, uint64_t stride, int Kd, int esz) {
+    const uint64_t bits = base | stride | (uint64_t)Kd * esz;
+    return bits % 16 == 0 ? 16 : bits % 4 == 0 ? 4 : bits % 2 == 0 && esz == 2 ? 2 : 0;
+}
+
+template <int MATS>
+hipError_t launch_full(const Launch &L, const FullArgs &a, int dtype, int rg, int max_mtiles) {
+    constexpr int NCOL = (MATS == 2 ? 16 : 32) * kFullWaves;
+    const long long tiles = (long long)max_mtiles * ((a.N + NCOL - 1) / NCOL), blocks = (tiles + 7) / 8 * 8;
+    const int gr = load_granule(reinterpret_cast<uintptr_t>(a.experts) | a.w_off | a.w3_off, a.stride, a.Kd,
+                                dtype == RBT_DT_BF16 ? 2 : 4);
+    if (blocks > 0x7FFFFFFFll || gr == 0) return hipErrorInvalidValue;
+    const dim3 g((unsigned)blocks), b(64 * kFullWaves);
+#define FULL_CASE(DT, RG, GR) \
+    if (dtype == DT && rg == RG && gr == GR) return launch(L, grouped_full_kernel<DT, MATS, RG, GR>, g, b, 0, a);
+#define FULL_TILES(DT, GR)  \
+    FULL_CASE(DT, 2, GR) \
+    FULL_CASE(DT, 4, GR)
+    FULL_TILES(RBT_DT_BF16, 16)
+    FULL_TILES(RBT_DT_BF16, 4)
+    FULL_TILES(RBT_DT_BF16, 2)
+    FULL_TILES(RBT_DT_F32, 16)
+    FULL_TILES(RBT_DT_F32, 4)
+#undef FULL_TILES
+#undef FULL_CASE
+    return hipErrorInvalidValue;
+}
+
+// Mean list rows up to which tiles have 32 rows: half the LDS and 162 instead of 196 registers, and a list
+// that passes 32 rows re-reads its weights from L2 (f32 200 tokens, 25 rows on average: 250 us either way;
+// with +2 on eight experts' logits 304 against 384 us).
+constexpr int kFullShortLists = 40;
+
+}  // namespace
+
+bool full_supported(int dtype, int T, int E, int K, int D, int H, const void *experts, uint64_t stride,
+                    const float *xb) {
+    const int esz = dtype == RBT_DT_BF16 ? 2 : 4;
+    const uint64_t base = reinterpret_cast<uintptr_t>(experts);
+    return T >= 1 && T <= 65535 && E <= kDispatchMaxE && (long long)T * K <= (1 << 24) && D % 4 == 0 &&
+           (reinterpret_cast<uintptr_t>(xb) & 15u) == 0 && load_granule(base, stride, D, esz) != 0 &&
+           load_granule(base, stride, H, esz) != 0 &&
+           // 32-bit buffer offsets: the gathered rows of xb, a tile's rows of h, and bytes of a weight row
+           (uint64_t)T * D * 4 < (uint64_t)kWrBufRecords && 128ull * full_h_stride(H) * 4 < (uint64_t)kWrBufRecords &&
+           (uint64_t)D * esz < (1u << 30) && (uint64_t)H * esz < (1u << 30);
+}
+
+// The grouped form reads each selected expert once, the per-pair GEMVs once per pair; it has two more
+// launches and longer kernels (~25 us at the smallest sizes). So it pays from a number of saved bytes on:
+// pairs minus experts expected to be selected, times an expert's bytes. Measured, GEMVs / grouped, us:
+//   f32, dim 2048, 64 experts, top-8, hidden 1024: 6 tokens (350 MB saved) 194 / 202, 8 (550 MB) 255 / 209,
+//     11 345 / 267, 200 5763 / 476
+//   bf16, dim 1600, 40 experts, top-6, hidden 800: 2 tokens (12 MB) 46 / 60, 8 (150 MB) 110 / 79, 1000
+//     11045 / 364
+//   bf16, dim 1000, 20 experts, top-3, hidden 330: 11 tokens (32 MB) 40 / 57, 50 (260 MB) 98 / 61
+// The shapes of the specialised GEMVs (experts_decode.hip) stream twice as fast and need more.
+bool full_pays(bool fast_gemv, int dtype, int T, int E, int K, int D, int H) {
+    const double p = (double)T * K, sel = E * (1.0 - pow(1.0 - (double)K / E, (double)T));
+    return (p - sel) * 3.0 * H * D * (dtype == RBT_DT_BF16 ? 2 : 4) >= (fast_gemv ? 450e6 : 100e6);
+}
+
+size_t full_workspace_bytes(int T, int E, int K, int D) {
+    const size_t P = (size_t)T * K;
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    return up(4 * (size_t)E) + 3 * up(4 * (size_t)(E + 1)) + up(4) + 2 * up(4 * P) + up(4 * P * (size_t)D);
+}
+
+hipError_t launch_grouped_full(const Launch &Ld, const Launch &Lg, const Launch &Lw, const Launch &Lc, int dtype,
+                               const void *experts, uint64_t stride, const float *xb, int T, int E, int K, int D, int H,
+                               const int32_t *routing, const float *weights, float *hbuf, void *ws, float *x_inout,
+                               float *moe_out, int32_t **counts_out) {
+    if (T <= 0 || K <= 0) return hipErrorInvalidValue;
+    const int P = T * K;
+    uint8_t *w = static_cast<uint8_t *>(ws);
+    auto carve = [&](size_t bytes) {
+        uint8_t *p = w;
+        w += (bytes + 255) / 256 * 256;
+        return p;
+    };
+    int32_t *counts = reinterpret_cast<int32_t *>(carve(4 * (size_t)E));
+    int32_t *offsets = reinterpret_cast<int32_t *>(carve(4 * (size_t)(E + 1)));
+    int32_t *m_off = reinterpret_cast<int32_t *>(carve(4 * (size_t)(E + 1)));
+    int32_t *m_off128 = reinterpret_cast<int32_t *>(carve(4 * (size_t)(E + 1)));  // written by the dispatch, not used
+    int32_t *choice = reinterpret_cast<int32_t *>(carve(4));
+    int32_t *perm = reinterpret_cast<int32_t *>(carve(4 * (size_t)P));
+    int32_t *pos_of = reinterpret_cast<int32_t *>(carve(4 * (size_t)P));
+    float *y = reinterpret_cast<float *>(carve(4 * (size_t)P * D));
+    if (counts_out) *counts_out = counts;
+    const int rg = P <= kFullShortLists * E ? 2 : 4;
+    hipError_t e = launch_dispatch(Ld, routing, P, E, counts, offsets, perm, pos_of, m_off, 16 * rg, m_off128,
+                                   choice, 2);
+    if (e != hipSuccess) return e;
+    const int max_mtiles = (P + 16 * rg - 1) / (16 * rg) + E;  // >= sum over experts of ceil(count / (16 rg))
+    const uint64_t mat = (uint64_t)H * D * (dtype == RBT_DT_BF16 ? 2 : 4);
+    const int hs = full_h_stride(H);
+    const uint8_t *ex = static_cast<const uint8_t *>(experts);
+    FullArgs a{ex, stride, 0, mat, H, D, xb, D, 1, perm, K, counts, offsets, m_off, choice, E, hbuf, hs};
+    e = launch_full<2>(Lg, a, dtype, rg, max_mtiles);
+    if (e != hipSuccess) return e;
+    a = FullArgs{ex, stride, 2 * mat, 0, D, H, hbuf, hs, 0, perm, K, counts, offsets, m_off, choice, E, y, D};
+    e = launch_full<1>(Lw, a, dtype, rg, max_mtiles);
+    if (e != hipSuccess) return e;
+    return launch_combine(Lc, y, pos_of, weights, T, K, D, x_inout, moe_out);
+}
+
+}  // namespace rbt

@@ -38,7 +38,6 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kDispatchMaxE = 256;
 constexpr int kDispRegs = 4;  // 64-pair steps per wave kept in registers by dispatch_kernel (4096 pairs)
 
 
@@ -317,39 +316,6 @@ struct GTile {
 // Requirements (prefill_supported): N % (256 / MATS) == 0, Kd % 64 == 0, 16-byte aligned rows.
 // The block's work on tile slot `bid` (the kernels below pass blockIdx.x); ring: the LDS ring of
 // STAGES * SBYTES bytes at LDS offset ring0.
-// Tile slot tau -> (expert e, column tile jt, row tile il of e's list), with m_off the prefix of the
-// experts' row tiles and nt column tiles. Expert-major (colmajor 0): e's tiles are consecutive, so an
-// expert's column tiles share its activation rows in one XCD's L2. Column-major (1): tau = jc * M + rt
-// over the M row tiles of all experts (expert e's column tile (jc + e) mod nt), so each XCD's
-// contiguous share of the slots spans every expert's row tiles for a few column tiles and a few long
-// lists load all XCDs alike. Either way an expert's row tiles of one column tile (one weight tile) are
-// consecutive, on one XCD.
-__device__ __forceinline__ void tile_of(int tau, const int32_t *__restrict__ m_off, int E, int nt, int colmajor,
-                                        int *e_out, int *jt_out, int *il_out) {
-    const int M = m_off[E];
-    const int jc = colmajor ? tau / M : 0, key = colmajor ? tau - jc * M : tau, scale = colmajor ? 1 : nt;
-    int lo = 0, hi = E - 1;  // the last e with m_off[e] * scale <= key
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (m_off[mid] * scale <= key)
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    const int e = lo;
-    if (colmajor) {
-        // diagonal: slot column jc holds column tile (jc + e) mod nt of expert e, so the tiles that run
-        // together on one XCD are not all the same column tile of many experts (the experts' blobs are
-        // a multiple of 4 MiB apart, so those would stream congruent address windows at the same time)
-        *jt_out = jc + e % nt < nt ? jc + e % nt : jc + e % nt - nt;
-        *il_out = key - m_off[e];
-    } else {
-        const int me = m_off[e + 1] - m_off[e], local = key - m_off[e] * nt;
-        *jt_out = local / me;
-        *il_out = local - *jt_out * me;
-    }
-    *e_out = e;
-}
 
 template <int MATS, int ROWS, int WROWS>
 __device__ __forceinline__ void gemm_lds_tile(
@@ -521,9 +487,6 @@ __global__ __launch_bounds__((64 * GTile<ROWS, WROWS>::kWaves), 1) void grouped_
 // Every wait is the compiler's own. Same operands, accumulation order and epilogue arithmetic as
 // grouped_gemm_kernel.
 constexpr int kWrRows = 128, kWrKC = 64, kWrAhead = 3, kWrWaves = 16;
-// buffer resources of the activation planes: records (bytes) past any valid offset, and the config
-// word of a raw 32-bit-format buffer
-constexpr int kWrBufRecords = 0x7FFF0000, kBufConfig = 0x00020000;
 // whole tiles of output columns, and k-steps a multiple of the kWrAhead + 1 register slots
 constexpr bool gemm_wr_supported(int mats, int N, int Kd) {
     return N % (mats == 2 ? 128 : 256) == 0 && Kd % (kWrKC * (kWrAhead + 1)) == 0;
@@ -1239,6 +1202,24 @@ void prefill_x_planes(void *ws, int T, int E, int K, int D, uint16_t **x_hi, uin
     *x_lo = r.x_lo;
 }
 
+hipError_t launch_dispatch(const Launch &L, const int32_t *routing, int P, int E, int32_t *counts, int32_t *offsets,
+                           int32_t *perm, int32_t *pos_of, int32_t *m_off, int mt_rows, int32_t *m_off2, int32_t *choice,
+                           int tall) {
+    if (P < 1 || E < 1 || E > kDispatchMaxE) return hipErrorInvalidValue;
+    return launch(L, dispatch_kernel, dim3(1), dim3(1024), 0, routing, P, E, counts, offsets, perm, pos_of, m_off,
+                  mt_rows, m_off2, choice, tall);
+}
+
+hipError_t launch_combine(const Launch &Lc, const float *y, const int32_t *pos_of, const float *weights, int T, int K,
+                          int D, float *x_inout, float *moe_out) {
+    const auto a16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
+    if (K <= 8 && D % 4 == 0 && a16(y) && (!x_inout || a16(x_inout)) && (!moe_out || a16(moe_out)))
+        return launch(Lc, combine_rows4_kernel, dim3((unsigned)((D / 4 + 255) / 256), (unsigned)T), dim3(256), 0,
+                      y, pos_of, weights, K, D, x_inout, moe_out);
+    return launch(Lc, combine_rows_kernel, dim3((unsigned)((D + 255) / 256), (unsigned)T), dim3(256), 0,
+                  y, pos_of, weights, K, D, x_inout, moe_out);
+}
+
 hipError_t launch_prefill(const Launch &Ld, const Launch &Lg, const Launch &Lw, const Launch &Lc, const void *experts,
                           uint64_t stride, const float *xb, int T, int E, int K, int D, int H, const int32_t *routing,
                           const float *weights, float *hbuf, void *ws, float *x_inout, float *moe_out,
@@ -1278,8 +1259,8 @@ hipError_t launch_prefill(const Launch &Ld, const Launch &Lg, const Launch &Lw, 
     const int mt_rows = small ? 32 : 64;
     const int tall = !tall_ok || small || tile_rows == 64 ? 1 : 2;
     const bool sel = !small && tall_ok;
-    e = launch(Ldd, dispatch_kernel, dim3(1), dim3(1024), 0, routing, P, E, counts, offsets, perm, pos_of, m_off,
-               mt_rows, sel ? r.m_off128 : nullptr, r.choice, tall);
+    e = launch_dispatch(Ldd, routing, P, E, counts, offsets, perm, pos_of, m_off, mt_rows, sel ? r.m_off128 : nullptr,
+                        r.choice, tall);
     if (e != hipSuccess) return e;
     // 128-row tiles (the dispatch picks them whenever tall == 2) in the wide kernel where the shape has it
     const bool wide = sel && tall == 2 && wide_ok && gemm_wide_supported(2, H, D) && gemm_wide_supported(1, D, H);
@@ -1317,12 +1298,7 @@ hipError_t launch_prefill(const Launch &Ld, const Launch &Lg, const Launch &Lw, 
                                r.choice, E, max_mtiles, y, nullptr, nullptr, tl, tstride, w2);
     if (e != hipSuccess) return e;
     if (!combine) return hipSuccess;
-    const auto a16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
-    if (K <= 8 && D % 4 == 0 && a16(y) && (!x_inout || a16(x_inout)) && (!moe_out || a16(moe_out)))
-        return launch(Lc, combine_rows4_kernel, dim3((unsigned)((D / 4 + 255) / 256), (unsigned)T), dim3(256), 0,
-                      (const float *)y, (const int32_t *)pos_of, weights, K, D, x_inout, moe_out);
-    return launch(Lc, combine_rows_kernel, dim3((unsigned)((D + 255) / 256), (unsigned)T), dim3(256), 0,
-                  (const float *)y, (const int32_t *)pos_of, weights, K, D, x_inout, moe_out);
+    return launch_combine(Lc, y, pos_of, weights, T, K, D, x_inout, moe_out);
 }
 
 }  // namespace rbt

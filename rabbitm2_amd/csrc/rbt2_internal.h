@@ -70,6 +70,44 @@ __device__ __forceinline__ void blob_operands(u32x4 &a, u32x4 &b) {
 }
 
 
+// buffer resources of activation rows: records (bytes) past any valid offset, and the config word of a
+// raw 32-bit-format buffer
+constexpr int kWrBufRecords = 0x7FFF0000, kBufConfig = 0x00020000;
+
+// Tile slot tau -> (expert e, column tile jt, row tile il of e's list), with m_off the prefix of the
+// experts' row tiles and nt column tiles. Expert-major (colmajor 0): e's tiles are consecutive, so an
+// expert's column tiles share its activation rows in one XCD's L2. Column-major (1): tau = jc * M + rt
+// over the M row tiles of all experts (expert e's column tile (jc + e) mod nt), so each XCD's
+// contiguous share of the slots spans every expert's row tiles for a few column tiles and a few long
+// lists load all XCDs alike. Either way an expert's row tiles of one column tile (one weight tile) are
+// consecutive, on one XCD.
+__device__ __forceinline__ void tile_of(int tau, const int32_t *__restrict__ m_off, int E, int nt, int colmajor,
+                                        int *e_out, int *jt_out, int *il_out) {
+    const int M = m_off[E];
+    const int jc = colmajor ? tau / M : 0, key = colmajor ? tau - jc * M : tau, scale = colmajor ? 1 : nt;
+    int lo = 0, hi = E - 1;  // the last e with m_off[e] * scale <= key
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (m_off[mid] * scale <= key)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    const int e = lo;
+    if (colmajor) {
+        // diagonal: slot column jc holds column tile (jc + e) mod nt of expert e, so the tiles that run
+        // together on one XCD are not all the same column tile of many experts (the experts' blobs are
+        // a multiple of 4 MiB apart, so those would stream congruent address windows at the same time)
+        *jt_out = jc + e % nt < nt ? jc + e % nt : jc + e % nt - nt;
+        *il_out = key - m_off[e];
+    } else {
+        const int me = m_off[e + 1] - m_off[e], local = key - m_off[e] * nt;
+        *jt_out = local / me;
+        *il_out = local - *jt_out * me;
+    }
+    *e_out = e;
+}
+
 // Cross-lane moves through DPP (a VALU operand modifier, no LDS round trip). Within each row of 16
 // lanes: swap neighbours, swap pairs, mirror each half-row, mirror the row -- after four steps every
 // lane of a row holds the same row total (each step adds commutative partners, so all lanes of a
@@ -203,6 +241,28 @@ void prefill_combine_inputs(void *ws, int T, int E, int K, int D, const float **
 hipError_t launch_combine_rmsnorm(const Launch &L, const float *y, const int32_t *pos_of, const float *weights, int K,
                                   int T, int n, float *x, const float *w, float eps, float *out, uint16_t *hi,
                                   uint16_t *lo);
+
+// The grouped path's dispatch (one block) and combine launches, which the grouped forms share. m_off2 and
+// choice may be NULL together (one tile height, expert-major slots).
+constexpr int kDispatchMaxE = 256;
+hipError_t launch_dispatch(const Launch &L, const int32_t *routing, int P, int E, int32_t *counts, int32_t *offsets,
+                           int32_t *perm, int32_t *pos_of, int32_t *m_off, int mt_rows, int32_t *m_off2, int32_t *choice,
+                           int tall);
+hipError_t launch_combine(const Launch &L, const float *y, const int32_t *pos_of, const float *weights, int T, int K,
+                          int D, float *x_inout, float *moe_out);
+
+// The grouped form at full f32 activation precision (grouped_full.hip): f32 weights, and bf16 weights of
+// any dims. full_h_stride: floats per h row in hbuf. ws holds full_workspace_bytes().
+inline int full_h_stride(int H) { return (H + 3) / 4 * 4; }
+bool full_supported(int dtype, int T, int E, int K, int D, int H, const void *experts, uint64_t stride,
+                    const float *xb);
+// Whether it is faster than the per-pair GEMVs (fast_gemv: experts_decode_supported()).
+bool full_pays(bool fast_gemv, int dtype, int T, int E, int K, int D, int H);
+size_t full_workspace_bytes(int T, int E, int K, int D);
+hipError_t launch_grouped_full(const Launch &Ld, const Launch &Lg, const Launch &Lw, const Launch &Lc, int dtype,
+                               const void *experts, uint64_t stride, const float *xb, int T, int E, int K, int D, int H,
+                               const int32_t *routing, const float *weights, float *hbuf, void *ws, float *x_inout,
+                               float *moe_out, int32_t **counts_out);
 
 // Router logits + softmax + top-k + the activation hi/lo split in one launch, for the grouped path
 // (AVX2 order, E <= 64). x_hi/x_lo may be NULL (no split).

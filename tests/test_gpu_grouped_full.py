@@ -1,0 +1,118 @@
+"""The full-precision grouped form (rabbitm2_amd/csrc/grouped_full.hip): f32 weights, and bf16 weights of
+dims that the bf16 tiles do not divide, from "prefill_min_tokens" tokens on.
+
+Each output is held to its value in 64 bits within the worst case of its own sums: a sum of n f32 products
+in blocks of 64 columns and then over the blocks is off by at most gamma = (64 + n / 32 + 16) * 2^-24 of the
+sum of its terms' absolute values (the parts of a bf16 product are exact); the gate and up errors travel
+through silu (slope at most 1.1) and W2, and the exp, divide and combine add a few roundings each.
+Routing equals the oracle's except at exact ties.
+"""
+import numpy as np
+import pytest
+
+from oracle import pyoracle as po
+from tests.common import SynthLayer, routing_check
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # (D, E, K, H, dtype, T, bias on expert 0)
+    (36, 5, 2, 25, po.DT_F32, 17, 0),      # partial last k-steps, h rows padded, 4-byte loads
+    (36, 4, 2, 25, po.DT_BF16, 20, 0),     # 2-byte loads of W2 rows
+    (32, 4, 1, 64, po.DT_F32, 13, 0),      # one k-step
+    (8, 4, 2, 7, po.DT_BF16, 12, 0),       # rows shorter than a k-step both ways
+    (64, 8, 2, 128, po.DT_BF16, 12, 0),    # 32-row tiles
+    (1000, 20, 3, 330, po.DT_BF16, 50, 0),
+    (100, 7, 7, 33, po.DT_BF16, 40, 0),    # K = E: every list 40 rows, 64-row tiles
+    (256, 8, 2, 256, po.DT_F32, 300, 30),  # one list of 300 rows: five row tiles
+    (260, 6, 1, 132, po.DT_BF16, 129, 0),  # past a column tile by 4
+    (128, 256, 4, 48, po.DT_F32, 64, 0),   # the most experts, most lists empty
+    (2048, 64, 8, 1024, po.DT_F32, 33, 0),
+]
+
+
+def reference(layer, xb, routing, weights):
+    """(moe, bound) in 64 bits for the given routing."""
+    T, D, H = xb.shape[0], layer.D, layer.H
+    u = 2.0 ** -24
+    g1, g2 = (64 + D / 32 + 16) * u, (64 + H / 32 + 16) * u
+    moe, bound = np.zeros((T, D)), np.zeros((T, D))
+    n = H * D
+    for e in np.unique(routing):
+        raw = layer.experts[e * layer.stride:e * layer.stride + 3 * n * layer.esz]
+        w = (po.bf16_to_f32(raw.view(np.uint16)) if layer.dtype == po.DT_BF16 else raw.view(np.float32)).astype(np.float64)
+        w1, w3, w2 = w[:n].reshape(H, D), w[n:2 * n].reshape(H, D), w[2 * n:].reshape(D, H)
+        t, k = np.nonzero(routing == e)
+        x = xb[t].astype(np.float64)
+        g, up = x @ w1.T, x @ w3.T
+        eg, eu = g1 * (np.abs(x) @ np.abs(w1).T), g1 * (np.abs(x) @ np.abs(w3).T)
+        s = g / (1.0 + np.exp(-g))
+        h = s * up
+        eh = 1.1 * np.abs(up) * eg + (np.abs(s) + 1.1 * eg) * eu + 8 * u * np.abs(h)
+        wk = weights[t, k].astype(np.float64)[:, None]
+        np.add.at(moe, t, wk * (h @ w2.T))
+        np.add.at(bound, t, wk * (eh @ np.abs(w2).T + (g2 + 12 * u) * ((np.abs(h) + eh) @ np.abs(w2).T)))
+    return moe, bound
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=["D%dE%dK%dH%ddt%dT%db%d" % s for s in SHAPES])
+def test_full_grouped_shapes(dev, shape):
+    D, E, K, H, dt, T, b = shape
+    bias = np.array([float(b)] + [0.0] * (E - 1), np.float32) if b else None
+    dev.set_option("prefill_min_tokens", 12)  # from 12 tokens on whatever the sizes
+    layer = SynthLayer(dev, D, E, K, H, dt, 1, seed=31, w_scale=1.0, fan_in=True, bias=bias)
+    try:
+        dev.set_router_order(po.ORDER_AVX2)
+        xb = layer.make_x(T, seed=32, bf16=False)
+        x = layer.make_x(T, seed=33)
+        got = layer.run_gpu(xb, x=x)
+        want = layer.oracle(xb, po.ORDER_AVX2, x=x)
+        assert routing_check(got["routing"], want["routing"], want["probs"])[1] == 0
+        counts = dev.expert_counts(E)
+        assert counts is not None and np.array_equal(counts, np.bincount(got["routing"].ravel(), minlength=E))
+        moe, bound = reference(layer, xb, got["routing"], got["weights"])
+        worst = np.max(np.abs(got["moe"] - moe) / np.maximum(bound, 1e-30))
+        rel = np.linalg.norm(got["moe"] - moe) / np.linalg.norm(moe)
+        print(f"D{D}E{E}K{K}H{H}T{T}: error {rel:.2e}, {worst:.3f} of the bound", flush=True)
+        assert worst <= 1.0
+        assert np.array_equal(got["x"], x + got["moe"])
+    finally:
+        layer.close()
+
+
+def test_full_grouped_nonfinite_rows_stay_apart(dev):
+    """A token with infinities and NaN leaves the other tokens' rows as they are without it."""
+    dev.set_option("prefill_min_tokens", 12)
+    layer = SynthLayer(dev, 68, 4, 4, 36, po.DT_BF16, 0, seed=35, w_scale=1.0, fan_in=True)
+    try:
+        dev.set_router_order(po.ORDER_AVX2)
+        xb = layer.make_x(16, seed=36, bf16=False)
+        clean = layer.run_gpu(xb)["moe"]
+        xb[5, 3], xb[5, 67] = np.inf, np.nan
+        xb[9, :4] = 3.4e38  # rounds past the largest bf16; its parts do not
+        got = layer.run_gpu(xb)["moe"]
+        keep = [t for t in range(16) if t not in (5, 9)]
+        assert got[keep].tobytes() == clean[keep].tobytes()
+        assert np.isnan(got[5]).any()
+    finally:
+        layer.close()
+
+
+def test_full_grouped_scratch_limit(dev):
+    """rbt_hip_moe_dev_noalloc takes the per-pair GEMVs where the grouped buffers pass its scratch array, so
+    the calls that fitted without them still run."""
+    D, E, K, H, T = 2048, 8, 8, 64, 1200  # y alone is 75 MiB; the GEMVs need 2.4 MiB
+    dev.set_option("prefill_min_tokens", 12)
+    layer = SynthLayer(dev, D, E, K, H, po.DT_F32, 1, seed=37, w_scale=1.0, fan_in=True)
+    xb = layer.make_x(T, seed=38)
+    xd, moe = dev.upload_array(xb), dev.malloc(4 * T * D)
+    try:
+        dev.set_router_order(po.ORDER_AVX2)
+        dev.moe_dev_noalloc(layer.desc(), xd, T, moe=moe)
+        got = dev.d2h(moe, (T, D), np.float32)
+        want = layer.run_gpu(xb)["moe"]
+        assert np.linalg.norm(got - want) <= 4e-6 * np.linalg.norm(want)
+    finally:
+        dev.free(xd)
+        dev.free(moe)
+        layer.close()
