@@ -200,7 +200,9 @@ int rbt_hip_forward(rbt_hip *h, int token, int pos, float *logits, int32_t *rout
  * position 0, then up to n_gen tokens (at most ctx - n_prompt; the eos token is kept and ends the
  * output, -1 = none) into out; *n_out = the count. The loop runs on the device: each step's argmax
  * writes the next step's token, and each step is one HIP graph replay (steps after an eos are run and
- * discarded). ms_out (may be NULL) receives [prompt ms, generation ms] from HIP events: the prompt up to
+ * discarded). The prompt's positions before its last are run in blocks of up to 512 (from 4 positions on,
+ * where the dims are multiples of 4), each weight read once per block, at the per-token steps' precision;
+ * the buffers for them are allocated by the first such prompt and freed with the decode state. ms_out (may be NULL) receives [prompt ms, generation ms] from HIP events: the prompt up to
  * the first generated token, then the steps after it (from option "generate_timed_from" on). */
 int rbt_hip_generate(rbt_hip *h, const int32_t *prompt, int n_prompt, int n_gen, int32_t eos, int32_t *out,
                      int *n_out, double *ms_out);

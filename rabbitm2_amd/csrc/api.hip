@@ -93,6 +93,15 @@ struct DecodeState {
     StepState *st = nullptr;      // [n_seq]
 };
 
+// Buffers of a prompt block (prompt_block): one allocation for `tokens` positions, made by the first prompt
+// long enough, freed with the decode state.
+struct PromptBuf {
+    int tokens = 0;
+    uint8_t *block = nullptr;
+    float *x = nullptr, *xb = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *ao = nullptr;
+    uint8_t *moe = nullptr;  // the MoE block's scratch (scratch_view)
+};
+
 // A tiled copy of one layer's experts (launch_prefill_layout), taken from the blobs at `experts`.
 struct TiledLayer {
     const void *experts = nullptr;
@@ -126,6 +135,7 @@ struct rbt_hip {
     std::vector<LayerOff> layers;
     Workspace ws;
     DecodeState ds;
+    PromptBuf prompt;
     Profile prof;
     int fused_decode = 1;  // option "fused_decode": batch-1 top-k inside the gate/up kernel
     int batch_mfma = 1;    // option "batch_mfma": batched dense matvecs on the matrix cores
@@ -604,6 +614,8 @@ int model_drop(rbt_hip *h) {
     HIP_OK(h, hipStreamSynchronize(h->stream));
     (void)hipFree(h->ds.block);
     h->ds = DecodeState{};
+    (void)hipFree(h->prompt.block);
+    h->prompt = PromptBuf{};
     (void)hipFree(h->rhist);
     h->rhist = nullptr;
     if (h->model) {
@@ -992,9 +1004,16 @@ int moe_block(rbt_hip *h, const rbt_moe_layer *L, const float *xb_dev, int T, fl
         h->expert_counts = counts;
         return done();
     }
-    HIP_OK(h, launch_router(lc(h, kProfRouter), lc(h, kProfTopk), h->order, L->dtype, xb_dev, L->router,
-                            L->router_bias, T, L->n_experts, L->dim, L->top_k, L->norm_topk, w.probs, routing,
-                            weights));
+    // the fused front end keeps a router row per lane: from 48 experts on it beats the two launches (dim 2048,
+    // 64 experts, 400 tokens 18.5 us; 40 experts, dim 1600, 1000 tokens 31.9 against 26.6 us)
+    if (form == kMoeGroupedFull && T > kRouterDecodeMaxT && L->n_experts >= 48 &&
+        router_prefill_supported(h->order, L->dtype, T, L->n_experts, L->dim, L->top_k, L->router, xb_dev))
+        HIP_OK(h, launch_router_prefill(lc(h, kProfRouter), L->dtype, xb_dev, L->router, L->router_bias, T, L->n_experts,
+                                        L->dim, L->top_k, L->norm_topk, routing, weights, nullptr, nullptr));
+    else
+        HIP_OK(h, launch_router(lc(h, kProfRouter), lc(h, kProfTopk), h->order, L->dtype, xb_dev, L->router,
+                                L->router_bias, T, L->n_experts, L->dim, L->top_k, L->norm_topk, w.probs, routing,
+                                weights));
     if (form == kMoeGroupedFull) {
         int32_t *counts = nullptr;
         HIP_OK(h, launch_grouped_full(lc(h, kProfDispatch), lc(h, kProfGateup), lc(h, kProfDown), lc(h, kProfCombine),
@@ -1014,6 +1033,109 @@ int moe_block(rbt_hip *h, const rbt_moe_layer *L, const float *xb_dev, int T, fl
                                       w.hbuf, T, L->top_k, L->dim, L->expert_hidden, x_dev, moe_dev));
     }
     return done();
+}
+
+// ---- a prompt in blocks of positions (rabbit2.c:703-714 token by token)
+constexpr int kPromptBlock = 512;  // positions per block at most
+// Positions from which a block beats the per-token steps (16 layers of the dim-2048 model): 4 positions 2.9
+// against 3.5 ms, 23 positions 3.5 against 16.2 ms, 399 positions 7.4 against 270 ms.
+constexpr int kPromptMinTokens = 4;
+
+// The MoE form of a prompt block of T tokens: the activations keep f32 precision, as in the per-token steps
+// (never the two-part grouped form).
+MoeForm prompt_form(const rbt_hip *h, const rbt_moe_layer *L, int T) {
+    return T > 1 && full_from(h, L->dtype, T, L->n_experts, L->top_k, L->dim, L->expert_hidden, L->experts,
+                              L->expert_stride, nullptr) &&
+                   full_supported(L->dtype, T, L->n_experts, L->top_k, L->dim, L->expert_hidden, L->experts,
+                                  L->expert_stride, nullptr)
+               ? kMoeGroupedFull
+               : kMoeGeneral;
+}
+
+// How many of n leading prompt positions of the single sequence are to be run in blocks (0: none, token by
+// token), with the buffers for them in place. Where they cannot be had, the tokens run one by one; -1 where
+// the stream itself fails.
+int prompt_reserve(rbt_hip *h, int n) {
+    const rbt_config &c = h->cfg;
+    const int qd = c.n_heads * c.head_dim, kvd = c.n_kv_heads * c.head_dim, T = std::min(n, kPromptBlock);
+    if (n < kPromptMinTokens || !dense_full_supported(c.dtype, T, c.dim, nullptr) ||
+        !dense_full_supported(c.dtype, T, qd, nullptr))
+        return 0;
+    PromptBuf &p = h->prompt;
+    if (T <= p.tokens) return n;
+    rbt_moe_layer ml;
+    if (!rbt_hip_layer(h, 0, &ml)) return 0;
+    size_t off = 0;
+    auto carve = [&](size_t floats) {
+        const size_t at = off;
+        off += up256(4 * floats);
+        return at;
+    };
+    const size_t t = (size_t)T, ox = carve(t * c.dim), oxb = carve(t * c.dim), oq = carve(t * qd), ok = carve(t * kvd),
+                 ov = carve(t * kvd), oa = carve(t * qd), om = off;
+    // room for either form at any block length up to T
+    off += std::max(moe_scratch_bytes(T, c.n_experts, c.top_k, c.expert_hidden, c.dim, kMoeGroupedFull),
+                    moe_scratch_bytes(T, c.n_experts, c.top_k, c.expert_hidden, c.dim, kMoeGeneral));
+    uint8_t *b = nullptr;
+    if (p.block) {  // smaller ones, which earlier work on the stream may still use
+        if (HIP_TRY(hipStreamSynchronize(h->stream)) != hipSuccess) return -1;
+        (void)hipFree(p.block);
+        p = PromptBuf{};
+    }
+    if (HIP_TRY(hipMalloc(&b, off)) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    p.block = b;
+    p.tokens = T;
+    p.x = reinterpret_cast<float *>(b + ox);
+    p.xb = reinterpret_cast<float *>(b + oxb);
+    p.q = reinterpret_cast<float *>(b + oq);
+    p.k = reinterpret_cast<float *>(b + ok);
+    p.v = reinterpret_cast<float *>(b + ov);
+    p.ao = reinterpret_cast<float *>(b + oa);
+    p.moe = b + om;
+    return n;
+}
+
+// forward() (rabbit2.c:453-542, without the final norm and lm_head) of positions p0 .. p0 + T - 1 of the
+// single sequence, whose tokens are in seq[] and whose earlier positions are in the cache. Everything is
+// enqueued on the handle stream.
+int prompt_block(rbt_hip *h, int p0, int T) {
+    const rbt_config &c = h->cfg;
+    const DecodeState &ds = h->ds;
+    const PromptBuf &p = h->prompt;
+    const int D = c.dim, hd = c.head_dim, qd = c.n_heads * hd, kvd = c.n_kv_heads * hd;
+    Launch L;
+    L.s = h->stream;
+    auto vec = [&](uint64_t off) { return reinterpret_cast<const float *>(h->model + off); };
+    const int32_t *user_counts = h->expert_counts;  // rbt_hip_expert_counts_dev is about the caller's calls
+    HIP_OK(h, launch_prompt_embed(L, c.dtype, h->model + h->tok_emb, D, c.vocab, ds.seq + p0, T, p.x));
+    for (int l = 0; l < c.n_layers; l++) {
+        const LayerOff &ly = h->layers[(size_t)l];
+        const void *W[3] = {h->model + ly.wq, h->model + ly.wk, h->model + ly.wv};
+        const void *Wo[3] = {h->model + ly.wo, nullptr, nullptr};
+        float *const out[3] = {p.q, p.k, p.v}, *const no_out[3] = {nullptr, nullptr, nullptr};
+        const int rows[3] = {qd, kvd, kvd}, wo_rows[3] = {D, 0, 0};
+        float *kc = ds.kc + (size_t)l * ds.ctx * kvd, *vc = ds.vc + (size_t)l * ds.ctx * kvd;
+        HIP_OK(h, launch_rmsnorm(L, p.x, vec(ly.attn_norm), D, c.rms_eps, p.xb, T));
+        HIP_OK(h, launch_dense_full(L, c.dtype, p.xb, T, D, W, out, rows, nullptr));
+        HIP_OK(h, launch_prompt_rope(L, p.q, p.k, p.v, c.qk_norm ? vec(ly.q_norm) : p.q,
+                                     c.qk_norm ? vec(ly.k_norm) : p.k, c.qk_norm, c.rms_eps, c.n_heads, c.n_kv_heads, hd,
+                                     p0, T, kc, vc, ds.rope_cs));
+        HIP_OK(h, launch_prompt_attention(L, p.q, c.n_heads, c.n_kv_heads, hd, p0, T, kc, vc, p.ao));
+        HIP_OK(h, launch_dense_full(L, c.dtype, p.ao, T, qd, Wo, no_out, wo_rows, p.x));
+        HIP_OK(h, launch_rmsnorm(L, p.x, vec(ly.ffn_norm), D, c.rms_eps, p.xb, T));
+        rbt_moe_layer ml;
+        if (!rbt_hip_layer(h, l, &ml)) return 0;
+        const MoeForm form = prompt_form(h, &ml, T);
+        Workspace w = scratch_view(p.moe, T, c.n_experts, c.top_k, c.expert_hidden, D, form);
+        if (!moe_block(h, &ml, p.xb, T, p.x, nullptr, nullptr, nullptr, w, form, false)) return 0;
+        if (h->rhist)
+            HIP_OK(h, launch_prompt_record(L, w.routing, l, c.n_layers, c.top_k, p0, T, h->rhist));
+    }
+    h->expert_counts = user_counts;
+    return 1;
 }
 
 }  // namespace
@@ -1062,6 +1184,7 @@ void rbt_hip_free(rbt_hip *h) {
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     ws_release(h->ws);
     (void)hipFree(h->ds.block);
+    (void)hipFree(h->prompt.block);
     for (int k = 0; k < kProfCount; k++) {
         for (int j = 0; j < 2; j++)
             if (h->prof.ev[k][j]) (void)hipEventDestroy(h->prof.ev[k][j]);
@@ -1572,6 +1695,8 @@ int rbt_hip_batch_init(rbt_hip *h, int n_seq, int ctx) {
     HIP_OK(h, hipStreamSynchronize(h->stream));
     (void)hipFree(h->ds.block);
     h->ds = DecodeState{};
+    (void)hipFree(h->prompt.block);
+    h->prompt = PromptBuf{};
     (void)hipFree(h->rhist);
     h->rhist = nullptr;
     DecodeState ds;
@@ -1718,7 +1843,10 @@ int rbt_hip_generate_stream(rbt_hip *h, const int32_t *prompt, int n_prompt, int
         HIP_OK(h, hipHostMalloc(&h->tok_host, sizeof(int32_t) * (size_t)n_gen, hipHostMallocDefault));
         h->tok_host_n = n_gen;
     }
-    const StepState st{0, n_prompt, 0, 0, h->seed ? h->seed : 0x9E3779B97F4A7C15ull, 0};  // rabbit2.c:723
+    // the prompt's positions before its last, in blocks where that pays; the rest step by step
+    const int blocked = prompt_reserve(h, n_prompt - 1);
+    if (blocked < 0) return fail(h, "generate: %s failed", failed_call());
+    const StepState st{blocked, n_prompt, 0, 0, h->seed ? h->seed : 0x9E3779B97F4A7C15ull, 0};  // rabbit2.c:723
     HIP_OK(h, hipMemcpyAsync(h->ds.seq, prompt, 4 * (size_t)n_prompt, hipMemcpyHostToDevice, h->stream));
     HIP_OK(h, hipMemcpyAsync(h->ds.st, &st, sizeof st, hipMemcpyHostToDevice, h->stream));
     const int prof = h->prof.mode;
@@ -1749,7 +1877,12 @@ int rbt_hip_generate_stream(rbt_hip *h, const int32_t *prompt, int n_prompt, int
     for (int i = 0; i < 4 && e == hipSuccess; i++) e = HIP_TRY(hipEventCreate(&ev[i]));
     if (e == hipSuccess) e = HIP_TRY(hipEventRecord(ev[0], h->stream));
     // the prompt: n_prompt forwards, the last one with lm_head + argmax (the first generated token)
-    for (int p = 0; p + 1 < n_prompt && e == hipSuccess; p++) e = HIP_TRY(hipGraphLaunch(g_adv, h->stream));
+    for (int p = 0; p < blocked && e == hipSuccess; p += kPromptBlock)
+        if (!prompt_block(h, p, std::min(kPromptBlock, blocked - p))) {
+            cleanup();
+            return 0;
+        }
+    for (int p = blocked; p + 1 < n_prompt && e == hipSuccess; p++) e = HIP_TRY(hipGraphLaunch(g_adv, h->stream));
     int n = n_gen;
     bool window = false;  // ev[3] recorded: before generated step t0, else with ev[2]
     auto mark_window = [&](int g) -> hipError_t {

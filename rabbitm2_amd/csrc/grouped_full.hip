@@ -32,6 +32,12 @@ struct FullArgs {
     int E;
     float *out;            // output rows in list order, out_stride floats apart
     int out_stride;
+    // dense form: T rows through up to three weight matrices [seg_rows][Kd], out[s][t][seg_rows[s]] (added to,
+    // with resid)
+    const uint8_t *seg_w[3];
+    float *seg_out[3];
+    int seg_rows[3];
+    int T, resid;
 };
 
 // x = hi + mid + lo exactly, each part a bf16 (its upper 16 bits): 8 + 8 + 8 bits of the significand by
@@ -57,7 +63,11 @@ __device__ __forceinline__ uint32_t pack_hi16(uint32_t a, uint32_t b) { return (
 //     three v_mfma_f32_16x16x32_bf16 per 32 columns; every product is exact in the f32 accumulator;
 //   f32 weights: v_mfma_f32_16x16x4_f32.
 // The sums are no further from 64 bits than the GEMVs' lanes and trees: bf16, a step's products are summed
-// from zero (the small parts first), eight steps' sums are added up, and those to the running sums; f32,
+// from zero (the small parts first), eight steps' sums are added up, and those to the running sums; every
+// other step multiplies the negated activations and is subtracted, because the bf16 products' sums are not
+// rounded to nearest: their errors lean one way, and what the errors of many rows have in common does not
+// average out behind the kernel as their values do (a 400-token prompt, whose attention averages 400 value
+// rows: logits 3.4-3.8e-7 from 64 bits without this, 2.4-2.6e-7 with it, 2.5-2.7e-7 token by token). f32:
 // 16 columns' products are summed from zero and added to the running sums, which carry their rounding
 // errors along. The tile order and the rotation of the k-steps by weight tile are
 // prefill.hip's (the row tiles of a weight tile run together on one XCD and stay in step).
@@ -71,7 +81,7 @@ __device__ __forceinline__ uint32_t pack_hi16(uint32_t a, uint32_t b) { return (
 // lists (spills).
 // GR: bytes per weight load, from the rows' alignment (16, 4 or 2); the last k-step of a row may be
 // partial: its loads are clamped into the row and the parts past the end set to zero.
-template <int DT, int MATS, int RG, int GR>
+template <int DT, int MATS, int RG, int GR, bool DENSE = false>
 __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const FullArgs a) {
     constexpr int ESZ = DT == RBT_DT_BF16 ? 2 : 4, KW = kFullWin / ESZ;  // columns per k-step
     constexpr int ROWS = 16 * RG, NT = 64 * kFullWaves, NCOL = (MATS == 2 ? 16 : 32) * kFullWaves;
@@ -80,18 +90,42 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
     constexpr int UNITS = ROWS * 8, AU = (UNITS + NT - 1) / NT;     // activation units of KW / 8 columns
     constexpr int UL = KW / 32;                                      // 16-byte loads per unit
     constexpr int SLOTS = kFullAhead + 1;  // register sets of weights
+    constexpr uint32_t kNegate = 0x80008000u;  // the sign bits of two bf16
     constexpr int AS = AU * UL > 2 ? 2 : SLOTS;  // register sets of activations (two where a set is large)
     __shared__ __align__(1024) uint8_t ring[2 * STAGE];
     const int tid = threadIdx.x, lane = tid & 63, W = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int ntiles_n = (a.N + NCOL - 1) / NCOL;
-    const int total = a.m_off[a.E] * ntiles_n, range = (total + 7) >> 3;
+    int ntiles_n, total, e = 0, jt, il, row0, rows, n0, N = a.N, seg = 0;
+    if constexpr (DENSE) {
+        ntiles_n = 0;
+#pragma unroll
+        for (int s = 0; s < 3; ++s) ntiles_n += (a.seg_rows[s] + NCOL - 1) / NCOL;
+        total = ntiles_n * ((a.T + ROWS - 1) / ROWS);
+    } else {
+        ntiles_n = (a.N + NCOL - 1) / NCOL;
+        total = a.m_off[a.E] * ntiles_n;
+    }
+    const int range = (total + 7) >> 3;
     const int slot = (int)(blockIdx.x >> 3), tau = (int)(blockIdx.x & 7) * range + slot;
     if (slot >= range || tau >= total) return;
-    int e, jt, il;
-    tile_of(tau, a.m_off, a.E, ntiles_n, (__builtin_amdgcn_readfirstlane(*a.choice) >> 1) & 1, &e, &jt, &il);
-    const int row0 = a.offsets[e] + il * ROWS;
-    const int rows = __builtin_amdgcn_readfirstlane(min(ROWS, a.counts[e] - il * ROWS));
-    const int n0 = jt * NCOL;
+    if constexpr (DENSE) {
+        const int mt = (a.T + ROWS - 1) / ROWS;
+        jt = tau / mt;
+        il = tau - jt * mt;
+        row0 = il * ROWS;
+        rows = min(ROWS, a.T - row0);
+        int j = jt;
+        while (seg < 2 && j >= (a.seg_rows[seg] + NCOL - 1) / NCOL) {
+            j -= (a.seg_rows[seg] + NCOL - 1) / NCOL;
+            ++seg;
+        }
+        n0 = j * NCOL;
+        N = a.seg_rows[seg];
+    } else {
+        tile_of(tau, a.m_off, a.E, ntiles_n, (__builtin_amdgcn_readfirstlane(*a.choice) >> 1) & 1, &e, &jt, &il);
+        row0 = a.offsets[e] + il * ROWS;
+        rows = __builtin_amdgcn_readfirstlane(min(ROWS, a.counts[e] - il * ROWS));
+        n0 = jt * NCOL;
+    }
     const int rowb = a.Kd * ESZ;  // bytes per weight row
     const int nch = (rowb + kFullWin - 1) / kFullWin;
     const bool tail = rowb % kFullWin != 0;
@@ -106,11 +140,11 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
             const int n = n0 + (MATS == 2 ? 16 * W : 32 * W + 16 * g) + 8 * s2 + (lane & 7);
-            wp[g][s2] = a.experts + (size_t)e * a.stride + (MATS == 2 && g ? a.w3_off : a.w_off) +
-                        (size_t)min(n, a.N - 1) * (size_t)rowb;
+            const uint8_t *base = DENSE ? a.seg_w[seg] : a.experts + (size_t)e * a.stride + (MATS == 2 && g ? a.w3_off : a.w_off);
+            wp[g][s2] = base + (size_t)min(n, N - 1) * (size_t)rowb;
         }
     // activation units of this thread: row u / 8, granule u % 8 of the step's KW columns
-    const size_t base_row = a.gather ? 0 : (size_t)row0;
+    const size_t base_row = !DENSE && a.gather ? 0 : (size_t)row0;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float *>(a.act) + base_row * (size_t)a.act_stride, 0, kWrBufRecords, kBufConfig);
     uint32_t aoff[AU], adst[AU];
@@ -119,7 +153,7 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
     for (int i = 0; i < AU; ++i) {
         const int u = tid + NT * i, r = u >> 3, g = u & 7;
         const int lr = row0 + (r < rows ? r : 0);
-        const size_t arow = a.gather ? (size_t)(a.perm[lr] / a.topk) : (size_t)lr;
+        const size_t arow = !DENSE && a.gather ? (size_t)(a.perm[lr] / a.topk) : (size_t)lr;
         acol[i] = (KW / 8) * g;
         aoff[i] = r < rows ? (uint32_t)((arow - base_row) * a.act_stride + acol[i]) * 4u : (uint32_t)kWrBufRecords;
         adst[i] = (uint32_t)(r * kFullWin + 16 * (g ^ ((r >> 1) & 7)));
@@ -138,7 +172,7 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
                 av[i][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0);
             }
     };
-    auto store_a = [&](const u32x4 (&av)[AU][UL], int buf) {
+    auto store_a = [&](const u32x4 (&av)[AU][UL], int buf, uint32_t flip) {
         uint8_t *st = ring + buf * STAGE;
 #pragma unroll
         for (int i = 0; i < AU; ++i) {
@@ -153,7 +187,7 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
                     split3(__uint_as_float(av[i][j >> 1][2 * (j & 1)]), x0[0], x0[1], x0[2]);
                     split3(__uint_as_float(av[i][j >> 1][2 * (j & 1) + 1]), x1[0], x1[1], x1[2]);
 #pragma unroll
-                    for (int q = 0; q < 3; ++q) p[q][j] = pack_hi16(x0[q], x1[q]);
+                    for (int q = 0; q < 3; ++q) p[q][j] = pack_hi16(x0[q], x1[q]) ^ flip;
                 }
 #pragma unroll
                 for (int q = 0; q < 3; ++q) *reinterpret_cast<u32x4 *>(st + q * ABYTES + adst[i]) = p[q];
@@ -224,7 +258,7 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
     auto step = [&](auto jc, auto fullc, int c) {
         constexpr int J = decltype(jc)::value;
         constexpr bool FULL = decltype(fullc)::value;
-        if (FULL || c + 1 < nch) store_a(aset[(J + 1) % AS], (c + 1) & 1);  // the buffer that step c - 1 read
+        if (FULL || c + 1 < nch) store_a(aset[(J + 1) % AS], (c + 1) & 1, J & 1 ? 0u : kNegate);  // the buffer that step c - 1 read
         if (FULL || c + AS < nch) load_a(aset[J % AS], c + AS);
         if (FULL || c + kFullAhead < nch) load_w(wv[(J + kFullAhead) % SLOTS], c + kFullAhead);
         const uint8_t *st = ring + (c & 1) * STAGE;
@@ -271,8 +305,8 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
                     }
                 }
                 if constexpr (DT == RBT_DT_BF16) {
-                    mid[q][0] += t[0];
-                    mid[q][1] += t[1];
+                    mid[q][0] = J & 1 ? mid[q][0] - t[0] : mid[q][0] + t[0];
+                    mid[q][1] = J & 1 ? mid[q][1] - t[1] : mid[q][1] + t[1];
                 }
             }
         }
@@ -289,7 +323,7 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
         if (p < AS && p < nch) load_a(aset[p % AS], p);
         if (p < kFullAhead && p < nch) load_w(wv[p], p);
     }
-    store_a(aset[0], 0);
+    store_a(aset[0], 0, 0u);
     __syncthreads();
     int c = 0;
     for (; c + 2 * SLOTS <= nch; c += SLOTS) {
@@ -314,7 +348,7 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
         for (int i = 0; i < 4; ++i) {
             const int r = 16 * q + 4 * (lane >> 4) + i;
             if (r >= rows) continue;
-            float *orow = a.out + (size_t)(row0 + r) * a.out_stride;
+            float *orow = DENSE ? a.seg_out[seg] + (size_t)(row0 + r) * N : a.out + (size_t)(row0 + r) * a.out_stride;
             if constexpr (MATS == 2) {
                 const int n = n0 + 16 * W + (lane & 15);
                 const float g = acc[q][0][i], u = acc[q][1][i];
@@ -324,7 +358,7 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
 #pragma unroll
                 for (int g = 0; g < 2; ++g) {
                     const int n = n0 + 32 * W + 16 * g + (lane & 15);
-                    if (n < a.N) orow[n] = acc[q][g][i];
+                    if (n < N) orow[n] = DENSE && a.resid ? orow[n] + acc[q][g][i] : acc[q][g][i];
                 }
             }
         }
@@ -337,16 +371,25 @@ int load_granule(uint64_t base, uint64_t stride, int Kd, int esz) {
     return bits % 16 == 0 ? 16 : bits % 4 == 0 ? 4 : bits % 2 == 0 && esz == 2 ? 2 : 0;
 }
 
-template <int MATS>
+template <int MATS, bool DENSE = false>
 hipError_t launch_full(const Launch &L, const FullArgs &a, int dtype, int rg, int max_mtiles) {
     constexpr int NCOL = (MATS == 2 ? 16 : 32) * kFullWaves;
-    const long long tiles = (long long)max_mtiles * ((a.N + NCOL - 1) / NCOL), blocks = (tiles + 7) / 8 * 8;
-    const int gr = load_granule(reinterpret_cast<uintptr_t>(a.experts) | a.w_off | a.w3_off, a.stride, a.Kd,
-                                dtype == RBT_DT_BF16 ? 2 : 4);
+    int ntiles_n = (a.N + NCOL - 1) / NCOL;
+    uint64_t base = reinterpret_cast<uintptr_t>(a.experts) | a.w_off | a.w3_off;
+    if (DENSE) {
+        ntiles_n = 0;
+        base = 0;
+        for (int s = 0; s < 3; ++s) {
+            ntiles_n += (a.seg_rows[s] + NCOL - 1) / NCOL;
+            if (a.seg_rows[s]) base |= reinterpret_cast<uintptr_t>(a.seg_w[s]);
+        }
+    }
+    const long long tiles = (long long)max_mtiles * ntiles_n, blocks = (tiles + 7) / 8 * 8;
+    const int gr = load_granule(base, a.stride, a.Kd, dtype == RBT_DT_BF16 ? 2 : 4);
     if (blocks > 0x7FFFFFFFll || gr == 0) return hipErrorInvalidValue;
     const dim3 g((unsigned)blocks), b(64 * kFullWaves);
 #define FULL_CASE(DT, RG, GR) \
-    if (dtype == DT && rg == RG && gr == GR) return launch(L, grouped_full_kernel<DT, MATS, RG, GR>, g, b, 0, a);
+    if (dtype == DT && rg == RG && gr == GR) return launch(L, grouped_full_kernel<DT, MATS, RG, GR, DENSE>, g, b, 0, a);
 #define FULL_TILES(DT, GR)  \
     FULL_CASE(DT, 2, GR) \
     FULL_CASE(DT, 4, GR)
@@ -364,6 +407,7 @@ hipError_t launch_full(const Launch &L, const FullArgs &a, int dtype, int rg, in
 // that passes 32 rows re-reads its weights from L2 (f32 200 tokens, 25 rows on average: 250 us either way;
 // with +2 on eight experts' logits 304 against 384 us).
 constexpr int kFullShortLists = 40;
+constexpr int kDenseTallTiles = 256;  // dense form: 64-row tiles from which they are taken
 
 }  // namespace
 
@@ -399,6 +443,31 @@ size_t full_workspace_bytes(int T, int E, int K, int D) {
     return up(4 * (size_t)E) + 3 * up(4 * (size_t)(E + 1)) + up(4) + 2 * up(4 * P) + up(4 * P * (size_t)D);
 }
 
+bool dense_full_supported(int dtype, int T, int Kd, const float *x) {
+    // row stride and alignment of x as the buffer loads need them; the model's tensors are 64-byte aligned
+    return T >= 1 && T <= 65535 && Kd % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 &&
+           load_granule(0, 0, Kd, dtype == RBT_DT_BF16 ? 2 : 4) != 0 && 128ull * Kd * 4 < (uint64_t)kWrBufRecords;
+}
+
+hipError_t launch_dense_full(const Launch &L, int dtype, const float *x, int T, int Kd, const void *const W[3],
+                             float *const out[3], const int rows[3], float *resid) {
+    FullArgs a{};
+    a.Kd = Kd;
+    a.act = x;
+    a.act_stride = Kd;
+    a.T = T;
+    a.resid = resid != nullptr;
+    int tiles64 = 0;
+    for (int s = 0; s < 3; ++s) {
+        a.seg_w[s] = static_cast<const uint8_t *>(W[s]);
+        a.seg_out[s] = resid ? resid : out[s];
+        a.seg_rows[s] = rows[s];
+        tiles64 += (rows[s] + 32 * kFullWaves - 1) / (32 * kFullWaves) * ((T + 63) / 64);
+    }
+    const int rg = tiles64 >= kDenseTallTiles ? 4 : 2;
+    return launch_full<1, true>(L, a, dtype, rg, (T + 16 * rg - 1) / (16 * rg));
+}
+
 hipError_t launch_grouped_full(const Launch &Ld, const Launch &Lg, const Launch &Lw, const Launch &Lc, int dtype,
                                const void *experts, uint64_t stride, const float *xb, int T, int E, int K, int D, int H,
                                const int32_t *routing, const float *weights, float *hbuf, void *ws, float *x_inout,
@@ -428,10 +497,10 @@ hipError_t launch_grouped_full(const Launch &Ld, const Launch &Lg, const Launch 
     const uint64_t mat = (uint64_t)H * D * (dtype == RBT_DT_BF16 ? 2 : 4);
     const int hs = full_h_stride(H);
     const uint8_t *ex = static_cast<const uint8_t *>(experts);
-    FullArgs a{ex, stride, 0, mat, H, D, xb, D, 1, perm, K, counts, offsets, m_off, choice, E, hbuf, hs};
+    FullArgs a{ex, stride, 0, mat, H, D, xb, D, 1, perm, K, counts, offsets, m_off, choice, E, hbuf, hs, {}, {}, {}, 0, 0};
     e = launch_full<2>(Lg, a, dtype, rg, max_mtiles);
     if (e != hipSuccess) return e;
-    a = FullArgs{ex, stride, 2 * mat, 0, D, H, hbuf, hs, 0, perm, K, counts, offsets, m_off, choice, E, y, D};
+    a = FullArgs{ex, stride, 2 * mat, 0, D, H, hbuf, hs, 0, perm, K, counts, offsets, m_off, choice, E, y, D, {}, {}, {}, 0, 0};
     e = launch_full<1>(Lw, a, dtype, rg, max_mtiles);
     if (e != hipSuccess) return e;
     return launch_combine(Lc, y, pos_of, weights, T, K, D, x_inout, moe_out);

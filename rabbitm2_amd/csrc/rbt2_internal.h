@@ -264,6 +264,27 @@ hipError_t launch_grouped_full(const Launch &Ld, const Launch &Lg, const Launch 
                                const int32_t *routing, const float *weights, float *hbuf, void *ws, float *x_inout,
                                float *moe_out, int32_t **counts_out);
 
+// Rows of T tokens through up to three dense matrices on the same kernel (full f32 activation precision):
+// out_s [T][rows_s] = x W_s^T, or with resid != NULL resid [T][rows_0] += (one matrix).
+bool dense_full_supported(int dtype, int T, int Kd, const float *x);
+hipError_t launch_dense_full(const Launch &L, int dtype, const float *x, int T, int Kd, const void *const W[3],
+                             float *const out[3], const int rows[3], float *resid);
+
+// ---- a prompt read in as a block of positions p0 .. p0 + T - 1 of sequence 0 (prompt.hip)
+// The embedding rows of the tokens seq[0 .. T).
+hipError_t launch_prompt_embed(const Launch &L, int dtype, const void *emb, int D, int vocab, const int32_t *seq, int T,
+                               float *x);
+// QK-norm and RoPE of the rows q, k: q rotated in place, k and v into the caches' rows p0 + t.
+hipError_t launch_prompt_rope(const Launch &L, float *q, const float *k, const float *v, const float *qw,
+                              const float *kw, int qk_norm, float eps, int n_heads, int n_kv, int hd, int p0, int T,
+                              float *kc, float *vc, const float2 *rope_cs);
+// Causal attention of those T positions over the cached rows, ao [T][n_heads * hd].
+hipError_t launch_prompt_attention(const Launch &L, const float *q, int n_heads, int n_kv, int hd, int p0, int T,
+                                   const float *kc, const float *vc, float *ao);
+// One layer's routing [T][K] into the routing history [ctx][n_layers][K] at positions p0 + t.
+hipError_t launch_prompt_record(const Launch &L, const int32_t *routing, int layer, int n_layers, int K, int p0, int T,
+                                int32_t *hist);
+
 // Router logits + softmax + top-k + the activation hi/lo split in one launch, for the grouped path
 // (AVX2 order, E <= 64). x_hi/x_lo may be NULL (no split).
 bool router_prefill_supported(int order, int dtype, int T, int E, int D, int K, const void *W, const float *xb);
