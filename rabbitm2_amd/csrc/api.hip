@@ -978,7 +978,11 @@ int moe_block(rbt_hip *h, const rbt_moe_layer *L, const float *xb_dev, int T, fl
         // kernels (the grouped path then splits the activations itself)
         const bool fused = router_prefill_supported(h->order, L->dtype, T, L->n_experts, L->dim, L->top_k,
                                                     L->router, xb_dev);
-        if (fused && T <= kRouterDecodeMaxT) {  // few tokens: decode router kernel, then top-k + split
+        // few tokens, or the scalar order: the logits, then top-k + split (scalar order, 512 tokens: 4.7 us
+        // against 7.4 + 7 us for the top-k and the split on their own)
+        const bool split = (fused && T <= kRouterDecodeMaxT) ||
+                           (h->order == RBT_ORDER_SCALAR && L->n_experts <= 64 && L->top_k <= L->n_experts);
+        if (split) {
             uint16_t *x_hi = nullptr, *x_lo = nullptr;
             prefill_x_planes(w.pre, T, L->n_experts, L->top_k, L->dim, &x_hi, &x_lo);
             HIP_OK(h, launch_router_logits(lc(h, kProfRouter), h->order, L->dtype, xb_dev, L->router, L->router_bias, T,
@@ -999,8 +1003,8 @@ int moe_block(rbt_hip *h, const rbt_moe_layer *L, const float *xb_dev, int T, fl
         int32_t *counts = nullptr;
         HIP_OK(h, launch_prefill(lc(h, kProfDispatch), lc(h, kProfGateup), lc(h, kProfDown), lc(h, kProfCombine),
                                  L->experts, L->expert_stride, xb_dev, T, L->n_experts, L->top_k, L->dim,
-                                 L->expert_hidden, routing, weights, w.hbuf, w.pre, x_dev, moe_dev, &counts, fused,
-                                 true, h->prefill_tile_rows, tiled_for(h, L), h->prefill_wide));
+                                 L->expert_hidden, routing, weights, w.hbuf, w.pre, x_dev, moe_dev, &counts,
+                                 fused || split, true, h->prefill_tile_rows, tiled_for(h, L), h->prefill_wide));
         h->expert_counts = counts;
         return done();
     }

@@ -175,8 +175,8 @@ hipError_t launch_router(const Launch &L, const Launch &Lk, int order, int dtype
 constexpr int kRouterDecodeMaxT = 64;
 // (sequence, head) attention blocks from which a step takes one position split (no merge launch).
 constexpr int kAttnDirectBlocks = 512;
-// Softmax + top-k of T tokens' logits [T][E] (E <= 64) and the bf16 hi/lo split of their rows xb [T][D]
-// (D % 8 == 0, 16-byte aligned) into x_hi / x_lo [T][D]: one block per token.
+// Softmax + top-k of T tokens' logits [T][E] (E <= 64) and, with x_hi / x_lo [T][D], the bf16 hi/lo split of
+// their rows xb [T][D] (D % 8 == 0, 16-byte aligned): one block per token.
 hipError_t launch_topk_split(const Launch &L, const float *logits, int T, int E, int K, int norm_topk, const float *xb,
                              int D, int32_t *routing, float *weights, uint16_t *x_hi, uint16_t *x_lo);
 // Router logits (AVX2 order, few tokens, bf16) with the RMSNorm in front folded in: x [T][D] is the

@@ -421,7 +421,7 @@ __device__ __forceinline__ void wave_softmax_topk(float v, int E, int K, int nor
 }
 
 // Softmax + top-k of token t's E <= 64 logits (wave 0 of block t, the engine's arithmetic as above) and
-// the bf16 hi/lo split of its activation row (every thread, 8 elements per 16-byte pair): the grouped
+// (with x_hi) the bf16 hi/lo split of its activation row (every thread, 8 elements per 16-byte pair): the grouped
 // expert path's front end for a few tokens whose logits and normalised rows router_decode_kernel<M,
 // true> has just written (E / 2 or E / 4 x T blocks for the chains instead of the fused prefill kernel's one
 // block per two tokens).
@@ -434,7 +434,7 @@ __global__ __launch_bounds__(256) void topk_split_kernel(const float *__restrict
     const int t = blockIdx.x, tid = threadIdx.x;
     const float v = tid < E ? logits[(size_t)t * E + tid] : 0.0f;
     const size_t row = (size_t)t * D;
-    for (int u = tid; u < D / 8; u += blockDim.x) {
+    for (int u = tid; x_hi && u < D / 8; u += blockDim.x) {
         const f32x4 a = ld_f4(xb + row + 8 * u), b = ld_f4(xb + row + 8 * u + 4);
         const float x8[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
         uint32_t hb[8], lb[8];
@@ -741,6 +741,167 @@ __global__ __launch_bounds__(256) void router_logits_batch_kernel(const float *_
     }
 }
 
+// Few tokens, either order, either type, where router_decode_kernel does not apply: the scalar order (whose
+// four chains of D / 4 dependent adds are the long pole) and f32 rows. One 128-thread block per two router
+// rows of one token. Every thread forms rounded products, four steps of four neighbouring chains at a time,
+// and stores them transposed, pt[row][chain][step]; then one lane per (row, chain) adds its line, four steps
+// per 16-byte read, so that a step of the chain is one add and nothing else (dim 2048, 64 rows, one token:
+// f32 scalar 24.8 -> 6.0 us, bf16 scalar 17.6 -> 6.4 us, f32 AVX2 7.6 -> 4.3 us, against chains that
+// multiply as they go).
+// D a multiple of 4 NCH, 16-byte aligned rows.
+constexpr int kFewRows = 2, kFewThreads = 128, kFewMaxLds = 65536;
+template <int NCH, int DT>
+__global__ __launch_bounds__(kFewThreads) void router_few_kernel(const float *__restrict__ xb, const void *__restrict__ Wv,
+                                                                 const float *__restrict__ bias, int E, int D,
+                                                                 float *__restrict__ logits) {
+    using W = typename RouterTile<DT, false>::W;
+    extern __shared__ __align__(16) float pt[];
+    const W *Wg = static_cast<const W *>(Wv);
+    const int tid = threadIdx.x, t = blockIdx.y, r0 = blockIdx.x * kFewRows;
+    const int M = D / NCH, pitch = M + 4;  // steps per chain; floats per chain line
+    const float *x = xb + (size_t)t * D;
+    // task u: chains 4 cq .. 4 cq + 3, steps 4 v .. 4 v + 3 (columns NCH (4 v + i) + 4 cq + j)
+    for (int u = tid; u < D / 16; u += kFewThreads) {
+        const int cq = u % (NCH / 4), v = u / (NCH / 4);
+        f32x4 xv[4], wv[kFewRows][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xv[i] = ld_f4(x + NCH * (4 * v + i) + 4 * cq);
+#pragma unroll
+        for (int rr = 0; rr < kFewRows; ++rr) {
+            const W *row = Wg + (size_t)min(r0 + rr, E - 1) * D + 4 * cq;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (DT == RBT_DT_F32) {
+                    wv[rr][i] = ld_f4(row + NCH * (4 * v + i));
+                } else {
+                    const uint2 p = *reinterpret_cast<const uint2 *>(row + NCH * (4 * v + i));
+                    wv[rr][i] = f32x4{bf16_lo(p.x), bf16_hi(p.x), bf16_lo(p.y), bf16_hi(p.y)};
+                }
+            }
+        }
+#pragma unroll
+        for (int rr = 0; rr < kFewRows; ++rr)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                *reinterpret_cast<f32x4 *>(pt + (size_t)(rr * NCH + 4 * cq + j) * pitch + 4 * v) =
+                    f32x4{wv[rr][0][j] * xv[0][j], wv[rr][1][j] * xv[1][j], wv[rr][2][j] * xv[2][j], wv[rr][3][j] * xv[3][j]};
+    }
+    __syncthreads();
+    if (tid >= kWave) return;
+    const f32x4 *line = reinterpret_cast<const f32x4 *>(pt + (size_t)min(tid, kFewRows * NCH - 1) * pitch);
+    float acc = 0.0f;
+    // eight reads in flight ahead of the adds
+    f32x4 cur[8], nxt[8];
+    const int n4 = M / 4;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) cur[i] = line[min(i, n4 - 1)];
+    for (int m = 0; m < n4; m += 8) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) nxt[i] = line[min(m + 8 + i, n4 - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (m + i < n4) {  // wave-uniform
+                acc = acc + cur[i].x;
+                acc = acc + cur[i].y;
+                acc = acc + cur[i].z;
+                acc = acc + cur[i].w;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) cur[i] = nxt[i];
+    }
+#pragma unroll
+    for (int rr = 0; rr < kFewRows; ++rr) {
+        float sum;
+        if constexpr (NCH == 16) {
+            sum = 0.0f;  // the engine's lanes a[j] + b[j], summed from j = 0
+#pragma unroll
+            for (int j = 0; j < 8; ++j) sum = sum + (lane_value(acc, 16 * rr + j) + lane_value(acc, 16 * rr + 8 + j));
+        } else {
+            sum = (lane_value(acc, 4 * rr) + lane_value(acc, 4 * rr + 1)) +
+                  (lane_value(acc, 4 * rr + 2) + lane_value(acc, 4 * rr + 3));
+        }
+        const int r = r0 + rr;
+        if (tid == rr && r < E) logits[(size_t)t * E + r] = bias ? sum + bias[r] : sum;
+    }
+}
+
+// Many tokens, scalar order: a block of 16 rows x 16 tokens, one lane per (token, row) with its four chains
+// (step m: one 16-byte read of x and one of the row, four rounded products, four adds), rows and x staged
+// through LDS a chunk at a time. D a multiple of 4, 16-byte aligned rows.
+constexpr int kScRows = 16, kScTok = 16, kScCols = 512;
+template <int DT>
+__global__ __launch_bounds__(kScRows * kScTok) void router_scalar_batch_kernel(const float *__restrict__ xb,
+                                                                           const void *__restrict__ Wv,
+                                                                           const float *__restrict__ bias, int T, int E,
+                                                                           int D, float *__restrict__ logits) {
+    using W = typename RouterTile<DT, false>::W;
+    constexpr int ESZ = (int)sizeof(W), TOK = kScTok, NT = kScRows * TOK;
+    constexpr int WP = kScCols * ESZ + 16, XP = kScCols * 4 + 16;  // row pitches in bytes
+    __shared__ __align__(16) unsigned char wt[kScRows * WP];
+    __shared__ __align__(16) unsigned char xt[TOK * XP];
+    const W *Wg = static_cast<const W *>(Wv);
+    const int tid = threadIdx.x, rl = tid & 15, tl = tid >> 4;
+    const int r0 = blockIdx.x * kScRows, t0 = blockIdx.y * TOK;
+    f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c0 = 0; c0 < D; c0 += kScCols) {
+        const int cn = min(kScCols, D - c0);
+        constexpr int per = 16 / ESZ;
+        const int wu = cn / per, wtot = kScRows * wu, xu = cn / 4, xtot = TOK * xu;
+        // 16-byte units (rows past the ends repeat the last), eight loads in flight per thread
+        for (int b0 = tid; b0 < wtot + xtot; b0 += NT * 8) {
+            u32x4 v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int u = min(b0 + i * NT, wtot + xtot - 1);
+                if (u < wtot) {
+                    const int rr = u / wu, k = u - rr * wu;
+                    v[i] = *reinterpret_cast<const u32x4 *>(Wg + (size_t)min(r0 + rr, E - 1) * D + c0 + k * per);
+                } else {
+                    const int tt = (u - wtot) / xu, k = (u - wtot) - tt * xu;
+                    v[i] = *reinterpret_cast<const u32x4 *>(xb + (size_t)min(t0 + tt, T - 1) * D + c0 + 4 * k);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int u = b0 + i * NT;
+                if (u < wtot) {
+                    const int rr = u / wu, k = u - rr * wu;
+                    *reinterpret_cast<u32x4 *>(wt + rr * WP + k * 16) = v[i];
+                } else if (u < wtot + xtot) {
+                    const int tt = (u - wtot) / xu, k = (u - wtot) - tt * xu;
+                    *reinterpret_cast<u32x4 *>(xt + tt * XP + k * 16) = v[i];
+                }
+            }
+        }
+        __syncthreads();
+        const unsigned char *wr = wt + rl * WP;
+        const float *xr = reinterpret_cast<const float *>(xt + tl * XP);
+#pragma unroll 8
+        for (int m = 0; m < cn / 4; ++m) {
+            f32x4 w;
+            if constexpr (DT == RBT_DT_F32) {
+                w = *reinterpret_cast<const f32x4 *>(wr + 16 * m);
+            } else {
+                const uint2 p = *reinterpret_cast<const uint2 *>(wr + 8 * m);
+                w = f32x4{bf16_lo(p.x), bf16_hi(p.x), bf16_lo(p.y), bf16_hi(p.y)};
+            }
+            const f32x4 x = *reinterpret_cast<const f32x4 *>(xr + 4 * m);
+            acc.x = acc.x + w.x * x.x;
+            acc.y = acc.y + w.y * x.y;
+            acc.z = acc.z + w.z * x.z;
+            acc.w = acc.w + w.w * x.w;
+        }
+        __syncthreads();
+    }
+    const int r = r0 + rl, t = t0 + tl;
+    if (r < E && t < T) {
+        const float sum = (acc.x + acc.y) + (acc.z + acc.w);
+        logits[(size_t)t * E + r] = bias ? sum + bias[r] : sum;
+    }
+}
+
 // grid (T), block 64 or 256 threads; dynamic LDS E floats when E <= kLdsProbsMax. Reads the logits
 // row of its token, leaves the probabilities in it, writes routing/weights.
 __global__ __launch_bounds__(256) void router_topk_kernel(int E, int K, int norm_topk, float *__restrict__ probs,
@@ -912,15 +1073,44 @@ inline bool batch_ok(int T, int D, int dtype, const void *W, const float *xb) {
            (D * esz) % 16 == 0 && D % 4 == 0;
 }
 
+// Tokens up to which a block per (token, row pair) beats the batch kernels (dim 2048, 64 experts, us):
+// f32 scalar order 32 tokens 8.8, 256 tokens 33.7 (batch kernel: 300 tokens 33.6); f32 AVX2 order 32 tokens
+// 5.1, 256 tokens 17.9 (batch kernel: 27.4 and 26); bf16 scalar order 32 tokens 9.5, 256 tokens 30.8 (batch
+// kernel: 300 tokens 34.0). Before either: f32 scalar 200 tokens 36.1, bf16 scalar 512 tokens 43.7, 2000
+// tokens 155 (now 43.7).
+constexpr int kFewMaxTokens = 256;
+
+// The logits by the kernels above where they apply (else hipErrorNotSupported).
+template <int NCH, int DT>
+hipError_t launch_logits_few(const Launch &L, const float *xb, const void *W, const float *bias, int T, int E, int D,
+                             float *logits) {
+    const bool al = ((reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(xb)) & 15u) == 0;
+    const size_t lds = (size_t)kFewRows * (D + 4 * NCH) * 4;
+    if (!al || T > kFewMaxTokens || D % (4 * NCH) != 0 || lds > kFewMaxLds) return hipErrorNotSupported;
+    return launch(L, router_few_kernel<NCH, DT>, dim3((unsigned)((E + kFewRows - 1) / kFewRows), (unsigned)T),
+                  dim3(kFewThreads), (uint32_t)lds, xb, W, bias, E, D, logits);
+}
+template <int DT>
+hipError_t launch_logits_scalar_batch(const Launch &L, const float *xb, const void *W, const float *bias, int T, int E,
+                                      int D, float *logits) {
+    const bool al = ((reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(xb)) & 15u) == 0;
+    if (!al || T <= 16 || D * (DT == RBT_DT_F32 ? 4 : 2) % 16 != 0) return hipErrorNotSupported;
+    return launch(L, router_scalar_batch_kernel<DT>,
+                  dim3((unsigned)((E + kScRows - 1) / kScRows), (unsigned)((T + kScTok - 1) / kScTok)),
+                  dim3(kScRows * kScTok), 0, xb, W, bias, T, E, D, logits);
+}
+
 template <int NCH, int DT>
 hipError_t launch_t(const Launch &L, const Launch &Lk, const float *xb, const void *W, const float *bias, int T, int E,
                     int D, int K, int norm_topk, float *probs, int32_t *routing, float *weights) {
-    hipError_t e;
+    hipError_t e = hipSuccess;
     if (NCH == 16 && decode_ok(T, D, DT, W, xb)) {
         e = launch_router_decode(L, xb, W, bias, T, E, D, probs);
+    } else if ((e = launch_logits_few<NCH, DT>(L, xb, W, bias, T, E, D, probs)) != hipErrorNotSupported) {
     } else if (NCH == 16 && batch_ok(T, D, DT, W, xb)) {
         e = launch(L, router_logits_batch_kernel<DT>, dim3((E + kBRows - 1) / kBRows, (T + kBTok - 1) / kBTok),
                    dim3(256), 0, xb, W, bias, T, E, D, probs);
+    } else if (NCH == 4 && (e = launch_logits_scalar_batch<DT>(L, xb, W, bias, T, E, D, probs)) != hipErrorNotSupported) {
     } else {
         // 64-thread blocks for small batches (4 or 16 rows each, so one token's router spreads over
         // many CUs); 256 threads (16 rows) for larger batches with the AVX2 order.
@@ -930,7 +1120,9 @@ hipError_t launch_t(const Launch &L, const Launch &Lk, const float *xb, const vo
                  : launch_logits<NCH, DT, false>(L, xb, W, bias, T, E, D, threads, probs);
     }
     if (e != hipSuccess) return e;
-    const int tk = E <= 64 ? 64 : 256;
+    // up to 64 experts one wave selects by ballots, a lane per expert (5 tokens 4.1 us against 7.0 by ranking)
+    if (E <= 64 && K <= E) return launch_topk_split(Lk, probs, T, E, K, norm_topk, xb, D, routing, weights, nullptr, nullptr);
+    const int tk = 256;
     const size_t lds_k = E <= kLdsProbsMax ? (size_t)E * 4 : 0;
     return launch(Lk, router_topk_kernel, dim3(T), dim3(tk), (uint32_t)lds_k, E, K, norm_topk, probs, routing,
                   weights);
@@ -944,6 +1136,9 @@ hipError_t launch_router_logits(const Launch &L, int order, int dtype, const flo
     if (T > 65535) return hipErrorInvalidValue;
     if (order == RBT_ORDER_AVX2) {
         if (decode_ok(T, D, dtype, W, xb)) return launch_router_decode(L, xb, W, bias, T, E, D, logits);
+        const hipError_t e = dtype == RBT_DT_BF16 ? launch_logits_few<16, RBT_DT_BF16>(L, xb, W, bias, T, E, D, logits)
+                                                  : launch_logits_few<16, RBT_DT_F32>(L, xb, W, bias, T, E, D, logits);
+        if (e != hipErrorNotSupported) return e;
         if (batch_ok(T, D, dtype, W, xb))
             return dtype == RBT_DT_BF16
                        ? launch(L, router_logits_batch_kernel<RBT_DT_BF16>,
@@ -959,6 +1154,12 @@ hipError_t launch_router_logits(const Launch &L, int order, int dtype, const flo
         return threads == 64 ? launch_logits<16, RBT_DT_F32, true>(L, xb, W, bias, T, E, D, 64, logits)
                              : launch_logits<16, RBT_DT_F32, false>(L, xb, W, bias, T, E, D, 256, logits);
     }
+    hipError_t e = dtype == RBT_DT_BF16 ? launch_logits_few<4, RBT_DT_BF16>(L, xb, W, bias, T, E, D, logits)
+                                        : launch_logits_few<4, RBT_DT_F32>(L, xb, W, bias, T, E, D, logits);
+    if (e == hipErrorNotSupported)
+        e = dtype == RBT_DT_BF16 ? launch_logits_scalar_batch<RBT_DT_BF16>(L, xb, W, bias, T, E, D, logits)
+                                 : launch_logits_scalar_batch<RBT_DT_F32>(L, xb, W, bias, T, E, D, logits);
+    if (e != hipErrorNotSupported) return e;
     return dtype == RBT_DT_BF16 ? launch_logits<4, RBT_DT_BF16, false>(L, xb, W, bias, T, E, D, 64, logits)
                                 : launch_logits<4, RBT_DT_F32, false>(L, xb, W, bias, T, E, D, 64, logits);
 }
@@ -975,10 +1176,11 @@ hipError_t launch_router_norm(const Launch &L, const float *x, const float *nw, 
 hipError_t launch_topk_split(const Launch &L, const float *logits, int T, int E, int K, int norm_topk, const float *xb,
                              int D, int32_t *routing, float *weights, uint16_t *x_hi, uint16_t *x_lo) {
     if (T <= 0) return hipSuccess;
-    if (T > 65535 || E < 1 || E > 64 || K < 1 || K > E || D % 8 != 0 ||
-        ((reinterpret_cast<uintptr_t>(xb) | reinterpret_cast<uintptr_t>(x_hi) | reinterpret_cast<uintptr_t>(x_lo)) & 15u))
+    if (T > 65535 || E < 1 || E > 64 || K < 1 || K > E || (x_hi == nullptr) != (x_lo == nullptr) ||
+        (x_hi && (D % 8 != 0 || ((reinterpret_cast<uintptr_t>(xb) | reinterpret_cast<uintptr_t>(x_hi) |
+                                  reinterpret_cast<uintptr_t>(x_lo)) & 15u))))
         return hipErrorInvalidValue;
-    return launch(L, topk_split_kernel, dim3((unsigned)T), dim3(256), 0, logits, E, K, norm_topk, xb, D, routing,
+    return launch(L, topk_split_kernel, dim3((unsigned)T), dim3(x_hi ? 256 : 64), 0, logits, E, K, norm_topk, xb, D, routing,
                   weights, x_hi, x_lo);
 }
 
