@@ -121,7 +121,7 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
         n0 = j * NCOL;
         N = a.seg_rows[seg];
     } else {
-        tile_of(tau, a.m_off, a.E, ntiles_n, (__builtin_amdgcn_readfirstlane(*a.choice) >> 1) & 1, &e, &jt, &il);
+        tile_of(tau, a.m_off, a.E, a.m_off[a.E], ntiles_n, (__builtin_amdgcn_readfirstlane(*a.choice) >> 1) & 1, &e, &jt, &il);
         row0 = a.offsets[e] + il * ROWS;
         rows = __builtin_amdgcn_readfirstlane(min(ROWS, a.counts[e] - il * ROWS));
         n0 = jt * NCOL;
@@ -440,7 +440,7 @@ bool full_pays(bool fast_gemv, int dtype, int T, int E, int K, int D, int H) {
 size_t full_workspace_bytes(int T, int E, int K, int D) {
     const size_t P = (size_t)T * K;
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-    return up(4 * (size_t)E) + 3 * up(4 * (size_t)(E + 1)) + up(4) + 2 * up(4 * P) + up(4 * P * (size_t)D);
+    return up(4 * (size_t)E) + 3 * up(4 * (size_t)(E + 1)) + up(8) + 2 * up(4 * P) + up(4 * P * (size_t)D);
 }
 
 bool dense_full_supported(int dtype, int T, int Kd, const float *x) {
@@ -484,14 +484,14 @@ hipError_t launch_grouped_full(const Launch &Ld, const Launch &Lg, const Launch 
     int32_t *offsets = reinterpret_cast<int32_t *>(carve(4 * (size_t)(E + 1)));
     int32_t *m_off = reinterpret_cast<int32_t *>(carve(4 * (size_t)(E + 1)));
     int32_t *m_off128 = reinterpret_cast<int32_t *>(carve(4 * (size_t)(E + 1)));  // written by the dispatch, not used
-    int32_t *choice = reinterpret_cast<int32_t *>(carve(4));
+    int32_t *choice = reinterpret_cast<int32_t *>(carve(8));
     int32_t *perm = reinterpret_cast<int32_t *>(carve(4 * (size_t)P));
     int32_t *pos_of = reinterpret_cast<int32_t *>(carve(4 * (size_t)P));
     float *y = reinterpret_cast<float *>(carve(4 * (size_t)P * D));
     if (counts_out) *counts_out = counts;
     const int rg = P <= kFullShortLists * E ? 2 : 4;
     hipError_t e = launch_dispatch(Ld, routing, P, E, counts, offsets, perm, pos_of, m_off, 16 * rg, m_off128,
-                                   choice, 2);
+                                   choice, 2, 0, reinterpret_cast<int32_t *>(y));
     if (e != hipSuccess) return e;
     const int max_mtiles = (P + 16 * rg - 1) / (16 * rg) + E;  // >= sum over experts of ceil(count / (16 rg))
     const uint64_t mat = (uint64_t)H * D * (dtype == RBT_DT_BF16 ? 2 : 4);

@@ -38,14 +38,105 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
+// Relative time of a wide 128-row tile and of a 64-row tile half as wide, for the plan that dispatch_kernel
+// makes: gate/up, dim 2048, rounds of 256 tiles take 108-120 and 38-42 us (from the second round on; one
+// round of wide tiles, 93-123 us, is never beaten). 64 experts, us per gate/up with wide / 64-row tiles:
+// evenly routed 900 tokens (280 wide tiles, 1040 of 64 rows) 211 / 191, 1024 tokens 224 / 202, 1300 tokens
+// 239 / 230, 2048 tokens 332 / 335; +2 on eight experts' logits 400 tokens (320, 768) 153 / 133, 777 tokens
+// (384, 1024) 216 / 162, 1500 tokens (512, 1600) 229 / 264.
+constexpr int kWideTileCost = 29, kShortTileCost = 10;
 constexpr int kDispRegs = 4;  // 64-pair steps per wave kept in registers by dispatch_kernel (4096 pairs)
 
+
+// One wave: the experts' totals s_tot become their first list positions; with write, also the outputs of the
+// dispatch that follow from the totals (see dispatch_kernel).
+__device__ __forceinline__ void dispatch_scan(int *s_tot, int P, int E, bool write, int32_t *__restrict__ counts,
+                                              int32_t *__restrict__ offsets, int32_t *__restrict__ m_off, int mt_rows,
+                                              int32_t *__restrict__ m_off2, int32_t *__restrict__ choice, int tall,
+                                              int wide_nt) {
+    const int lane = threadIdx.x & 63;
+    int c[4], mt[4], mt2[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int e = 4 * lane + i;
+        const int tot = e < E ? s_tot[e] : 0;
+        c[i] = tot;
+        mt[i] = (tot + mt_rows - 1) / mt_rows;
+        mt2[i] = (tot + 127) / 128;
+    }
+    // a list longer than 4x the mean: the slots go column-major (tile_of) so the long lists' tiles
+    // spread over the XCDs
+    int cmax = max(max(c[0], c[1]), max(c[2], c[3]));
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) cmax = max(cmax, __shfl_xor(cmax, d, 64));
+    const bool skewed = (long long)cmax * E > 4ll * P;
+    // exclusive scans across the wave of the lanes' sums (4 experts per lane, ascending)
+    int sc = ((c[0] + c[1]) + c[2]) + c[3], sm = ((mt[0] + mt[1]) + mt[2]) + mt[3];
+    int sm2 = ((mt2[0] + mt2[1]) + mt2[2]) + mt2[3];
+    int ic = sc, im = sm, im2 = sm2;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int uc = __shfl_up(ic, d, 64), um = __shfl_up(im, d, 64), um2 = __shfl_up(im2, d, 64);
+        if (lane >= d) {
+            ic += uc;
+            im += um;
+            im2 += um2;
+        }
+    }
+    int oc = ic - sc, om = im - sm, om2 = im2 - sm2;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int e = 4 * lane + i;
+        if (e < E) {
+            if (write) {
+                counts[e] = c[i];
+                offsets[e] = oc;
+                m_off[e] = om;
+                if (m_off2) m_off2[e] = om2;
+            }
+            s_tot[e] = oc;  // the expert's first list position
+        }
+        if (write && e == E - 1) {
+            offsets[E] = oc + c[i];
+            m_off[E] = om + mt[i];
+            if (m_off2) {
+                m_off2[E] = om2 + mt2[i];
+                // wide tiles cost kWideTileCost / kShortTileCost of a 64-row one, and a round of 256
+                // ends with its last tile
+                const int rw = ((om2 + mt2[i]) * wide_nt + 255) / 256, rs = ((om + mt[i]) * 2 * wide_nt + 255) / 256;
+                const bool shorter = tall == 1 || (wide_nt && rw > 1 && rs * kShortTileCost < rw * kWideTileCost);
+                choice[0] = shorter ? 0 : (1 | (skewed ? 2 : 0));  // 64-row tiles: expert-major
+                choice[1] = shorter ? om + mt[i] : om2 + mt2[i];    // the plan's row tiles
+            }
+        }
+        oc += c[i];
+        om += mt[i];
+        om2 += mt2[i];
+    }
+}
+
+// One 64-pair step of a wave: the rank of each lane's pair among the wave's earlier pairs of its expert, by
+// ballots over the bits of the expert id; row: the wave's running counts.
+__device__ __forceinline__ int rank_pairs(int *row, int e, bool valid, uint64_t below, int lane) {
+    uint64_t same = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        const bool bit = (e >> b) & 1;
+        const uint64_t ones = __ballot(bit);
+        same &= bit ? ones : ~ones;
+    }
+    const int before = __popcll(same & below);
+    const int cur = valid ? row[e] : 0;  // read by every lane before any update (in-order LDS)
+    if (valid && (same >> lane) == 1ull) row[e] = cur + before + 1;  // last lane of its expert
+    return cur + before;
+}
 
 // ---------------------------------------------------------------- dispatch (one block, 1024 threads)
 // routing [P] with pair p = t*K + k. Outputs: counts[E]; offsets[E+1] (exclusive prefix of counts);
 // perm[P]: pair ids grouped by expert, increasing within an expert; pos_of[P]: inverse of perm;
 // m_off[E+1]: exclusive prefix of ceil(counts / mt_rows) (the grouped GEMMs' row tiles per expert);
-// with m_off2 given, also m_off2[E+1] for 128-row tiles and *choice, the grouped GEMMs' plan: bit 0 the
+// with m_off2 given, also m_off2[E+1] for 128-row tiles and choice[2], the grouped GEMMs' plan (and its row
+// tiles): bit 0 the
 // tile height (1: 128 rows, 0: mt_rows; tall = 1 forces mt_rows, else 128), bit 1 the slot order of
 // the 128-row tiles (column-major when some list is longer than 4x the mean, else expert-major; see
 // tile_of). Measured
@@ -64,7 +155,7 @@ __global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t *__restric
                                                         int32_t *__restrict__ perm, int32_t *__restrict__ pos_of,
                                                         int32_t *__restrict__ m_off, int mt_rows,
                                                         int32_t *__restrict__ m_off2, int32_t *__restrict__ choice,
-                                                        int tall) {
+                                                        int tall, int wide_nt) {
     constexpr int NW = 16;
     __shared__ int s_w[NW][kDispatchMaxE];  // A: running counts per wave; B: each wave's base positions
     __shared__ int s_tot[kDispatchMaxE];    // B: each expert's total, then its first list position
@@ -77,20 +168,6 @@ __global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t *__restric
     for (int i = tid; i < NW * kDispatchMaxE; i += 1024) (&s_w[0][0])[i] = 0;
     __syncthreads();
     const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
-    // one 64-pair step: the rank of each pair among the wave's earlier pairs of its expert
-    auto rank_step = [&](int p, int e, bool valid) {
-        uint64_t same = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const bool bit = (e >> b) & 1;
-            const uint64_t ones = __ballot(bit);
-            same &= bit ? ones : ~ones;
-        }
-        const int before = __popcll(same & below);
-        const int cur = valid ? s_w[wv][e] : 0;  // read by every lane before any update (in-order LDS)
-        if (valid && (same >> lane) == 1ull) s_w[wv][e] = cur + before + 1;  // last lane of its expert
-        return cur + before;
-    };
     // the first kDispRegs steps keep expert and rank in registers (all their routing loads issued
     // together, nothing re-read in C); later steps, for more than 16 * 64 * kDispRegs pairs, keep the
     // rank in pos_of and read the routing again
@@ -99,12 +176,12 @@ __global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t *__restric
     for (int i = 0; i < kDispRegs; ++i) ereg[i] = base + 64 * i + lane < end ? min(max(rv[i], 0), E - 1) : -1;
 #pragma unroll
     for (int i = 0; i < kDispRegs; ++i)
-        if (base + 64 * i < end) rreg[i] = rank_step(base + 64 * i + lane, max(ereg[i], 0), ereg[i] >= 0);
+        if (base + 64 * i < end) rreg[i] = rank_pairs(s_w[wv], max(ereg[i], 0), ereg[i] >= 0, below, lane);
     for (int p0 = base + 64 * kDispRegs; p0 < end; p0 += 64) {  // wave-uniform loop
         const int p = p0 + lane;
         const bool valid = p < end;
         const int e = valid ? min(max(routing[p], 0), E - 1) : 0;
-        const int rk = rank_step(p, e, valid);
+        const int rk = rank_pairs(s_w[wv], e, valid, below, lane);
         if (valid) pos_of[p] = rk;
     }
     __syncthreads();
@@ -122,59 +199,8 @@ __global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t *__restric
         pre[j] = run;
     }
     __syncthreads();
-    if (wv == 0) {
-        int c[4], mt[4], mt2[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int e = 4 * lane + i;
-            const int tot = e < E ? s_tot[e] : 0;
-            c[i] = tot;
-            mt[i] = (tot + mt_rows - 1) / mt_rows;
-            mt2[i] = (tot + 127) / 128;
-        }
-        // a list longer than 4x the mean: the slots go column-major (tile_of) so the long lists' tiles
-        // spread over the XCDs
-        int cmax = max(max(c[0], c[1]), max(c[2], c[3]));
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) cmax = max(cmax, __shfl_xor(cmax, d, 64));
-        const bool skewed = (long long)cmax * E > 4ll * P;
-        // exclusive scans across the wave of the lanes' sums (4 experts per lane, ascending)
-        int sc = ((c[0] + c[1]) + c[2]) + c[3], sm = ((mt[0] + mt[1]) + mt[2]) + mt[3];
-        int sm2 = ((mt2[0] + mt2[1]) + mt2[2]) + mt2[3];
-        int ic = sc, im = sm, im2 = sm2;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int uc = __shfl_up(ic, d, 64), um = __shfl_up(im, d, 64), um2 = __shfl_up(im2, d, 64);
-            if (lane >= d) {
-                ic += uc;
-                im += um;
-                im2 += um2;
-            }
-        }
-        int oc = ic - sc, om = im - sm, om2 = im2 - sm2;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int e = 4 * lane + i;
-            if (e < E) {
-                counts[e] = c[i];
-                offsets[e] = oc;
-                m_off[e] = om;
-                if (m_off2) m_off2[e] = om2;
-                s_tot[e] = oc;  // the expert's first list position
-            }
-            if (e == E - 1) {
-                offsets[E] = oc + c[i];
-                m_off[E] = om + mt[i];
-                if (m_off2) {
-                    m_off2[E] = om2 + mt2[i];
-                    *choice = tall == 1 ? 0 : (1 | (skewed ? 2 : 0));  // 64-row tiles: expert-major
-                }
-            }
-            oc += c[i];
-            om += mt[i];
-            om2 += mt2[i];
-        }
-    }
+    if (wv == 0)
+        dispatch_scan(s_tot, P, E, true, counts, offsets, m_off, mt_rows, m_off2, choice, tall, wide_nt);
     __syncthreads();
     // B3: each wave's first position for each expert
 #pragma unroll
@@ -200,6 +226,79 @@ __global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t *__restric
             perm[pos] = p;
             pos_of[p] = pos;
         }
+    }
+}
+
+// ---------------------------------------------------------------- dispatch of many pairs (two launches)
+// The same outputs, bit for bit, by up to kDispBlocks blocks of S pairs each. Count: a block ranks its pairs
+// (waves of consecutive slices, as dispatch_kernel) and leaves each pair's rank among the block's pairs of
+// its expert in pos_of and the block's counts in bcnt[block][E]. Place: every block adds up the counts before
+// it, scans the totals (block 0 writes them) and places its pairs. One block walks 64 pairs per wave and step,
+// ~1.8 us each: 6144 pairs 12 us, 32768 pairs 60 us, against 12 us each in two launches.
+constexpr int kDispBlocks = 64, kDispMinPerBlock = 2048, kDispOneBlockPairs = 6144;
+__global__ __launch_bounds__(1024) void dispatch_count_kernel(const int32_t *__restrict__ routing, int P, int E, int S,
+                                                              int32_t *__restrict__ bcnt, int32_t *__restrict__ pos_of) {
+    constexpr int NW = 16;
+    __shared__ int s_w[NW][kDispatchMaxE];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int first = blockIdx.x * S, last = min(P, first + S);
+    const int W = S / NW, base = first + wv * W, end = min(last, base + W);  // S is a multiple of 64 NW
+    for (int i = tid; i < NW * kDispatchMaxE; i += 1024) (&s_w[0][0])[i] = 0;
+    __syncthreads();
+    const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
+    int next = routing[min(base + lane, P - 1)];  // one step ahead, unconditional
+    for (int p0 = base; p0 < end; p0 += 64) {     // wave-uniform
+        const int p = p0 + lane, cur = next;
+        next = routing[min(p + 64, P - 1)];
+        const bool valid = p < end;
+        const int rk = rank_pairs(s_w[wv], valid ? min(max(cur, 0), E - 1) : 0, valid, below, lane);
+        if (valid) pos_of[p] = rk;
+    }
+    __syncthreads();
+    for (int e = tid; e < E; e += 1024) {  // the waves' counts become their first ranks in the block
+        int run = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const int n = s_w[w][e];
+            s_w[w][e] = run;
+            run += n;
+        }
+        bcnt[blockIdx.x * E + e] = run;
+    }
+    __syncthreads();
+    for (int p0 = base; p0 < end; p0 += 64) {
+        const int p = p0 + lane;
+        if (p < end) pos_of[p] += s_w[wv][min(max(routing[p], 0), E - 1)];
+    }
+}
+
+__global__ __launch_bounds__(1024) void dispatch_place_kernel(const int32_t *__restrict__ routing, int P, int E, int S,
+                                                              const int32_t *__restrict__ bcnt,
+                                                              int32_t *__restrict__ counts, int32_t *__restrict__ offsets,
+                                                              int32_t *__restrict__ perm, int32_t *__restrict__ pos_of,
+                                                              int32_t *__restrict__ m_off, int mt_rows,
+                                                              int32_t *__restrict__ m_off2, int32_t *__restrict__ choice,
+                                                              int tall, int wide_nt) {
+    __shared__ int s_tot[kDispatchMaxE], s_base[kDispatchMaxE];
+    const int tid = threadIdx.x, nb = gridDim.x, blk = blockIdx.x;
+    if (tid < E) {
+        int tot = 0, before = 0;
+#pragma unroll 8
+        for (int b = 0; b < nb; ++b) {
+            const int n = bcnt[b * E + tid];
+            tot += n;
+            before += b < blk ? n : 0;
+        }
+        s_tot[tid] = tot;
+        s_base[tid] = before;
+    }
+    __syncthreads();
+    if (tid < 64) dispatch_scan(s_tot, P, E, blk == 0, counts, offsets, m_off, mt_rows, m_off2, choice, tall, wide_nt);
+    __syncthreads();
+    for (int p = blk * S + tid; p < min(P, (blk + 1) * S); p += 1024) {
+        const int e = min(max(routing[p], 0), E - 1), pos = s_tot[e] + s_base[e] + pos_of[p];
+        perm[pos] = p;
+        pos_of[p] = pos;
     }
 }
 
@@ -277,7 +376,7 @@ __device__ __forceinline__ void wait_stages(int ahead, int n) {
 // per wave.
 constexpr int kGWRows = 256, kGKC = 64;  // the 64-row tile; prefill_supported's shape rules
 constexpr int kSmallTileRowsPerExpert = 16;  // mean list rows per expert up to which tiles have 32 rows
-template <int ROWS, int WROWS>
+template <int ROWS, int WROWS, int WAVES>
 struct GTile {
     static constexpr int kWRows = WROWS;                   // weight rows per tile
     static constexpr int kKC = ROWS == 64 ? 64 : 128;      // k per stage
@@ -288,7 +387,7 @@ struct GTile {
     static constexpr int kWBytes = kWRows * kRowB;         // 32 KiB
     static constexpr int kABytes = ROWS * kRowB;
     static constexpr int kStageBytes = kWBytes + 2 * kABytes;
-    static constexpr int kWaves = ROWS == 32 ? 8 : 16;    // waves per block (each needs a W1/W3 pair)
+    static constexpr int kWaves = WAVES;                   // waves per block (each needs a W1/W3 pair)
     static constexpr int kRG = ROWS / 16;                  // row groups of 16 (one per wave)
     static constexpr int kCH = kWaves / kRG;               // weight-row splits (waves per row group)
     static constexpr int kNB = kWRows / 16 / kCH;          // weight blocks of 16 per wave
@@ -317,14 +416,14 @@ struct GTile {
 // The block's work on tile slot `bid` (the kernels below pass blockIdx.x); ring: the LDS ring of
 // STAGES * SBYTES bytes at LDS offset ring0.
 
-template <int MATS, int ROWS, int WROWS>
+template <int MATS, int ROWS, int WROWS, int WAVES>
 __device__ __forceinline__ void gemm_lds_tile(
     uint8_t *ring, uint32_t ring0, unsigned bid, const uint8_t *__restrict__ experts, uint64_t stride, uint64_t w_off,
     uint64_t w3_off, int N, int Kd, const uint16_t *__restrict__ a_hi, const uint16_t *__restrict__ a_lo, int gather,
     const int32_t *__restrict__ perm, int topk, const int32_t *__restrict__ counts, const int32_t *__restrict__ offsets,
-    const int32_t *__restrict__ m_off, int E, int colmajor, float *__restrict__ out_f32, uint16_t *__restrict__ out_hi,
+    const int32_t *__restrict__ m_off, int E, int M, int colmajor, float *__restrict__ out_f32, uint16_t *__restrict__ out_hi,
     uint16_t *__restrict__ out_lo) {
-    using TS = GTile<ROWS, WROWS>;
+    using TS = GTile<ROWS, WROWS, WAVES>;
     constexpr int NTILE = WROWS / MATS;  // output columns per tile
     constexpr int STAGES = TS::kStages, SBYTES = TS::kStageBytes, NB = TS::kNB, AI = TS::kAI, WI = TS::kWI;
     constexpr int ROWB = TS::kRowB, GRAN = TS::kGran, RPC = TS::kRowsPerCopy, WBYTES = TS::kWBytes;
@@ -333,13 +432,13 @@ __device__ __forceinline__ void gemm_lds_tile(
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), rg = w % TS::kRG,
               ch = w / TS::kRG;
     const int ntiles_n = N / NTILE;
-    const int total = m_off[E] * ntiles_n;
+    const int total = M * ntiles_n;
     const int range = (total + 7) >> 3;
     const int slot = (int)(bid >> 3);
     const int tau = (int)(bid & 7) * range + slot;
     if (slot >= range || tau >= total) return;
     int e, jt, il;
-    tile_of(tau, m_off, E, ntiles_n, colmajor, &e, &jt, &il);
+    tile_of(tau, m_off, E, M, ntiles_n, colmajor, &e, &jt, &il);
     const int row0 = offsets[e] + il * ROWS;
     const int rows = __builtin_amdgcn_readfirstlane(min(ROWS, counts[e] - il * ROWS));  // uniform: scalar branches below
     const int n0 = jt * NTILE;
@@ -463,16 +562,18 @@ __device__ __forceinline__ void gemm_lds_tile(
     }
 }
 
+constexpr int lds_waves(int rows) { return rows == 32 ? 8 : 16; }
 template <int MATS, int ROWS, int WROWS>
-__global__ __launch_bounds__((64 * GTile<ROWS, WROWS>::kWaves), 1) void grouped_gemm_kernel(
+__global__ __launch_bounds__(64 * lds_waves(ROWS), 1) void grouped_gemm_kernel(
     const uint8_t *__restrict__ experts, uint64_t stride, uint64_t w_off, uint64_t w3_off, int N, int Kd,
     const uint16_t *__restrict__ a_hi, const uint16_t *__restrict__ a_lo, int gather, const int32_t *__restrict__ perm,
     int topk, const int32_t *__restrict__ counts, const int32_t *__restrict__ offsets,
     const int32_t *__restrict__ m_off, int E, float *__restrict__ out_f32, uint16_t *__restrict__ out_hi,
     uint16_t *__restrict__ out_lo) {
-    __shared__ __align__(1024) uint8_t ring[GTile<ROWS, WROWS>::kStages * GTile<ROWS, WROWS>::kStageBytes];
-    gemm_lds_tile<MATS, ROWS, WROWS>(ring, (uint32_t)(uintptr_t)ring, blockIdx.x, experts, stride, w_off, w3_off, N,
-                                     Kd, a_hi, a_lo, gather, perm, topk, counts, offsets, m_off, E, 0, out_f32, out_hi,
+    using TS = GTile<ROWS, WROWS, lds_waves(ROWS)>;
+    __shared__ __align__(1024) uint8_t ring[TS::kStages * TS::kStageBytes];
+    gemm_lds_tile<MATS, ROWS, WROWS, lds_waves(ROWS)>(ring, (uint32_t)(uintptr_t)ring, blockIdx.x, experts, stride, w_off, w3_off, N,
+                                     Kd, a_hi, a_lo, gather, perm, topk, counts, offsets, m_off, E, m_off[E], 0, out_f32, out_hi,
                                      out_lo);
 }
 
@@ -533,7 +634,7 @@ __device__ __forceinline__ void gemm_wr_tile(
     uint8_t *smem, unsigned bid, const uint8_t *__restrict__ experts, uint64_t stride, uint64_t w_off, uint64_t w3_off,
     int N, int Kd, const uint16_t *__restrict__ a_hi, const uint16_t *__restrict__ a_lo, int gather,
     const int32_t *__restrict__ perm, int topk, const int32_t *__restrict__ counts, const int32_t *__restrict__ offsets,
-    const int32_t *__restrict__ m_off, int E, int colmajor, float *__restrict__ out_f32, uint16_t *__restrict__ out_hi,
+    const int32_t *__restrict__ m_off, int E, int M, int colmajor, float *__restrict__ out_f32, uint16_t *__restrict__ out_hi,
     uint16_t *__restrict__ out_lo, const uint8_t *__restrict__ tiled, uint64_t tiled_stride, uint64_t tiled_off) {
     constexpr int NT = 64 * kWrWaves;             // threads
     constexpr int NTILE = MATS == 2 ? 128 : 256;  // output columns per tile
@@ -546,13 +647,13 @@ __device__ __forceinline__ void gemm_wr_tile(
     uint8_t(*ring)[2 * ABYTES] = reinterpret_cast<uint8_t(*)[2 * ABYTES]>(smem);
     const int tid = threadIdx.x, lane = tid & 63, W = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int ntiles_n = N / NTILE;
-    const int total = m_off[E] * ntiles_n;
+    const int total = M * ntiles_n;
     const int range = (total + 7) >> 3;
     const int slot = (int)(bid >> 3);
     const int tau = (int)(bid & 7) * range + slot;
     if (slot >= range || tau >= total) return;
     int e, jt, il;
-    tile_of(tau, m_off, E, ntiles_n, colmajor, &e, &jt, &il);
+    tile_of(tau, m_off, E, M, ntiles_n, colmajor, &e, &jt, &il);
     const int row0 = offsets[e] + il * kWrRows;
     const int rows = __builtin_amdgcn_readfirstlane(min(kWrRows, counts[e] - il * kWrRows));
     const int n0 = jt * NTILE;
@@ -728,8 +829,8 @@ __device__ __forceinline__ void gemm_wr_tile(
 // tiles over m_off64; bit 1: column-major slot order, see tile_of), and every block runs that path on
 // its tile slot. Both paths take 16 waves; the LDS is the larger
 // ring (the 64-row tiles').
-constexpr int kSelLds = GTile<64, 256>::kStages * GTile<64, 256>::kStageBytes;
-static_assert(kSelLds >= 2 * 2 * kWrRows * 2 * kWrKC && GTile<64, 256>::kWaves == kWrWaves, "shared launch shape");
+constexpr int kSelLds = GTile<64, 256, 16>::kStages * GTile<64, 256, 16>::kStageBytes;
+static_assert(kSelLds >= 2 * 2 * kWrRows * 2 * kWrKC && lds_waves(64) == kWrWaves, "shared launch shape");
 template <int MATS, bool BLOB>
 __global__ __launch_bounds__(64 * kWrWaves, 1) void grouped_gemm_sel_kernel(
     const uint8_t *__restrict__ experts, uint64_t stride, uint64_t w_off, uint64_t w3_off, int N, int Kd,
@@ -742,11 +843,11 @@ __global__ __launch_bounds__(64 * kWrWaves, 1) void grouped_gemm_sel_kernel(
     const int plan = __builtin_amdgcn_readfirstlane(*choice), colmajor = plan >> 1;
     if (plan & 1)
         gemm_wr_tile<MATS, BLOB>(smem, blockIdx.x, experts, stride, w_off, w3_off, N, Kd, a_hi, a_lo, gather, perm, topk,
-                           counts, offsets, m_off128, E, colmajor, out_f32, out_hi, out_lo, tiled, tiled_stride,
+                           counts, offsets, m_off128, E, m_off128[E], colmajor, out_f32, out_hi, out_lo, tiled, tiled_stride,
                            tiled_off);
     else
-        gemm_lds_tile<MATS, 64, 256>(smem, (uint32_t)(uintptr_t)smem, blockIdx.x, experts, stride, w_off, w3_off, N,
-                                     Kd, a_hi, a_lo, gather, perm, topk, counts, offsets, m_off64, E, colmajor,
+        gemm_lds_tile<MATS, 64, 256, 16>(smem, (uint32_t)(uintptr_t)smem, blockIdx.x, experts, stride, w_off, w3_off, N,
+                                     Kd, a_hi, a_lo, gather, perm, topk, counts, offsets, m_off64, E, m_off64[E], colmajor,
                                      out_f32, out_hi, out_lo);
 }
 
@@ -765,36 +866,34 @@ constexpr bool gemm_wide_supported(int mats, int N, int Kd) {
     return N % (mats == 2 ? 256 : 512) == 0 && Kd % (2 * kWrKC) == 0;
 }
 
+constexpr int wide_lds(int mats) {  // the gate/up epilogue's exchange, or the two-stage activation ring
+    return mats == 2 ? kWdWaves * (kWrRows / 16 / 2) * kWdGroups * 64 * 16 : 2 * 2 * kWrRows * 2 * kWrKC;
+}
+// The block's work on wide tile slot `bid`; smem: wide_lds(MATS) bytes of LDS.
 template <int MATS, bool BLOB>
-__global__ __launch_bounds__(64 * kWdWaves, 1) void grouped_gemm_wide_kernel(
-    const uint8_t *__restrict__ experts, uint64_t stride, uint64_t w_off, uint64_t w3_off, int N, int Kd,
-    const uint16_t *__restrict__ a_hi, const uint16_t *__restrict__ a_lo, int gather, const int32_t *__restrict__ perm,
-    int topk, const int32_t *__restrict__ counts, const int32_t *__restrict__ offsets,
-    const int32_t *__restrict__ m_off, const int32_t *__restrict__ choice, int E, float *__restrict__ out_f32,
-    uint16_t *__restrict__ out_hi, uint16_t *__restrict__ out_lo, const uint8_t *__restrict__ tiled,
-    uint64_t tiled_stride, uint64_t tiled_off) {
+__device__ __forceinline__ void gemm_wide_tile(
+    uint8_t *smem, unsigned bid, const uint8_t *__restrict__ experts, uint64_t stride, uint64_t w_off, uint64_t w3_off,
+    int N, int Kd, const uint16_t *__restrict__ a_hi, const uint16_t *__restrict__ a_lo, int gather,
+    const int32_t *__restrict__ perm, int topk, const int32_t *__restrict__ counts, const int32_t *__restrict__ offsets,
+    const int32_t *__restrict__ m_off, int E, int M, int colmajor, float *__restrict__ out_f32, uint16_t *__restrict__ out_hi,
+    uint16_t *__restrict__ out_lo, const uint8_t *__restrict__ tiled, uint64_t tiled_stride, uint64_t tiled_off) {
     constexpr int NT = 64 * kWdWaves;              // threads
     constexpr int NTILE = MATS == 2 ? 256 : 512;   // output columns per tile
     constexpr int RG = kWrRows / 16;               // row groups of 16
     constexpr int ROWB = 2 * kWrKC;                // bytes of an activation row per k-step
     constexpr int ABYTES = kWrRows * ROWB;         // one plane of a k-step, 16 KiB
     constexpr int AU = 2 * ABYTES / 16 / NT;       // 16-byte activation units per thread per k-step (4)
-    constexpr int XBYTES = kWdWaves * (RG / 2) * kWdGroups * 64 * 16;  // gate/up epilogue exchange, 128 KiB
-    constexpr int LDSB = MATS == 2 ? XBYTES : 2 * 2 * ABYTES;
-    static_assert(AU * NT * 16 == 2 * ABYTES && LDSB >= 2 * 2 * ABYTES, "ring sizes");
-    __shared__ __align__(1024) uint8_t smem[LDSB];
+    static_assert(AU * NT * 16 == 2 * ABYTES && wide_lds(MATS) >= 2 * 2 * ABYTES, "ring sizes");
     uint8_t(*ring)[2 * ABYTES] = reinterpret_cast<uint8_t(*)[2 * ABYTES]>(smem);
     const int tid = threadIdx.x, lane = tid & 63, W = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int colmajor = (__builtin_amdgcn_readfirstlane(*choice) >> 1) & 1;
-    const unsigned bid = blockIdx.x;
     const int ntiles_n = N / NTILE;
-    const int total = m_off[E] * ntiles_n;
+    const int total = M * ntiles_n;
     const int range = (total + 7) >> 3;
     const int slot = (int)(bid >> 3);
     const int tau = (int)(bid & 7) * range + slot;
     if (slot >= range || tau >= total) return;
     int e, jt, il;
-    tile_of(tau, m_off, E, ntiles_n, colmajor, &e, &jt, &il);
+    tile_of(tau, m_off, E, M, ntiles_n, colmajor, &e, &jt, &il);
     const int row0 = offsets[e] + il * kWrRows;
     const int rows = __builtin_amdgcn_readfirstlane(min(kWrRows, counts[e] - il * kWrRows));
     const int n0 = jt * NTILE;
@@ -992,6 +1091,35 @@ __global__ __launch_bounds__(64 * kWdWaves, 1) void grouped_gemm_wide_kernel(
     }
 }
 
+// The wide tiles or 64-row tiles, as the dispatch chose from the histogram (*choice bit 0: wide tiles over
+// m_off128, else 64-row tiles over m_off64; bit 1: column-major slots of the wide tiles), eight waves either way.
+constexpr int kWsLds = GTile<64, 256, kWdWaves>::kStages * GTile<64, 256, kWdWaves>::kStageBytes;
+static_assert(kWsLds >= wide_lds(1) && kWsLds >= wide_lds(2), "shared launch shape");
+template <int MATS, bool BLOB>
+__global__ __launch_bounds__(64 * kWdWaves, 1) void grouped_gemm_wide_kernel(
+    const uint8_t *__restrict__ experts, uint64_t stride, uint64_t w_off, uint64_t w3_off, int N, int Kd,
+    const uint16_t *__restrict__ a_hi, const uint16_t *__restrict__ a_lo, int gather, const int32_t *__restrict__ perm,
+    int topk, const int32_t *__restrict__ counts, const int32_t *__restrict__ offsets,
+    const int32_t *__restrict__ m_off64, const int32_t *__restrict__ m_off128, const int32_t *__restrict__ choice, int E,
+    float *__restrict__ out_f32, uint16_t *__restrict__ out_hi, uint16_t *__restrict__ out_lo,
+    const uint8_t *__restrict__ tiled, uint64_t tiled_stride, uint64_t tiled_off) {
+    __shared__ __align__(1024) uint8_t smem[kWsLds];
+    // the grid covers the larger of the two plans: a block without a tile ends after one load (it holds a CU's
+    // LDS meanwhile)
+    const int2 ch = *reinterpret_cast<const int2 *>(choice);
+    const int plan = __builtin_amdgcn_readfirstlane(ch.x), M = __builtin_amdgcn_readfirstlane(ch.y);
+    const int slots = (M * (N / ((plan & 1 ? 512 : 256) / MATS)) + 7) >> 3;
+    if ((int)(blockIdx.x >> 3) >= slots) return;
+    if (plan & 1)
+        gemm_wide_tile<MATS, BLOB>(smem, blockIdx.x, experts, stride, w_off, w3_off, N, Kd, a_hi, a_lo, gather, perm, topk,
+                                   counts, offsets, m_off128, E, M, (plan >> 1) & 1, out_f32, out_hi, out_lo, tiled,
+                                   tiled_stride, tiled_off);
+    else
+        gemm_lds_tile<MATS, 64, 256, kWdWaves>(smem, (uint32_t)(uintptr_t)smem, blockIdx.x, experts, stride, w_off, w3_off,
+                                               N, Kd, a_hi, a_lo, gather, perm, topk, counts, offsets, m_off64, E, M, 0,
+                                               out_f32, out_hi, out_lo);
+}
+
 // moe[t][d] = sum_k w[t][k] * y[pos_of[t*K+k]][d] in selection order (rabbit2.c:540); x += moe.
 __global__ __launch_bounds__(256) void combine_rows_kernel(const float *__restrict__ y,
                                                           const int32_t *__restrict__ pos_of,
@@ -1082,7 +1210,7 @@ hipError_t launch_gemm(const Launch &L, const uint8_t *experts, uint64_t stride,
     const long long tiles = (long long)max_mtiles * (N / (WROWS / MATS));
     const long long blocks = (tiles + 7) / 8 * 8;
     if (blocks > 0x7FFFFFFFll) return hipErrorInvalidValue;
-    return launch(L, grouped_gemm_kernel<MATS, ROWS, WROWS>, dim3((unsigned)blocks), dim3(64 * GTile<ROWS, WROWS>::kWaves),
+    return launch(L, grouped_gemm_kernel<MATS, ROWS, WROWS>, dim3((unsigned)blocks), dim3(64 * lds_waves(ROWS)),
                   0, experts, stride, w_off, w3_off, N, Kd, a_hi, a_lo, gather, perm, topk, counts, offsets, m_off, E,
                   out_f32, out_hi, out_lo);
 }
@@ -1112,19 +1240,21 @@ hipError_t launch_gemm_sel(const Launch &L, const uint8_t *experts, uint64_t str
 template <int MATS>
 hipError_t launch_gemm_wide(const Launch &L, const uint8_t *experts, uint64_t stride, uint64_t w_off, uint64_t w3_off,
                             int N, int Kd, const uint16_t *a_hi, const uint16_t *a_lo, int gather, const int32_t *perm,
-                            int topk, const int32_t *counts, const int32_t *offsets, const int32_t *m_off128,
-                            const int32_t *choice, int E, int max_mtiles, float *out_f32, uint16_t *out_hi,
+                            int topk, const int32_t *counts, const int32_t *offsets, const int32_t *m_off64,
+                            const int32_t *m_off128, const int32_t *choice, int E, int max_mtiles, float *out_f32, uint16_t *out_hi,
                             uint16_t *out_lo, const uint8_t *tiled, uint64_t tiled_stride, uint64_t tiled_off) {
     if (!gemm_wide_supported(MATS, N, Kd)) return hipErrorInvalidValue;
-    const long long tiles = (long long)max_mtiles * (N / (MATS == 2 ? 256 : 512));  // >= the 128-row tiles
+    // the 64-row tiles, >= the wide ones. (Blocks that take every gridDim.x-th slot of a grid for the wide ones
+    // lose more than the idle blocks cost: 777 tokens, +2 on eight experts' logits, 187 against 162 us.)
+    const long long tiles = (long long)max_mtiles * (N / (MATS == 2 ? 128 : 256));
     const long long blocks = (tiles + 7) / 8 * 8;
     if (blocks > 0x7FFFFFFFll) return hipErrorInvalidValue;
     if (tiled)
         return launch(L, grouped_gemm_wide_kernel<MATS, false>, dim3((unsigned)blocks), dim3(64 * kWdWaves), 0, experts,
-                      stride, w_off, w3_off, N, Kd, a_hi, a_lo, gather, perm, topk, counts, offsets, m_off128, choice, E,
+                      stride, w_off, w3_off, N, Kd, a_hi, a_lo, gather, perm, topk, counts, offsets, m_off64, m_off128, choice, E,
                       out_f32, out_hi, out_lo, tiled, tiled_stride, tiled_off);
     return launch(L, grouped_gemm_wide_kernel<MATS, true>, dim3((unsigned)blocks), dim3(64 * kWdWaves), 0, experts,
-                  stride, w_off, w3_off, N, Kd, a_hi, a_lo, gather, perm, topk, counts, offsets, m_off128, choice, E,
+                  stride, w_off, w3_off, N, Kd, a_hi, a_lo, gather, perm, topk, counts, offsets, m_off64, m_off128, choice, E,
                   out_f32, out_hi, out_lo, tiled, tiled_stride, tiled_off);
 }
 
@@ -1156,7 +1286,7 @@ bool prefill_supported(int dtype, int T, int min_tokens, int E, int K, int D, in
 size_t prefill_workspace_bytes(int T, int E, int K, int D) {
     const size_t P = (size_t)T * K;
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-    return up(4 * (size_t)E) + 3 * up(4 * (size_t)(E + 1)) + up(4) + 2 * up(4 * P) + up(4 * P * (size_t)D) +
+    return up(4 * (size_t)E) + 3 * up(4 * (size_t)(E + 1)) + up(8) + 2 * up(4 * P) + up(4 * P * (size_t)D) +
            2 * up(2 * (size_t)T * D);
 }
 
@@ -1180,7 +1310,7 @@ PrefillWs carve_ws(void *ws, int T, int E, int K, int D) {
     r.offsets = reinterpret_cast<int32_t *>(carve(4 * (size_t)(E + 1)));
     r.m_off = reinterpret_cast<int32_t *>(carve(4 * (size_t)(E + 1)));
     r.m_off128 = reinterpret_cast<int32_t *>(carve(4 * (size_t)(E + 1)));
-    r.choice = reinterpret_cast<int32_t *>(carve(4));
+    r.choice = reinterpret_cast<int32_t *>(carve(8));
     r.perm = reinterpret_cast<int32_t *>(carve(4 * (size_t)P));
     r.pos_of = reinterpret_cast<int32_t *>(carve(4 * (size_t)P));
     r.y = reinterpret_cast<float *>(carve(4 * (size_t)P * D));
@@ -1204,10 +1334,22 @@ void prefill_x_planes(void *ws, int T, int E, int K, int D, uint16_t **x_hi, uin
 
 hipError_t launch_dispatch(const Launch &L, const int32_t *routing, int P, int E, int32_t *counts, int32_t *offsets,
                            int32_t *perm, int32_t *pos_of, int32_t *m_off, int mt_rows, int32_t *m_off2, int32_t *choice,
-                           int tall) {
+                           int tall, int wide_nt, int32_t *bcnt) {
     if (P < 1 || E < 1 || E > kDispatchMaxE) return hipErrorInvalidValue;
+    if (bcnt && P > kDispOneBlockPairs) {
+        int per = (P + kDispBlocks - 1) / kDispBlocks;
+        per = ((per > kDispMinPerBlock ? per : kDispMinPerBlock) + 1023) / 1024 * 1024;
+        const dim3 g((unsigned)((P + per - 1) / per)), b(1024);
+        Launch L1 = L, L2 = L;
+        L1.stop = nullptr;
+        L2.start = nullptr;
+        const hipError_t e = launch(L1, dispatch_count_kernel, g, b, 0, routing, P, E, per, bcnt, pos_of);
+        if (e != hipSuccess) return e;
+        return launch(L2, dispatch_place_kernel, g, b, 0, routing, P, E, per, (const int32_t *)bcnt, counts, offsets, perm,
+                      pos_of, m_off, mt_rows, m_off2, choice, tall, wide_nt);
+    }
     return launch(L, dispatch_kernel, dim3(1), dim3(1024), 0, routing, P, E, counts, offsets, perm, pos_of, m_off,
-                  mt_rows, m_off2, choice, tall);
+                  mt_rows, m_off2, choice, tall, wide_nt);
 }
 
 hipError_t launch_combine(const Launch &Lc, const float *y, const int32_t *pos_of, const float *weights, int T, int K,
@@ -1259,11 +1401,11 @@ hipError_t launch_prefill(const Launch &Ld, const Launch &Lg, const Launch &Lw, 
     const int mt_rows = small ? 32 : 64;
     const int tall = !tall_ok || small || tile_rows == 64 ? 1 : 2;
     const bool sel = !small && tall_ok;
-    e = launch_dispatch(Ldd, routing, P, E, counts, offsets, perm, pos_of, m_off, mt_rows, sel ? r.m_off128 : nullptr,
-                        r.choice, tall);
-    if (e != hipSuccess) return e;
-    // 128-row tiles (the dispatch picks them whenever tall == 2) in the wide kernel where the shape has it
+    // the wide kernel where the shape has it; it takes 64-row tiles where the dispatch finds them faster
     const bool wide = sel && tall == 2 && wide_ok && gemm_wide_supported(2, H, D) && gemm_wide_supported(1, D, H);
+    e = launch_dispatch(Ldd, routing, P, E, counts, offsets, perm, pos_of, m_off, mt_rows, sel ? r.m_off128 : nullptr,
+                        r.choice, tall, wide && tile_rows == 0 ? H / 256 : 0, reinterpret_cast<int32_t *>(y));
+    if (e != hipSuccess) return e;
     const uint8_t *ex = static_cast<const uint8_t *>(experts);
     const int max_mtiles = (P + mt_rows - 1) / mt_rows + E;  // >= sum over experts of ceil(count / mt_rows)
     const uint64_t w3 = (uint64_t)H * D * 2, w2 = 2 * (uint64_t)H * D * 2;
@@ -1277,7 +1419,7 @@ hipError_t launch_prefill(const Launch &Ld, const Launch &Lg, const Launch &Lw, 
         e = launch_gemm<2, 64, 256>(Lg, ex, stride, 0, w3, H, D, x_hi, x_lo, 1, perm, K, counts, offsets, m_off, E,
                                     max_mtiles, nullptr, h_hi, h_lo);
     else if (wide)
-        e = launch_gemm_wide<2>(Lg, ex, stride, 0, w3, H, D, x_hi, x_lo, 1, perm, K, counts, offsets, r.m_off128,
+        e = launch_gemm_wide<2>(Lg, ex, stride, 0, w3, H, D, x_hi, x_lo, 1, perm, K, counts, offsets, m_off, r.m_off128,
                                 r.choice, E, max_mtiles, nullptr, h_hi, h_lo, tl, tstride, 0);
     else
         e = launch_gemm_sel<2>(Lg, ex, stride, 0, w3, H, D, x_hi, x_lo, 1, perm, K, counts, offsets, m_off, r.m_off128,
@@ -1291,7 +1433,7 @@ hipError_t launch_prefill(const Launch &Ld, const Launch &Lg, const Launch &Lw, 
         e = launch_gemm<1, 64, 256>(Lw, ex, stride, w2, 0, D, H, h_hi, h_lo, 0, perm, K, counts, offsets, m_off, E,
                                     max_mtiles, y, nullptr, nullptr);
     else if (wide)
-        e = launch_gemm_wide<1>(Lw, ex, stride, w2, 0, D, H, h_hi, h_lo, 0, perm, K, counts, offsets, r.m_off128,
+        e = launch_gemm_wide<1>(Lw, ex, stride, w2, 0, D, H, h_hi, h_lo, 0, perm, K, counts, offsets, m_off, r.m_off128,
                                 r.choice, E, max_mtiles, y, nullptr, nullptr, tl, tstride, w2);
     else
         e = launch_gemm_sel<1>(Lw, ex, stride, w2, 0, D, H, h_hi, h_lo, 0, perm, K, counts, offsets, m_off, r.m_off128,

@@ -81,9 +81,9 @@ constexpr int kWrBufRecords = 0x7FFF0000, kBufConfig = 0x00020000;
 // contiguous share of the slots spans every expert's row tiles for a few column tiles and a few long
 // lists load all XCDs alike. Either way an expert's row tiles of one column tile (one weight tile) are
 // consecutive, on one XCD.
-__device__ __forceinline__ void tile_of(int tau, const int32_t *__restrict__ m_off, int E, int nt, int colmajor,
+// M: the row tiles of all experts (m_off[E]).
+__device__ __forceinline__ void tile_of(int tau, const int32_t *__restrict__ m_off, int E, int M, int nt, int colmajor,
                                         int *e_out, int *jt_out, int *il_out) {
-    const int M = m_off[E];
     const int jc = colmajor ? tau / M : 0, key = colmajor ? tau - jc * M : tau, scale = colmajor ? 1 : nt;
     int lo = 0, hi = E - 1;  // the last e with m_off[e] * scale <= key
     while (lo < hi) {
@@ -243,11 +243,12 @@ hipError_t launch_combine_rmsnorm(const Launch &L, const float *y, const int32_t
                                   uint16_t *lo);
 
 // The grouped path's dispatch (one block) and combine launches, which the grouped forms share. m_off2 and
-// choice may be NULL together (one tile height, expert-major slots).
+// choice may be NULL together (one tile height, expert-major slots). bcnt: 64 x E ints of scratch that are
+// free until the dispatch is done (the down GEMM's output buffer), for the form of many pairs.
 constexpr int kDispatchMaxE = 256;
 hipError_t launch_dispatch(const Launch &L, const int32_t *routing, int P, int E, int32_t *counts, int32_t *offsets,
                            int32_t *perm, int32_t *pos_of, int32_t *m_off, int mt_rows, int32_t *m_off2, int32_t *choice,
-                           int tall);
+                           int tall, int wide_nt = 0, int32_t *bcnt = nullptr);
 hipError_t launch_combine(const Launch &L, const float *y, const int32_t *pos_of, const float *weights, int T, int K,
                           int D, float *x_inout, float *moe_out);
 
