@@ -452,18 +452,21 @@ __global__ __launch_bounds__(256) void topk_split_kernel(const float *__restrict
 }
 
 // Prefill front end in one launch (AVX2 order, E <= 64, bf16): router logits, softmax + top-k, and the
-// bf16 hi/lo split of x for the grouped GEMMs. One block per kPTok tokens covers all router rows, so the
+// bf16 hi/lo split of x for the grouped GEMMs. One block per 2 TPW tokens covers all router rows, so the
 // top-k runs in the block. Wave (token tl, quarter q) holds the 64 router rows in its lanes and runs
 // chains 4q..4q+3 of each: eight waves per block, two per SIMD, since a SIMD issues two waves' VALU
 // operations in the time one wave issues one. Router columns stream through LDS in double-buffered
 // chunks of kPCols (coalesced global reads; each lane then reads its row's 8-byte slice per step). x is
-// the same for the whole wave: it is read with scalar loads, kPGroup steps at a time and one group
+// the same for the whole wave: it is read with scalar loads, G steps at a time and one group
 // ahead, and enters the multiplies as a scalar operand, so no lane-by-lane copy of it returns from
 // memory. What bounds it at 512 tokens is the staging: every block pulls the whole 256 KiB router from
 // L2, and a CU's outstanding misses at L2 latency give it ~26 GB/s (about 10 of the kernel's 16 us);
 // the VALU work (a widen, a rounded multiply and a rounded add per weight) runs under that.
-constexpr int kPTok = 2, kPCols = 512, kPGroup = 8, kPThreads = kPTok * 64 * 4;
-template <int DT>
+// TPW tokens per wave (2 TPW per block): two from kPManyTokens tokens on, where the blocks of one fill the chip
+// more than once: a block then stages the router for four tokens and widens each weight once for two
+// (dim 2048, 64 experts: 640 tokens 28 -> 19.6 us, 2048 tokens 52 -> 38, 4096 tokens 106 -> 77).
+constexpr int kPCols = 512, kPThreads = 2 * 64 * 4, kPManyTokens = 513;
+template <int DT, int TPW>
 __global__ __launch_bounds__(kPThreads) void router_prefill_kernel(const float *__restrict__ xb,
                                                                    const void *__restrict__ Wv,
                                                                    const float *__restrict__ bias, int T, int E, int D,
@@ -476,7 +479,8 @@ __global__ __launch_bounds__(kPThreads) void router_prefill_kernel(const float *
     constexpr int WP = CW * 2 + 16;           // row pitch in bytes
     constexpr int UPR = CW * 2 / 16;          // 16-byte units per row per chunk
     constexpr int WU = 64 * UPR / kPThreads;  // per thread per chunk
-    constexpr int G = kPGroup;
+    constexpr int kPTok = 2 * TPW;            // tokens per block
+    constexpr int G = TPW == 1 ? 8 : 4;       // steps per group: x takes 4 G TPW scalar registers per set
     constexpr int SU = 2;                     // split: 16-byte loads in flight per thread
     __shared__ __align__(16) unsigned char wt[2][64 * WP];
     __shared__ __align__(16) float s_part[kPTok][16][64];  // the 16 chains of each (token, row)
@@ -491,8 +495,10 @@ __global__ __launch_bounds__(kPThreads) void router_prefill_kernel(const float *
     const int ntok = min(kPTok, T - t0);
     const int body = (D / 16) * 16;
     const int nch = (body + CW - 1) / CW;
-    const bool live = tl < ntok;  // wave-uniform
-    const float *xrow = xb + (size_t)(t0 + (live ? tl : 0)) * D + 4 * q;  // wave-uniform: scalar loads
+    const bool live = tl * TPW < ntok;  // wave-uniform
+    const float *xrow[TPW];             // wave-uniform: scalar loads; tokens past the batch repeat the last
+#pragma unroll
+    for (int i = 0; i < TPW; ++i) xrow[i] = xb + (size_t)(t0 + min(tl * TPW + i, ntok - 1)) * D + 4 * q;
     const float bias_r = bias ? bias[min(r, E - 1)] : 0.0f;  // read now, used at the end
 
     u32x4 wv4[WU];
@@ -538,14 +544,20 @@ __global__ __launch_bounds__(kPThreads) void router_prefill_kernel(const float *
         }
     }
 
-    float acc[4];
+    float acc[TPW][4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] = 0.0f;
-    auto step = [&](const uint2 a, const float *xs) {
-        acc[0] = acc[0] + bf16_lo(a.x) * xs[0];
-        acc[1] = acc[1] + bf16_hi(a.x) * xs[1];
-        acc[2] = acc[2] + bf16_lo(a.y) * xs[2];
-        acc[3] = acc[3] + bf16_hi(a.y) * xs[3];
+    for (int i = 0; i < TPW; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
+    auto step = [&](const uint2 a, int o) {
+#pragma unroll
+        for (int i = 0; i < TPW; ++i) {
+            const float *xs = xrow[i] + o;
+            acc[i][0] = acc[i][0] + bf16_lo(a.x) * xs[0];
+            acc[i][1] = acc[i][1] + bf16_hi(a.x) * xs[1];
+            acc[i][2] = acc[i][2] + bf16_lo(a.y) * xs[2];
+            acc[i][3] = acc[i][3] + bf16_hi(a.y) * xs[3];
+        }
     };
     if (nch > 0) store(0);
     __syncthreads();
@@ -555,7 +567,6 @@ __global__ __launch_bounds__(kPThreads) void router_prefill_kernel(const float *
         const int c0 = c * CW, steps = min(CW, body - c0) / 16, full = steps / (2 * G) * (2 * G);
         if (live) {  // every lane (rows past E repeat row E - 1 and are not used): uniform control flow
             const unsigned char *wr = wt[c & 1] + r * WP + 8 * q;
-            const float *xc = xrow + c0;
             // groups of G steps in two register sets: while one set's group multiplies, the other set
             // takes the next group's router slices (LDS) and x (scalar loads at constant offsets from
             // one base, so few address registers). The fetch after the last group is clamped into the
@@ -565,64 +576,72 @@ __global__ __launch_bounds__(kPThreads) void router_prefill_kernel(const float *
             // asm), which places the wait before it; scheduling barriers keep each fetch ahead of the
             // other set's multiplies.
             uint2 wa[G], wb[G];
-            float xa[G * 4], xb4[G * 4];
-            auto fetch = [&](uint2 (&w)[G], float (&x)[G * 4], int g, float after) {
+            float xa[TPW][G * 4], xb4[TPW][G * 4];
+            auto fetch = [&](uint2 (&w)[G], float (&x)[TPW][G * 4], int g, float after) {
                 g = min(g, steps - G);
-                int xo = 16 * g;
+                int xo = c0 + 16 * g;
                 asm volatile("" : "+s"(xo) : "s"(after));
                 const unsigned char *wp = wr + 32 * g;
-                const float *xp = xc + xo;
 #pragma unroll
                 for (int i = 0; i < G; ++i) w[i] = *reinterpret_cast<const uint2 *>(wp + 32 * i);
 #pragma unroll
-                for (int k = 0; k < G * 4; ++k) x[k] = xp[16 * (k / 4) + k % 4];
+                for (int i = 0; i < TPW; ++i)
+#pragma unroll
+                    for (int k = 0; k < G * 4; ++k) x[i][k] = xrow[i][xo + 16 * (k / 4) + k % 4];
             };
             // all of a group's products first, then its adds in step order: dependent operations sit
             // far apart, so neither wave of a SIMD waits on a result
-            auto run = [&](const uint2 (&w)[G], const float (&x)[G * 4]) {
-                float pr[G][4];
+            auto run = [&](const uint2 (&w)[G], const float (&x)[TPW][G * 4]) {
+                float pr[TPW][G][4];
 #pragma unroll
                 for (int i = 0; i < G; ++i) {
-                    pr[i][0] = bf16_lo(w[i].x) * x[4 * i];
-                    pr[i][1] = bf16_hi(w[i].x) * x[4 * i + 1];
-                    pr[i][2] = bf16_lo(w[i].y) * x[4 * i + 2];
-                    pr[i][3] = bf16_hi(w[i].y) * x[4 * i + 3];
+                    const float f[4] = {bf16_lo(w[i].x), bf16_hi(w[i].x), bf16_lo(w[i].y), bf16_hi(w[i].y)};
+#pragma unroll
+                    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) pr[t][i][j] = f[j] * x[t][4 * i + j];
                 }
 #pragma unroll
                 for (int i = 0; i < G; ++i)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[j] = acc[j] + pr[i][j];
+                    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc[t][j] = acc[t][j] + pr[t][i][j];
             };
             if (full > 0) fetch(wa, xa, 0, 0.0f);
             for (int g = 0; g < full; g += 2 * G) {
-                fetch(wb, xb4, g + G, xa[0]);
+                fetch(wb, xb4, g + G, xa[0][0]);
                 __builtin_amdgcn_sched_barrier(0);
                 run(wa, xa);
                 __builtin_amdgcn_sched_barrier(0);
-                fetch(wa, xa, g + 2 * G, xb4[0]);
+                fetch(wa, xa, g + 2 * G, xb4[0][0]);
                 __builtin_amdgcn_sched_barrier(0);
                 run(wb, xb4);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            for (int m = full; m < steps; ++m) step(*reinterpret_cast<const uint2 *>(wr + 32 * m), xc + 16 * m);
+            for (int m = full; m < steps; ++m) step(*reinterpret_cast<const uint2 *>(wr + 32 * m), c0 + 16 * m);
         }
         if (more) store(c + 1);  // the other buffer: last read in chunk c-1, before the barrier below
         __syncthreads();
     }
     if (live) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) s_part[tl][4 * q + j][r] = acc[j];
+        for (int i = 0; i < TPW; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) s_part[tl * TPW + i][4 * q + j][r] = acc[i][j];
     }
     __syncthreads();
-    if (q == 0 && live && r < E) {
+    // the four waves of a token pair share its TPW tokens' sums: wave q takes token q
+    const int tk = tl * TPW + q;
+    if (q < TPW && tk < ntok && r < E) {
         float sum = 0.0f;  // the engine's lanes a[j] + b[j] (chains j and 8 + j), summed from j = 0
 #pragma unroll
-        for (int j = 0; j < 8; ++j) sum = sum + (s_part[tl][j][r] + s_part[tl][8 + j][r]);
+        for (int j = 0; j < 8; ++j) sum = sum + (s_part[tk][j][r] + s_part[tk][8 + j][r]);
         const uint16_t *wrow = Wg + (size_t)r * D;
-        const float *x = xb + (size_t)(t0 + tl) * D;
+        const float *x = xb + (size_t)(t0 + tk) * D;
         for (int i = body; i < D; ++i) sum = sum + widen<DT>(wrow[i]) * x[i];
         if (bias) sum = sum + bias_r;
-        s_log[tl][r] = sum;
+        s_log[tk][r] = sum;
     }
     __syncthreads();
     if (wv < ntok) {
@@ -1194,8 +1213,11 @@ hipError_t launch_router_prefill(const Launch &L, int dtype, const float *xb, co
                                  uint16_t *x_hi, uint16_t *x_lo) {
     if (T <= 0) return hipSuccess;
     if (dtype != RBT_DT_BF16) return hipErrorNotSupported;  // the grouped path is bf16 only
-    const dim3 g((unsigned)((T + kPTok - 1) / kPTok)), b(kPThreads);
-    return launch(L, router_prefill_kernel<RBT_DT_BF16>, g, b, 0, xb, W, bias, T, E, D, K, norm_topk, routing, weights,
+    const dim3 b(kPThreads);
+    if (T >= kPManyTokens)
+        return launch(L, router_prefill_kernel<RBT_DT_BF16, 2>, dim3((unsigned)((T + 3) / 4)), b, 0, xb, W, bias, T, E, D, K,
+                      norm_topk, routing, weights, x_hi, x_lo);
+    return launch(L, router_prefill_kernel<RBT_DT_BF16, 1>, dim3((unsigned)((T + 1) / 2)), b, 0, xb, W, bias, T, E, D, K, norm_topk, routing, weights,
                   x_hi, x_lo);
 }
 
