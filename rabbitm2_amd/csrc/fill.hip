@@ -72,4 +72,20 @@ hipError_t launch_fill_normal(const Launch &L, void *dst, int dtype, uint64_t n,
                   offset);
 }
 
+namespace {
+// 16-byte units from one side of the bus to the other; one unit per thread keeps every request in flight.
+__global__ __launch_bounds__(256) void host_copy_kernel(const u32x4 *__restrict__ src, u32x4 *__restrict__ dst, unsigned n) {
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+}  // namespace
+
+hipError_t launch_host_copy(const Launch &L, const void *src, void *dst, size_t bytes) {
+    const size_t n = (bytes + 15) / 16;
+    if (n == 0) return hipSuccess;
+    if (n > (1u << 30) || ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15u)) return hipErrorInvalidValue;
+    return launch(L, host_copy_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, static_cast<const u32x4 *>(src),
+                  static_cast<u32x4 *>(dst), (unsigned)n);
+}
+
 }  // namespace rbt

@@ -381,6 +381,9 @@ hipError_t launch_record_routing(const Launch &L, const StepState *st, const int
 // Dense matvec (one row per wave).
 hipError_t launch_matvec(const Launch &L, int dtype, const void *W, const float *x, float *out, int rows, int cols);
 
+// Copies whole 16-byte units (bytes rounded up) between device memory and mapped pinned host memory.
+hipError_t launch_host_copy(const Launch &L, const void *src, void *dst, size_t bytes);
+
 // Synthetic normal fill (SplitMix64 + Box-Muller), see rbt_hip_fill_normal.
 hipError_t launch_fill_normal(const Launch &L, void *dst, int dtype, uint64_t n, uint64_t seed, uint64_t stream,
                               uint64_t first, float scale, float offset);
