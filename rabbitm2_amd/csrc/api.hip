@@ -1072,8 +1072,8 @@ MoeForm prompt_form(const rbt_hip *h, const rbt_moe_layer *L, int T) {
 int prompt_reserve(rbt_hip *h, int n) {
     const rbt_config &c = h->cfg;
     const int qd = c.n_heads * c.head_dim, kvd = c.n_kv_heads * c.head_dim, T = std::min(n, kPromptBlock);
-    if (n < kPromptMinTokens || !dense_full_supported(c.dtype, T, c.dim, nullptr) ||
-        !dense_full_supported(c.dtype, T, qd, nullptr))
+    if (n < kPromptMinTokens || !dense_full_supported(c.dtype, T, c.dim, std::max(qd, kvd), nullptr) ||
+        !dense_full_supported(c.dtype, T, qd, c.dim, nullptr))
         return 0;
     PromptBuf &p = h->prompt;
     if (T <= p.tokens) return n;

@@ -19,6 +19,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kFullWaves = 4, kFullAhead = 3;  // waves per block; k-steps of weights in flight ahead
 constexpr int kFullWin = 128;                  // bytes of a weight row per k-step
+constexpr int kPastWeights = 0x70000000;       // an offset past any weight matrix (full_supported)
+constexpr int kBufStream = 2;                  // buffer loads of data read once: non-temporal
 
 struct FullArgs {
     const uint8_t *experts;
@@ -79,10 +81,9 @@ __device__ __forceinline__ uint32_t pack_hi16(uint32_t a, uint32_t b) { return (
 // each step's barrier, 22 + 27 against 17 + 17 us at dim 1000, hidden 330, 50 tokens; activations one step
 // ahead instead of four: 26 + 31 us; tiles of 128 rows and eight waves: 307 against 217 us on the 150-row
 // lists (spills).
-// GR: bytes per weight load, from the rows' alignment (16, 4 or 2); the last k-step of a row may be
-// partial: its loads are clamped into the row and the parts past the end set to zero.
-template <int DT, int MATS, int RG, int GR, bool DENSE = false>
-__global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const FullArgs a) {
+// GR: bytes per weight load, from the rows' alignment (16, 4 or 2); the last k-step of a row may be partial.
+template <int DT, int MATS, int RG, int GR, bool DENSE = false, int KS = 1>
+__global__ __launch_bounds__(64 * kFullWaves * KS, 2) void grouped_full_kernel(const FullArgs a) {
     constexpr int ESZ = DT == RBT_DT_BF16 ? 2 : 4, KW = kFullWin / ESZ;  // columns per k-step
     constexpr int ROWS = 16 * RG, NT = 64 * kFullWaves, NCOL = (MATS == 2 ? 16 : 32) * kFullWaves;
     constexpr int PARTS = DT == RBT_DT_BF16 ? 3 : 1;
@@ -92,8 +93,10 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
     constexpr int SLOTS = kFullAhead + 1;  // register sets of weights
     constexpr uint32_t kNegate = 0x80008000u;  // the sign bits of two bf16
     constexpr int AS = AU * UL > 2 ? 2 : SLOTS;  // register sets of activations (two where a set is large)
-    __shared__ __align__(1024) uint8_t ring[2 * STAGE];
-    const int tid = threadIdx.x, lane = tid & 63, W = __builtin_amdgcn_readfirstlane(tid >> 6);
+    __shared__ __align__(1024) uint8_t rings[KS * 2 * STAGE];
+    const int kg = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);  // this wave's part of the k-steps
+    const int tid = threadIdx.x - kg * NT, lane = tid & 63, W = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint8_t *ring = rings + kg * 2 * STAGE;
     int ntiles_n, total, e = 0, jt, il, row0, rows, n0, N = a.N, seg = 0;
     if constexpr (DENSE) {
         ntiles_n = 0;
@@ -128,21 +131,25 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
     }
     const int rowb = a.Kd * ESZ;  // bytes per weight row
     const int nch = (rowb + kFullWin - 1) / kFullWin;
-    const bool tail = rowb % kFullWin != 0;
     const int rot = (e + jt * max(1, nch / ntiles_n)) % nch;
-    auto cidx = [&](int c) { return c + rot < nch ? c + rot : c + rot - nch; };
+    const int nst = nch / KS, first = (rot + kg * nst) % nch;  // k-steps of this wave (nch a multiple of KS)
+    auto cidx = [&](int c) { return c + first < nch ? c + first : c + first - nch; };
 
-    // weight rows of this lane: column group g, half s2 (rows 8 s2 .. 8 s2 + 7 of the group's 16)
-    const uint8_t *wp[2][2];
+    // weight rows of this lane: column group g, half s2 (rows 8 s2 .. 8 s2 + 7 of the group's 16), as buffer loads
+    // from the tile's first row on: rows past the matrix, columns past the row and steps past the last get an
+    // offset past the buffer's end, which reads as zeros without a request
+    __amdgpu_buffer_rsrc_t rw[2];
+    uint32_t wrow[2][2];
     const int woff = 16 * blob_chunk(lane);
 #pragma unroll
-    for (int g = 0; g < 2; ++g)
+    for (int g = 0; g < 2; ++g) {
+        const uint8_t *base = DENSE ? a.seg_w[seg] : a.experts + (size_t)e * a.stride + (MATS == 2 && g ? a.w3_off : a.w_off);
+        rw[g] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(base) + (size_t)n0 * (size_t)rowb, 0,
+                                                  (int)((uint32_t)(N - n0) * (uint32_t)rowb), kBufConfig);
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-            const int n = n0 + (MATS == 2 ? 16 * W : 32 * W + 16 * g) + 8 * s2 + (lane & 7);
-            const uint8_t *base = DENSE ? a.seg_w[seg] : a.experts + (size_t)e * a.stride + (MATS == 2 && g ? a.w3_off : a.w_off);
-            wp[g][s2] = base + (size_t)min(n, N - 1) * (size_t)rowb;
-        }
+        for (int s2 = 0; s2 < 2; ++s2)
+            wrow[g][s2] = (uint32_t)((MATS == 2 ? 16 * W : 32 * W + 16 * g) + 8 * s2 + (lane & 7)) * (uint32_t)rowb;
+    }
     // activation units of this thread: row u / 8, granule u % 8 of the step's KW columns
     const size_t base_row = !DENSE && a.gather ? 0 : (size_t)row0;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
@@ -162,13 +169,13 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
     u32x4 aset[AS][AU][UL];
     u32x4 wv[SLOTS][2][2];
     auto load_a = [&](u32x4 (&av)[AU][UL], int c) {
-        const int cc = cidx(c);
+        const int k0 = c < nst ? KW * cidx(c) : a.Kd;  // steps past the last: zeros, without a request
 #pragma unroll
         for (int i = 0; i < AU; ++i)
 #pragma unroll
             for (int j = 0; j < UL; ++j) {
-                uint32_t off = aoff[i] + (uint32_t)(KW * cc + 4 * j) * 4u;
-                if (KW * cc + acol[i] + 4 * j >= a.Kd) off = (uint32_t)kWrBufRecords;  // past the row: zeros
+                uint32_t off = aoff[i] + (uint32_t)(k0 + 4 * j) * 4u;
+                if (k0 + acol[i] + 4 * j >= a.Kd) off = (uint32_t)kWrBufRecords;  // past the row: zeros
                 av[i][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0);
             }
     };
@@ -195,45 +202,27 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
         }
     };
     auto load_w = [&](u32x4 (&dst)[2][2], int c) {
-        const int off = cidx(c) * kFullWin + woff;
+        const int off = c < nst ? cidx(c) * kFullWin + woff : rowb;
 #pragma unroll
         for (int g = 0; g < 2; ++g)
 #pragma unroll
             for (int s2 = 0; s2 < 2; ++s2) {
-                const uint8_t *p = wp[g][s2];
+                auto at = [&](int o) { return (int)(o < rowb ? wrow[g][s2] + (uint32_t)o : (uint32_t)kPastWeights); };
                 if constexpr (GR == 16) {
-                    dst[g][s2] = ld_stream_u4(p + min(off, rowb - 16));
+                    dst[g][s2] = __builtin_amdgcn_raw_buffer_load_b128(rw[g], at(off), 0, kBufStream);
                 } else if constexpr (GR == 4) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        dst[g][s2][j] = __builtin_nontemporal_load(
-                            reinterpret_cast<const uint32_t *>(p + min(off + 4 * j, rowb - 4)));
+                        dst[g][s2][j] = __builtin_amdgcn_raw_buffer_load_b32(rw[g], at(off + 4 * j), 0, kBufStream);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        const uint16_t w0 = __builtin_nontemporal_load(
-                            reinterpret_cast<const uint16_t *>(p + min(off + 4 * j, rowb - 2)));
-                        const uint16_t w1 = __builtin_nontemporal_load(
-                            reinterpret_cast<const uint16_t *>(p + min(off + 4 * j + 2, rowb - 2)));
+                        const uint16_t w0 = __builtin_amdgcn_raw_buffer_load_b16(rw[g], at(off + 4 * j), 0, kBufStream);
+                        const uint16_t w1 = __builtin_amdgcn_raw_buffer_load_b16(rw[g], at(off + 4 * j + 2), 0, kBufStream);
                         dst[g][s2][j] = (uint32_t)w0 | ((uint32_t)w1 << 16);
                     }
                 }
             }
-    };
-    // the loads of a row's last, partial k-step past the row's end become zeros
-    auto mask_w = [&](u32x4 (&w)[2][2], int c) {
-        const int off = (nch - 1) * kFullWin + woff;
-        if (!tail || cidx(c) != nch - 1) return;
-#pragma unroll
-        for (int g = 0; g < 2; ++g)
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    uint32_t v = off + 4 * j < rowb ? w[g][s2][j] : 0u;
-                    if (GR == 2 && off + 4 * j + 2 >= rowb) v &= 0xFFFFu;
-                    w[g][s2][j] = v;
-                }
     };
 
     // bf16: mid holds the sums of the last steps, acc of everything before them; f32: the sums, and what
@@ -254,15 +243,15 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
     // k-step c, its operands in slot J = c % SLOTS. Loads return in issue order and a wait covers every older
     // load, so a step issues activations (AS steps ahead, stored to LDS one step ahead) before weights
     // (kFullAhead steps ahead): the LDS store waits for activations issued AS - 1 steps ago and not for
-    // the weights behind them. FULL: every load of the step exists (no branches, so the waits stay exact).
-    auto step = [&](auto jc, auto fullc, int c) {
+    // the weights behind them. Every load is issued in every step, past the last one too (no branches, so the
+    // waits stay exact, and one copy of the steps: the code of a second, branching set for the last steps
+    // was fetched anew by every block, GUARDNEW).
+    auto step = [&](auto jc, int c) {
         constexpr int J = decltype(jc)::value;
-        constexpr bool FULL = decltype(fullc)::value;
-        if (FULL || c + 1 < nch) store_a(aset[(J + 1) % AS], (c + 1) & 1, J & 1 ? 0u : kNegate);  // the buffer that step c - 1 read
-        if (FULL || c + AS < nch) load_a(aset[J % AS], c + AS);
-        if (FULL || c + kFullAhead < nch) load_w(wv[(J + kFullAhead) % SLOTS], c + kFullAhead);
+        store_a(aset[(J + 1) % AS], (c + 1) & 1, J & 1 ? 0u : kNegate);  // the buffer that step c - 1 read
+        load_a(aset[J % AS], c + AS);
+        load_w(wv[(J + kFullAhead) % SLOTS], c + kFullAhead);
         const uint8_t *st = ring + (c & 1) * STAGE;
-        mask_w(wv[J], c);
         blob_operands(wv[J][0][0], wv[J][0][1]);
         blob_operands(wv[J][1][0], wv[J][1][1]);
 #pragma unroll
@@ -320,27 +309,40 @@ __global__ __launch_bounds__(64 * kFullWaves, 2) void grouped_full_kernel(const 
     // prologue, in the steady state's order
 #pragma unroll
     for (int p = 0; p < SLOTS; ++p) {
-        if (p < AS && p < nch) load_a(aset[p % AS], p);
-        if (p < kFullAhead && p < nch) load_w(wv[p], p);
+        if (p < AS) load_a(aset[p % AS], p);
+        if (p < kFullAhead) load_w(wv[p], p);
     }
     store_a(aset[0], 0, 0u);
     __syncthreads();
-    int c = 0;
-    for (; c + 2 * SLOTS <= nch; c += SLOTS) {
-        step(I0{}, std::true_type{}, c);
-        step(I1{}, std::true_type{}, c + 1);
-        step(I2{}, std::true_type{}, c + 2);
-        step(I3{}, std::true_type{}, c + 3);
+    for (int c = 0;; c += SLOTS) {
+        step(I0{}, c);
+        if (c + 1 >= nst) break;
+        step(I1{}, c + 1);
+        if (c + 2 >= nst) break;
+        step(I2{}, c + 2);
+        if (c + 3 >= nst) break;
+        step(I3{}, c + 3);
         if (DT == RBT_DT_BF16 && (c & SLOTS)) flush();
-    }
-    for (; c < nch; c += SLOTS) {
-        step(I0{}, std::false_type{}, c);
-        if (c + 1 < nch) step(I1{}, std::false_type{}, c + 1);
-        if (c + 2 < nch) step(I2{}, std::false_type{}, c + 2);
-        if (c + 3 < nch) step(I3{}, std::false_type{}, c + 3);
+        if (c + SLOTS >= nst) break;
     }
     flush();
 
+    if constexpr (KS > 1) {  // the parts' sums meet in the first part's waves, through the (idle) rings
+        static_assert(KS == 2 && 2 * STAGE * KS >= kFullWaves * RG * 2 * 64 * 16, "two parts, exchange in the rings");
+        f32x4 *xch = reinterpret_cast<f32x4 *>(rings);  // [wave][q][g][lane]
+        if (kg == 1) {
+#pragma unroll
+            for (int q = 0; q < RG; ++q)
+#pragma unroll
+                for (int g = 0; g < 2; ++g) xch[((W * RG + q) * 2 + g) * 64 + lane] = acc[q][g];
+        }
+        __syncthreads();
+        if (kg == 1) return;
+#pragma unroll
+        for (int q = 0; q < RG; ++q)
+#pragma unroll
+            for (int g = 0; g < 2; ++g) acc[q][g] += xch[((W * RG + q) * 2 + g) * 64 + lane];
+    }
     // acc[q][g] lane holds column (lane % 16) of group g for list rows 16 q + 4 (lane / 16) + i
 #pragma unroll
     for (int q = 0; q < RG; ++q) {
@@ -371,7 +373,7 @@ int load_granule(uint64_t base, uint64_t stride, int Kd, int esz) {
     return bits % 16 == 0 ? 16 : bits % 4 == 0 ? 4 : bits % 2 == 0 && esz == 2 ? 2 : 0;
 }
 
-template <int MATS, bool DENSE = false>
+template <int MATS, bool DENSE = false, int KS = 1>
 hipError_t launch_full(const Launch &L, const FullArgs &a, int dtype, int rg, int max_mtiles) {
     constexpr int NCOL = (MATS == 2 ? 16 : 32) * kFullWaves;
     int ntiles_n = (a.N + NCOL - 1) / NCOL;
@@ -387,12 +389,12 @@ hipError_t launch_full(const Launch &L, const FullArgs &a, int dtype, int rg, in
     const long long tiles = (long long)max_mtiles * ntiles_n, blocks = (tiles + 7) / 8 * 8;
     const int gr = load_granule(base, a.stride, a.Kd, dtype == RBT_DT_BF16 ? 2 : 4);
     if (blocks > 0x7FFFFFFFll || gr == 0) return hipErrorInvalidValue;
-    const dim3 g((unsigned)blocks), b(64 * kFullWaves);
+    const dim3 g((unsigned)blocks), b(64 * kFullWaves * KS);
 #define FULL_CASE(DT, RG, GR) \
-    if (dtype == DT && rg == RG && gr == GR) return launch(L, grouped_full_kernel<DT, MATS, RG, GR, DENSE>, g, b, 0, a);
-#define FULL_TILES(DT, GR)  \
-    FULL_CASE(DT, 2, GR) \
-    FULL_CASE(DT, 4, GR)
+    if (dtype == DT && rg == RG && gr == GR) return launch(L, grouped_full_kernel<DT, MATS, RG, GR, DENSE, KS>, g, b, 0, a);
+#define FULL_TILES(DT, GR) \
+    FULL_CASE(DT, 2, GR)   \
+    if constexpr (KS == 1) { FULL_CASE(DT, 4, GR) }
     FULL_TILES(RBT_DT_BF16, 16)
     FULL_TILES(RBT_DT_BF16, 4)
     FULL_TILES(RBT_DT_BF16, 2)
@@ -418,9 +420,9 @@ bool full_supported(int dtype, int T, int E, int K, int D, int H, const void *ex
     return T >= 1 && T <= 65535 && E <= kDispatchMaxE && (long long)T * K <= (1 << 24) && D % 4 == 0 &&
            (reinterpret_cast<uintptr_t>(xb) & 15u) == 0 && load_granule(base, stride, D, esz) != 0 &&
            load_granule(base, stride, H, esz) != 0 &&
-           // 32-bit buffer offsets: the gathered rows of xb, a tile's rows of h, and bytes of a weight row
+           // 32-bit buffer offsets: the gathered rows of xb, a tile's rows of h, and a weight matrix
            (uint64_t)T * D * 4 < (uint64_t)kWrBufRecords && 128ull * full_h_stride(H) * 4 < (uint64_t)kWrBufRecords &&
-           (uint64_t)D * esz < (1u << 30) && (uint64_t)H * esz < (1u << 30);
+           (uint64_t)D * H * esz < (uint64_t)kPastWeights / 2;
 }
 
 // The grouped form reads each selected expert once, the per-pair GEMVs once per pair; it has two more
@@ -443,10 +445,11 @@ size_t full_workspace_bytes(int T, int E, int K, int D) {
     return up(4 * (size_t)E) + 3 * up(4 * (size_t)(E + 1)) + up(8) + 2 * up(4 * P) + up(4 * P * (size_t)D);
 }
 
-bool dense_full_supported(int dtype, int T, int Kd, const float *x) {
+bool dense_full_supported(int dtype, int T, int Kd, int rows, const float *x) {
     // row stride and alignment of x as the buffer loads need them; the model's tensors are 64-byte aligned
     return T >= 1 && T <= 65535 && Kd % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0 &&
-           load_granule(0, 0, Kd, dtype == RBT_DT_BF16 ? 2 : 4) != 0 && 128ull * Kd * 4 < (uint64_t)kWrBufRecords;
+           load_granule(0, 0, Kd, dtype == RBT_DT_BF16 ? 2 : 4) != 0 && 128ull * Kd * 4 < (uint64_t)kWrBufRecords &&
+           (uint64_t)rows * Kd * (dtype == RBT_DT_BF16 ? 2 : 4) < (uint64_t)kPastWeights / 2;
 }
 
 hipError_t launch_dense_full(const Launch &L, int dtype, const float *x, int T, int Kd, const void *const W[3],
@@ -464,7 +467,11 @@ hipError_t launch_dense_full(const Launch &L, int dtype, const float *x, int T, 
         a.seg_rows[s] = rows[s];
         tiles64 += (rows[s] + 32 * kFullWaves - 1) / (32 * kFullWaves) * ((T + 63) / 64);
     }
-    const int rg = tiles64 >= kDenseTallTiles ? 4 : 2;
+    // Few tiles leave CUs idle, and a CU moves ~27 GB/s whatever its tile: short tiles then, with the k-steps in
+    // two parts (dim 2048, us: wo of 400 rows 34 -> 29, of 24 rows 34 -> 29; q/k/v of 400 rows in 64-row tiles
+    // 68 against 80)
+    const int rg = tiles64 >= kDenseTallTiles ? 4 : 2, nch = (Kd * (dtype == RBT_DT_BF16 ? 2 : 4) + kFullWin - 1) / kFullWin;
+    if (rg == 2 && nch % 2 == 0) return launch_full<1, true, 2>(L, a, dtype, 2, (T + 31) / 32);
     return launch_full<1, true>(L, a, dtype, rg, (T + 16 * rg - 1) / (16 * rg));
 }
 

@@ -267,7 +267,8 @@ hipError_t launch_grouped_full(const Launch &Ld, const Launch &Lg, const Launch 
 
 // Rows of T tokens through up to three dense matrices on the same kernel (full f32 activation precision):
 // out_s [T][rows_s] = x W_s^T, or with resid != NULL resid [T][rows_0] += (one matrix).
-bool dense_full_supported(int dtype, int T, int Kd, const float *x);
+// rows: of the largest matrix.
+bool dense_full_supported(int dtype, int T, int Kd, int rows, const float *x);
 hipError_t launch_dense_full(const Launch &L, int dtype, const float *x, int T, int Kd, const void *const W[3],
                              float *const out[3], const int rows[3], float *resid);
 
