@@ -8,7 +8,8 @@
 // the .rbt2 blob layout w1[H][D] | w3[H][D] | w2[D][H] (rabbit2.c:173, rbt2.py:152-156).
 //
 // gateup: one wave per JW consecutive hidden units j of one (token, slot) pair; per lane 2*JW*NC
-//   16-byte weight loads + NC x loads, then 2*JW wave sums; h[p][j] = silu(g)*u in f32.
+//   16-byte weight loads + NC x loads, then 2*JW wave sums; h[p][j] = silu(g)*u in f32. Where several of a
+//   call's tokens share experts (gateup_multi_kernel) the waves of an expert's first pair do all its pairs.
 // down:   one block per (token, 4*RW output rows); the token's K hidden vectors are staged once in
 //   LDS; per wave, KC slots x RW rows x NH 16-byte weight loads in flight, then the K dot products
 //   are combined in selection order exactly like the engine's loop.
@@ -238,6 +239,95 @@ __global__ __launch_bounds__(256) void gateup_fast_kernel(const uint8_t *__restr
     }
 }
 
+// Gate/up of a few tokens (gateup_reads_once()): the grid of gateup_fast_kernel, but an expert that several
+// pairs selected is read once, by the waves of its first pair (the others' end): a wave keeps its JW hidden
+// units' rows of W1 and W3 in registers and runs every such pair's token through them, the next token's x on
+// its way meanwhile. Each output has the products and sums of the per-pair kernel, so the bits are the same.
+// Bound: HBM reads of the distinct experts (~6.3 TB/s at 8 tokens). Measured, us, one read per pair / this
+// (dim 2048, 64 experts, top-8, hidden 1024): bf16 5 tokens 48.7 / 43.7, 8 tokens 77 / 62, 11 tokens
+// 106 / 81; f32 4 tokens 80.6 / 68, 8 tokens 159 / 104.
+template <int DT, int NC, int JW>
+__global__ __launch_bounds__(256) void gateup_multi_kernel(const uint8_t *__restrict__ experts, uint64_t stride,
+                                                           const int32_t *__restrict__ routing,
+                                                           const float *__restrict__ xb, int P, int K, int H,
+                                                           float *__restrict__ hbuf) {
+    constexpr int kEsz = Elem<DT>::kEsz, kPer = Elem<DT>::kPer;
+    constexpr int D = NC * kWave * kPer;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int per = H / JW;  // items per pair
+    const long long item = (long long)blockIdx.x * (blockDim.x / kWave) + (threadIdx.x / kWave);
+    const int p = __builtin_amdgcn_readfirstlane((int)(item / per));
+    if (p >= P) return;
+    const int j0 = (int)(item - (long long)p * per) * JW;
+    // the pairs of this pair's expert: bits p' of two masks; the first one's waves do the work
+    const int r0 = routing[min(lane, P - 1)], r1 = routing[min(lane + 64, P - 1)];
+    const int e = __builtin_amdgcn_readlane(p < 64 ? r0 : r1, p & 63);
+    uint64_t m0 = __ballot(lane < P && r0 == e), m1 = __ballot(lane + 64 < P && r1 == e);
+    if ((m0 ? __builtin_ctzll(m0) : 64 + __builtin_ctzll(m1)) != p) return;  // wave-uniform
+
+    const uint8_t *w1 = experts + (size_t)e * stride + (size_t)j0 * D * kEsz;
+    const uint8_t *w3 = w1 + (size_t)H * D * kEsz;
+    u32x4 a[JW][NC], b[JW][NC];
+#pragma unroll
+    for (int jj = 0; jj < JW; ++jj)
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const size_t off = ((size_t)jj * D + (size_t)(lane + kWave * i) * kPer) * kEsz;
+            a[jj][i] = ld_stream_u4(w1 + off);
+            b[jj][i] = ld_stream_u4(w3 + off);
+        }
+    f32x4 x0[NC], x1[NC], y0[NC], y1[NC];
+    auto load_x = [&](f32x4 (&u)[NC], f32x4 (&v)[NC], int q) {
+        const float *x = xb + (size_t)(q / K) * D;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const float *xp = x + (lane + kWave * i) * kPer;
+            u[i] = *reinterpret_cast<const f32x4 *>(xp);
+            if constexpr (DT == RBT_DT_BF16) v[i] = *reinterpret_cast<const f32x4 *>(xp + 4);
+        }
+    };
+    auto pop = [&]() {  // the next pair, or the last one again
+        if (m0) {
+            const int q = __builtin_ctzll(m0);
+            m0 &= m0 - 1;
+            return q;
+        }
+        const int q = 64 + __builtin_ctzll(m1);
+        m1 &= m1 - 1;
+        return q;
+    };
+    int q = pop();
+    load_x(x0, x1, q);
+    __builtin_amdgcn_sched_barrier(0);
+    while (true) {
+        const bool more = (m0 | m1) != 0;
+        const int qn = more ? pop() : q;
+        if (more) load_x(y0, y1, qn);  // wave-uniform
+        float g[JW], u[JW];
+#pragma unroll
+        for (int jj = 0; jj < JW; ++jj) {
+            g[jj] = 0.0f;
+            u[jj] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                g[jj] += dot16r<DT>(a[jj][i], x0[i], x1[i]);
+                u[jj] += dot16r<DT>(b[jj][i], x0[i], x1[i]);
+            }
+        }
+#pragma unroll
+        for (int jj = 0; jj < JW; ++jj) {
+            const float gs = wave_sum(g[jj]), us = wave_sum(u[jj]);
+            if (lane == jj) hbuf[(size_t)q * H + j0 + jj] = (gs / (1.0f + expf(-gs))) * us;
+        }
+        if (!more) break;
+        for (int i = 0; i < NC; ++i) {
+            x0[i] = y0[i];
+            x1[i] = y1[i];
+        }
+        q = qn;
+    }
+}
+
 // grid (ceil(D / (BT/64*RW)), T), block BT, dynamic LDS K*H*4 bytes; requires H == NH * 64 * kPer.
 // HS: 16-byte units of h staged per thread (K*H/4 <= BT*HS). PD: slots of weight rows in flight when
 // the block waits for h (0: every slot of the first chunk).
@@ -363,6 +453,11 @@ __global__ __launch_bounds__(BT) void down_fast_kernel(const uint8_t *__restrict
     }
 }
 
+// Wave-steps of a row up to which gateup_multi_kernel keeps two waves per SIMD: with the next token's x it
+// holds 208 registers at 4 bf16 steps and 400 at 8 (8 tokens of dim 4096: no gain; 4 tokens 42 -> 52 us).
+template <int DT>
+constexpr int kMultiMaxNC = DT == RBT_DT_BF16 ? 4 : 8;
+
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 template <int DT, int NC>
@@ -374,6 +469,10 @@ hipError_t gateup_nc(const Launch &L, const uint8_t *E, uint64_t stride, int32_t
     if (logits)
         return launch(L, gateup_fast_kernel<DT, NC, JW, true>, g, b, 0, E, stride, routing, xb, K, H, items, hbuf,
                       logits, nE, norm_topk, weights);
+    if constexpr (NC <= kMultiMaxNC<DT>)
+        if (gateup_reads_once(DT, T, nE, K, NC * kWave * Elem<DT>::kPer, H))
+            return launch(L, gateup_multi_kernel<DT, NC, JW>, g, b, 0, E, stride, (const int32_t *)routing, xb, T * K,
+                          K, H, hbuf);
     return launch(L, gateup_fast_kernel<DT, NC, JW, false>, g, b, 0, E, stride, routing, xb, K, H, items, hbuf,
                   logits, nE, norm_topk, weights);
 }
@@ -423,6 +522,18 @@ hipError_t decode_dt(const Launch &Lg, const Launch &Ld, const uint8_t *E, uint6
 }
 
 }  // namespace
+
+// The pairs of an expert are two 64-bit masks, hence 128 pairs. Finding them delays the first weight load by
+// 2-5 us, so the reads expected to be saved (pairs less the experts expected to be selected, W1 and W3) have
+// to be worth it, 60 MB at ~7 TB/s. One read per pair / one per expert, us, top-8 of 64, dim 2048 but the
+// last: bf16 3 tokens (24 MB) 29 / 32, 4 (46 MB) 38.7 / 38.5, 5 (67 MB) 48.7 / 43.7; 6 of 256 experts
+// (29 MB) 60 / 62, 11 of 256 (107 MB) 108 / 104; 5 of dim 1024, hidden 512 (17 MB) 12.5 / 13.8.
+bool gateup_reads_once(int dtype, int T, int E, int K, int D, int H) {
+    const int esz = dtype == RBT_DT_BF16 ? 2 : 4;
+    const int max_nc = dtype == RBT_DT_BF16 ? kMultiMaxNC<RBT_DT_BF16> : kMultiMaxNC<RBT_DT_F32>;
+    const double p = (double)T * K, sel = E * (1.0 - pow(1.0 - (double)K / E, (double)T));
+    return p <= kMultiPairs && (long long)D * esz <= 1024ll * max_nc && (p - sel) * 2.0 * H * D * esz >= 60e6;
+}
 
 bool experts_decode_supported(int dtype, int T, int K, int D, int H, const void *experts, uint64_t stride,
                               const float *xb, const float *hbuf) {

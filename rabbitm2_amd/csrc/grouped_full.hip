@@ -428,15 +428,16 @@ bool full_supported(int dtype, int T, int E, int K, int D, int H, const void *ex
 // The grouped form reads each selected expert once, the per-pair GEMVs once per pair; it has two more
 // launches and longer kernels (~25 us at the smallest sizes). So it pays from a number of saved bytes on:
 // pairs minus experts expected to be selected, times an expert's bytes. Measured, GEMVs / grouped, us:
-//   f32, dim 2048, 64 experts, top-8, hidden 1024: 6 tokens (350 MB saved) 194 / 202, 8 (550 MB) 255 / 209,
-//     11 345 / 267, 200 5763 / 476
+//   f32, dim 2048, 64 experts, top-8, hidden 1024: 8 tokens (550 MB saved) 191 / 205, 11 (970 MB) 245 / 265,
+//     200 5763 / 426
 //   bf16, dim 1600, 40 experts, top-6, hidden 800: 2 tokens (12 MB) 46 / 60, 8 (150 MB) 110 / 79, 1000
 //     11045 / 364
 //   bf16, dim 1000, 20 experts, top-3, hidden 330: 11 tokens (32 MB) 40 / 57, 50 (260 MB) 98 / 61
-// The shapes of the specialised GEMVs (experts_decode.hip) stream twice as fast and need more.
+// The shapes of the specialised GEMVs (experts_decode.hip) stream twice as fast and need more, and
+// more again where their gate/up reads an expert once too and only W2 is read per pair.
 bool full_pays(bool fast_gemv, int dtype, int T, int E, int K, int D, int H) {
     const double p = (double)T * K, sel = E * (1.0 - pow(1.0 - (double)K / E, (double)T));
-    return (p - sel) * 3.0 * H * D * (dtype == RBT_DT_BF16 ? 2 : 4) >= (fast_gemv ? 450e6 : 100e6);
+    return (p - sel) * 3.0 * H * D * (dtype == RBT_DT_BF16 ? 2 : 4) >= (!fast_gemv ? 100e6 : gateup_reads_once(dtype, T, E, K, D, H) ? 1000e6 : 450e6);
 }
 
 size_t full_workspace_bytes(int T, int E, int K, int D) {

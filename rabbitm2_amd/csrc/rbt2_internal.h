@@ -201,6 +201,9 @@ hipError_t launch_down_combine(const Launch &L, int dtype, const void *experts, 
 // down kernels.
 bool experts_decode_supported(int dtype, int T, int K, int D, int H, const void *experts, uint64_t stride,
                               const float *xb, const float *hbuf);
+// Whether its gate/up reads the weights of an expert once for all pairs that selected it.
+constexpr int kMultiPairs = 128;
+bool gateup_reads_once(int dtype, int T, int E, int K, int D, int H);
 hipError_t launch_experts_decode(const Launch &Lg, const Launch &Ld, int dtype, const void *experts, uint64_t stride,
                                  int32_t *routing, float *weights, const float *xb, float *hbuf, int T, int K, int D,
                                  int H, float *x_inout, float *moe_out, const float *logits, int E, int norm_topk);
