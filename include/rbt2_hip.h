@@ -88,9 +88,9 @@ int rbt_hip_set_router_order(rbt_hip *h, int order);
  *                         caller made one with rbt_hip_prefill_layout (none exists otherwise: by
  *                         default every kernel reads the .rbt2 blobs); 0: the blobs only.
  *   "prefill_tile_rows"   0 (default): the grouped GEMMs take tiles of 32 rows of an expert's list
- *                         while the experts average at most 16 rows, else 128 rows where the shape
- *                         has them (64 otherwise), in an order the device picks from the call's
- *                         tokens-per-expert histogram; 32 / 64 / 128: that tile height always (128
+ *                         while the experts average at most 16 rows, else 128 or 64 rows (64 only,
+ *                         where the shape has no 128-row tiles) in a height and an order the device
+ *                         picks from the call's tokens-per-expert histogram; 32 / 64 / 128: that tile height always (128
  *                         where the shape has it). Outputs agree within the parity tolerance (the
  *                         reduction runs in other chunks).
  *   "prefill_wide"        1 (default): 128-row tiles span 512 weight rows (gate/up: 256 W1 + 256 W3
@@ -202,8 +202,9 @@ int rbt_hip_forward(rbt_hip *h, int token, int pos, float *logits, int32_t *rout
  * writes the next step's token, and each step is one HIP graph replay (steps after an eos are run and
  * discarded). The prompt's positions before its last are run in blocks of up to 512 (from 4 positions on,
  * where the dims are multiples of 4), each weight read once per block, at the per-token steps' precision;
- * the buffers for them are allocated by the first such prompt and freed with the decode state. ms_out (may be NULL) receives [prompt ms, generation ms] from HIP events: the prompt up to
- * the first generated token, then the steps after it (from option "generate_timed_from" on). */
+ * the buffers for them are allocated by the first such prompt and freed with the decode state. ms_out (may
+ * be NULL) receives [prompt ms, generation ms] from HIP events: the prompt up to the first generated token,
+ * then the steps after it (from option "generate_timed_from" on). */
 int rbt_hip_generate(rbt_hip *h, const int32_t *prompt, int n_prompt, int n_gen, int32_t eos, int32_t *out,
                      int *n_out, double *ms_out);
 

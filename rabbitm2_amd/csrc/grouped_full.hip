@@ -74,11 +74,11 @@ __device__ __forceinline__ uint32_t pack_hi16(uint32_t a, uint32_t b) { return (
 // errors along. The tile order and the rotation of the k-steps by weight tile are
 // prefill.hip's (the row tiles of a weight tile run together on one XCD and stay in step).
 // Bound: short lists by the weight stream (dim 2048, 64 experts, top-8, hidden 1024, f32: 12 tokens, about
-// 51 experts, 161 + 86 us, 5.2 TB/s; 200 tokens, two row groups per tile, 309 + 160 us against 3936 + 1939
+// 51 experts, 166 + 86 us, 5.2 TB/s; 200 tokens, two row groups per tile, 297 + 153 us against 3936 + 1939
 // us of per-pair GEMVs, of which the compensated sums take 58 + 26); long ones by the wave's own chain of
-// LDS reads and products (bf16, dim 1600, 40 experts of 150 rows, hidden 800: 210 + 120 us, 440 TFLOP/s
+// LDS reads and products (bf16, dim 1600, 40 experts of 150 rows, hidden 800: 207 + 116 us, 440 TFLOP/s
 // issued). Four waves per block, two blocks per CU: with eight-wave blocks (one per CU) every wave waits at
-// each step's barrier, 22 + 27 against 17 + 17 us at dim 1000, hidden 330, 50 tokens; activations one step
+// each step's barrier, 22 + 27 against 18 + 17 us at dim 1000, hidden 330, 50 tokens; activations one step
 // ahead instead of four: 26 + 31 us; tiles of 128 rows and eight waves: 307 against 217 us on the 150-row
 // lists (spills).
 // GR: bytes per weight load, from the rows' alignment (16, 4 or 2); the last k-step of a row may be partial.
@@ -405,7 +405,7 @@ hipError_t launch_full(const Launch &L, const FullArgs &a, int dtype, int rg, in
     return hipErrorInvalidValue;
 }
 
-// Mean list rows up to which tiles have 32 rows: half the LDS and 162 instead of 196 registers, and a list
+// Mean list rows up to which tiles have 32 rows: half the LDS and 162 instead of 212 registers, and a list
 // that passes 32 rows re-reads its weights from L2 (f32 200 tokens, 25 rows on average: 250 us either way;
 // with +2 on eight experts' logits 304 against 384 us).
 constexpr int kFullShortLists = 40;

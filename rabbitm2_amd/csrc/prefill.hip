@@ -6,9 +6,10 @@
 // moe += w_k * tmp in selection order, x += moe. Expert blob layout w1[H][D] | w3[H][D] | w2[D][H]
 // (rabbit2.c:173, rabbit2/tools/rbt2.py:152-156), bf16 elements.
 //
-// 1. dispatch_kernel: per-expert lists of the (token, slot) pairs, stable in pair order (counts,
-//    row offsets, perm, inverse perm) and the per-expert count of row tiles (64 rows, or 32 when the
-//    experts average at most 16 rows).
+// 1. dispatch_kernel (dispatch_count_kernel and dispatch_place_kernel for many pairs): per-expert lists of
+//    the (token, slot) pairs, stable in pair order (counts, row offsets, perm, inverse perm), the per-expert
+//    count of row tiles (64 or 128 rows, or 32 when the experts average at most 16 rows) and the choice
+//    between the two heights.
 // 2. grouped_gemm_kernel<2>: for each expert's rows, h = silu(W1 a) * (W3 a), written as bf16 hi/lo
 //    planes; grouped_gemm_kernel<1>: y = W2 h (f32 rows). Both on v_mfma_f32_16x16x32_bf16.
 //    The f32 activations are split into bf16 hi + lo parts and both parts are multiplied (two MFMAs
@@ -16,9 +17,9 @@
 //    instead of 8. A full 64-row tile then does 64 rows x 2 parts x 2 flop = 256 flop per weight
 //    element, 128 flop per weight byte: below the bf16 MFMA/HBM ridge (2.5 PFLOP/s / 8 TB/s =
 //    312), so the kernels stay bound by HBM.
-//    Tiles: 128 rows x 512 weight rows per block of 8 waves (grouped_gemm_wide_kernel, where the
-//    shape has them), 128 or 64 rows x 256 weight rows per block of 16 waves, or 32 x 128 per 8 waves
-//    for decode-sized batches; the 64- and 32-row tiles run the reduction in chunks of 64 (128)
+//    Tiles: 128 rows x 512 or 64 rows x 256 weight rows per block of 8 waves, the dispatch's choice
+//    (grouped_gemm_wide_kernel, where the shape has them), 128 or 64 rows x 256 weight rows per block of
+//    16 waves, or 32 x 128 per 8 waves for decode-sized batches; the 64- and 32-row tiles run the reduction in chunks of 64 (128)
 //    through a three- or four-stage LDS ring filled by direct HBM -> LDS copies, the 128-row tiles
 //    keep their weight operands in registers. 128-row tiles cover the whole list of an expert with
 //    up to 128 rows, so its weight tile is streamed by one block once.
@@ -136,14 +137,13 @@ __device__ __forceinline__ int rank_pairs(int *row, int e, bool valid, uint64_t 
 // perm[P]: pair ids grouped by expert, increasing within an expert; pos_of[P]: inverse of perm;
 // m_off[E+1]: exclusive prefix of ceil(counts / mt_rows) (the grouped GEMMs' row tiles per expert);
 // with m_off2 given, also m_off2[E+1] for 128-row tiles and choice[2], the grouped GEMMs' plan (and its row
-// tiles): bit 0 the
-// tile height (1: 128 rows, 0: mt_rows; tall = 1 forces mt_rows, else 128), bit 1 the slot order of
-// the 128-row tiles (column-major when some list is longer than 4x the mean, else expert-major; see
-// tile_of). Measured
-// on the OLMoE layer at 512 tokens: 128-row tiles beat 64-row ones with uniform routing (209 against
-// 262 us per call) and, in column-major order, with +2 on 8 experts' logits (247 against 255 us) and
-// +4 on 4 (223 against 231 us); expert-major order keeps the uniform case's activation rows in one
-// XCD's L2 per expert (209 against 214 us).
+// tiles): bit 0 the tile height (1: 128 rows, 0: mt_rows; tall = 1 forces mt_rows; else 128, unless wide_nt > 0
+// and the rounds of tiles are cheaper with 64 rows, see kWideTileCost), bit 1 the slot order of the 128-row
+// tiles (column-major when some list is longer than 4x the mean, else expert-major; see tile_of). Without wide
+// tiles, at 512 tokens of the OLMoE layer, 128-row tiles beat 64-row ones with uniform routing (209 against
+// 262 us per call) and, in column-major order, with +2 on 8 experts' logits (247 against 255 us) and +4 on 4
+// (223 against 231 us); expert-major order keeps the uniform case's activation rows in one XCD's L2 per
+// expert (209 against 214 us).
 // Wave w owns the pair slice [w*S, (w+1)*S). A: each wave ranks its pairs, 64 at a time, against
 // equal experts (ballots over the expert-id bits) and keeps per-expert running counts in its own LDS
 // row; a pair's rank inside its wave's slice stays in a register (pos_of holds it past the first
