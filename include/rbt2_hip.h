@@ -91,8 +91,10 @@ int rbt_hip_set_router_order(rbt_hip *h, int order);
  *                         while the experts average at most 16 rows, else 128 or 64 rows (64 only,
  *                         where the shape has no 128-row tiles) in a height and an order the device
  *                         picks from the call's tokens-per-expert histogram; 32 / 64 / 128: that tile height always (128
- *                         where the shape has it). Outputs agree within the parity tolerance (the
- *                         reduction runs in other chunks).
+ *                         where the shape has it). Outputs agree within the parity tolerance (32-row
+ *                         tiles reduce in other chunks); where the device picks the height (H a multiple
+ *                         of 256, D of 512), 64 and 128 rows give the same bits, so a token's output does
+ *                         not depend on how the call's other tokens are routed.
  *   "prefill_wide"        1 (default): 128-row tiles span 512 weight rows (gate/up: 256 W1 + 256 W3
  *                         rows; H a multiple of 256, D of 512), so each activation row fetched
  *                         serves twice the weight bytes; 0: 256 weight rows. Outputs agree within

@@ -375,6 +375,10 @@ __device__ __forceinline__ void wait_stages(int ahead, int n) {
 // for a second block. Copies: 1 KiB each (8 rows of 128 B or 4 of 256 B), 4 weight + 2 activation
 // per wave.
 constexpr int kGWRows = 256, kGKC = 64;  // the 64-row tile; prefill_supported's shape rules
+// the shapes of the wide 128-row tiles (512 weight rows, the k-chunks in pairs; grouped_gemm_wide_kernel)
+constexpr bool gemm_wide_supported(int mats, int N, int Kd) {
+    return N % (mats == 2 ? 256 : 512) == 0 && Kd % (2 * kGKC) == 0;
+}
 constexpr int kSmallTileRowsPerExpert = 16;  // mean list rows per expert up to which tiles have 32 rows
 template <int ROWS, int WROWS, int WAVES>
 struct GTile {
@@ -478,8 +482,12 @@ __device__ __forceinline__ void gemm_lds_tile(
     // same column window of its rows at the same time, so the whole chip's requests fall on the few
     // DRAM channels that window maps to. The rotation is a function of the weight tile (expert,
     // column tile), so the m-tiles that share a tile read it in the same order and stay in step (their
-    // second reads hit L2); the per-output summation order is still fixed for a given input.
-    const int rot = (e * ntiles_n + jt) % nch;
+    // second reads hit L2). Where the shape has wide tiles, a 64-row tile takes the rotation of the wide tile
+    // that holds its columns (same chunks, same products, hi before lo): an output's bits then do not depend on
+    // which of the two heights the dispatch picks from the other tokens' routing.
+    const int nw = ntiles_n / 2;
+    const int rot = ROWS == 64 && gemm_wide_supported(MATS, N, Kd) ? (e + (jt >> 1) * max(1, nch / nw)) % nch
+                                                                   : (e * ntiles_n + jt) % nch;
     auto issue = [&](int c) {
         const uint32_t sb = ring0 + (uint32_t)((c % STAGES) * SBYTES);
         const int cc = c + rot < nch ? c + rot : c + rot - nch;
@@ -862,9 +870,6 @@ __global__ __launch_bounds__(64 * kWrWaves, 1) void grouped_gemm_sel_kernel(
 // operands and products per output element as gemm_wr_tile (k-chunks of 64, each as two 32-wide
 // halves, hi then lo); the chunks are rotated per wide tile, so sums agree within rounding.
 constexpr int kWdWaves = 8, kWdGroups = 4;
-constexpr bool gemm_wide_supported(int mats, int N, int Kd) {
-    return N % (mats == 2 ? 256 : 512) == 0 && Kd % (2 * kWrKC) == 0;
-}
 
 constexpr int wide_lds(int mats) {  // the gate/up epilogue's exchange, or the two-stage activation ring
     return mats == 2 ? kWdWaves * (kWrRows / 16 / 2) * kWdGroups * 64 * 16 : 2 * 2 * kWrRows * 2 * kWrKC;

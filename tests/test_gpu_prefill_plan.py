@@ -1,8 +1,8 @@
 """The grouped path's plan from the tokens-per-expert histogram (rabbitm2_amd/csrc/prefill.hip): wide 128-row tiles
 or 64-row tiles, by the number of rounds that either takes, and the dispatch of many pairs in two launches.
 
-Whatever the plan, the outputs are those of the tile height it picked, bit for bit (the option that forces a
-height runs the same sums), and the histogram is the routing's. The plan's rule is restated here. Sizes: one
+Whatever the plan, the outputs are those of either tile height, bit for bit (both run the same sums), and the
+histogram is the routing's. The plan's rule is restated here. Sizes: one
 round of wide tiles, both sides of the rule, and 6144 / 6152 pairs around the one-block dispatch.
 """
 import numpy as np
@@ -50,6 +50,24 @@ def test_plan_matches_forced_height(dev, layers, T, skew):
     print(f"T {T} skew {skew}: {rows}-row tiles, longest list {counts.max()}", flush=True)
     assert np.array_equal(got["routing"], want["routing"])
     assert got["moe"].tobytes() == want["moe"].tobytes()
+
+
+@pytest.mark.parametrize("D,E,K,H,T", [(2048, 64, 8, 1024, 777), (512, 16, 4, 256, 200), (1024, 8, 2, 768, 500)])
+def test_rows_do_not_depend_on_the_height(dev, D, E, K, H, T):
+    """Both heights run the same chunks in the same order, so the height that the other tokens' routing leads to
+    does not show in a token's output."""
+    layer = SynthLayer(dev, D, E, K, H, po.DT_BF16, 1, seed=65, w_scale=1.0, fan_in=True)
+    dev.set_router_order(po.ORDER_AVX2)
+    xb = layer.make_x(T, seed=66, bf16=False)
+    got = {}
+    try:
+        for rows in (0, 64, 128):
+            dev.set_option("prefill_tile_rows", rows)
+            got[rows] = layer.run_gpu(xb)["moe"].tobytes()
+    finally:
+        dev.set_option("prefill_tile_rows", 0)
+        layer.close()
+    assert got[64] == got[128] and got[0] == got[128]
 
 
 @pytest.mark.parametrize("E,K,T", [(8, 2, 3073), (256, 6, 1025), (61, 7, 20000), (5, 1, 6145)])
