@@ -804,10 +804,9 @@ def prefill_workloads(dev, routers, experts, stride, xb, moe, bias_dev, reps, al
                 kern[kname] = {"avg_us": round(1000.0 * tot / n, 2)}
         dev.profile(0)
         counts = dev.expert_counts(E)
-        # the GEMMs' row tiles, by the device's rule: 32 rows while the experts average at most 16, else
-        # 128 rows (512 weight rows wide at this shape), their slots column-major where some list is
-        # longer than 4x the mean
-        tile_rows = 32 if P <= 16 * E else 128
+        # the GEMMs' row tiles as the device chose them (128-row tiles are 512 weight rows wide at this shape),
+        # 128-row tiles' slots column-major where some list is longer than 4x the mean
+        tile_rows = dev.tile_rows()
         tile_weight_rows = 512 if tile_rows == 128 and H % 256 == 0 and D % 512 == 0 else 256
         tiles = int(sum((c + tile_rows - 1) // tile_rows for c in counts))
         slot_order = "column-major" if tile_rows == 128 and int(counts.max()) * E > 4 * P else "expert-major"

@@ -174,6 +174,9 @@ int rbt_hip_moe_dev_noalloc(rbt_hip *h, const rbt_moe_layer *L, const float *xb_
 /* Tokens-per-expert histogram of the last rbt_hip_moe_dev call that used the grouped (prefill)
  * path, [n_experts] int32, device pointer owned by the handle; NULL if none. */
 const int32_t *rbt_hip_expert_counts_dev(rbt_hip *h);
+/* List rows per GEMM tile of that call (32, 64 or 128; where the device picks the height, its choice):
+ * *rows, 0 if there was none. Waits for the handle stream. */
+int rbt_hip_tile_rows(rbt_hip *h, int *rows);
 
 /* ---- the dense seam (replaces matvec(), rabbit2.c:357, for weights of the uploaded model) ----
  * out[r] = dot(W[r,:], x), W at byte offset w_offset of the uploaded image, [rows][cols] in the

@@ -146,7 +146,7 @@ struct rbt_hip {
     int prefill_tile_rows = 0;  // option "prefill_tile_rows": rows per grouped-GEMM tile, 0 = by batch
     bool prefill_wide = true;   // option "prefill_wide": 128-row tiles 512 weight rows wide
     int gen_timed_from = 1;     // option "generate_timed_from": first generated step of ms_out[1]
-    const int32_t *expert_counts = nullptr;  // histogram of the last grouped-path call
+    GroupedCall grouped;  // of the last grouped-path call
     // staging for the host-pointer entry points: device buffer and its pinned host twin
     void *stage = nullptr;
     uint64_t stage_bytes = 0;
@@ -381,7 +381,7 @@ int ws_reserve(rbt_hip *h, int T, int E, int K, int H) {
               nH = H > w.H ? H : w.H;
     HIP_OK(h, hipStreamSynchronize(h->stream));
     ws_release(w);
-    h->expert_counts = nullptr;
+    h->grouped = GroupedCall{};
     HIP_OK(h, hipMalloc(&w.probs, sizeof(float) * (size_t)nT * nE));
     HIP_OK(h, hipMalloc(&w.routing, sizeof(int32_t) * (size_t)nT * nK));
     HIP_OK(h, hipMalloc(&w.weights, sizeof(float) * (size_t)nT * nK));
@@ -401,7 +401,7 @@ int pre_reserve(rbt_hip *h, size_t bytes) {
     (void)hipFree(w.pre);
     w.pre = nullptr;
     w.pre_bytes = 0;
-    h->expert_counts = nullptr;
+    h->grouped = GroupedCall{};
     HIP_OK(h, hipMalloc(&w.pre, bytes));
     w.pre_bytes = bytes;
     return 1;
@@ -668,7 +668,7 @@ int moe_grouped_norm(rbt_hip *h, const rbt_moe_layer *L, const float *nw, float 
                                  w.probs, xb));
     HIP_OK(h, launch_topk_split(lc(h, kProfTopk), w.probs, T, L->n_experts, L->top_k, L->norm_topk, xb, L->dim, routing,
                                 w.weights, x_hi, x_lo));
-    int32_t *counts = nullptr;
+    GroupedCall call;
     // the combine's event pair is taken only by the launch that runs it (launch_prefill's combine, or
     // the fused combine + RMSNorm below), so a deferred-profile pair is never left unrecorded
     Launch no_combine;
@@ -676,9 +676,9 @@ int moe_grouped_norm(rbt_hip *h, const rbt_moe_layer *L, const float *nw, float 
     HIP_OK(h, launch_prefill(lc(h, kProfDispatch), lc(h, kProfGateup), lc(h, kProfDown),
                              next_nw ? no_combine : lc(h, kProfCombine), L->experts, L->expert_stride, xb, T,
                              L->n_experts, L->top_k, L->dim, L->expert_hidden, routing, w.weights, w.hbuf, w.pre, x,
-                             nullptr, &counts, true, next_nw == nullptr, h->prefill_tile_rows, tiled_for(h, L),
+                             nullptr, &call, true, next_nw == nullptr, h->prefill_tile_rows, tiled_for(h, L),
                              h->prefill_wide));
-    h->expert_counts = counts;
+    h->grouped = call;
     if (next_nw) {  // the combine, fused with the RMSNorm the next step starts with (xb and its planes)
         const float *y = nullptr;
         const int32_t *pos_of = nullptr;
@@ -1010,12 +1010,12 @@ int moe_block(rbt_hip *h, const rbt_moe_layer *L, const float *xb_dev, int T, fl
                                     L->router_bias, T, L->n_experts, L->dim, L->top_k, L->norm_topk, w.probs,
                                     routing, weights));
         }
-        int32_t *counts = nullptr;
+        GroupedCall call;
         HIP_OK(h, launch_prefill(lc(h, kProfDispatch), lc(h, kProfGateup), lc(h, kProfDown), lc(h, kProfCombine),
                                  L->experts, L->expert_stride, xb_dev, T, L->n_experts, L->top_k, L->dim,
-                                 L->expert_hidden, routing, weights, w.hbuf, w.pre, x_dev, moe_dev, &counts,
+                                 L->expert_hidden, routing, weights, w.hbuf, w.pre, x_dev, moe_dev, &call,
                                  fused || split, true, h->prefill_tile_rows, tiled_for(h, L), h->prefill_wide));
-        h->expert_counts = counts;
+        h->grouped = call;
         return done();
     }
     // the fused front end keeps a router row per lane: from 48 experts on it beats the two launches (dim 2048,
@@ -1029,11 +1029,11 @@ int moe_block(rbt_hip *h, const rbt_moe_layer *L, const float *xb_dev, int T, fl
                                 L->router_bias, T, L->n_experts, L->dim, L->top_k, L->norm_topk, w.probs, routing,
                                 weights));
     if (form == kMoeGroupedFull) {
-        int32_t *counts = nullptr;
+        GroupedCall call;
         HIP_OK(h, launch_grouped_full(lc(h, kProfDispatch), lc(h, kProfGateup), lc(h, kProfDown), lc(h, kProfCombine),
                                       L->dtype, L->experts, L->expert_stride, xb_dev, T, L->n_experts, L->top_k, L->dim,
-                                      L->expert_hidden, routing, weights, w.hbuf, w.pre, x_dev, moe_dev, &counts));
-        h->expert_counts = counts;
+                                      L->expert_hidden, routing, weights, w.hbuf, w.pre, x_dev, moe_dev, &call));
+        h->grouped = call;
         return done();
     }
     if (decode_kernels) {
@@ -1123,7 +1123,7 @@ int prompt_block(rbt_hip *h, int p0, int T) {
     Launch L;
     L.s = h->stream;
     auto vec = [&](uint64_t off) { return reinterpret_cast<const float *>(h->model + off); };
-    const int32_t *user_counts = h->expert_counts;  // rbt_hip_expert_counts_dev is about the caller's calls
+    const GroupedCall user_call = h->grouped;  // rbt_hip_expert_counts_dev is about the caller's calls
     HIP_OK(h, launch_prompt_embed(L, c.dtype, h->model + h->tok_emb, D, c.vocab, ds.seq + p0, T, p.x));
     for (int l = 0; l < c.n_layers; l++) {
         const LayerOff &ly = h->layers[(size_t)l];
@@ -1148,7 +1148,7 @@ int prompt_block(rbt_hip *h, int p0, int T) {
         if (h->rhist)
             HIP_OK(h, launch_prompt_record(L, w.routing, l, c.n_layers, c.top_k, p0, T, h->rhist));
     }
-    h->expert_counts = user_counts;
+    h->grouped = user_call;
     return 1;
 }
 
@@ -1479,7 +1479,19 @@ int rbt_hip_moe_dev_noalloc(rbt_hip *h, const rbt_moe_layer *L, const float *xb_
     return moe_block(h, L, xb_dev, T, x_dev, moe_dev, routing_dev, weights_dev, w, form, false);
 }
 
-const int32_t *rbt_hip_expert_counts_dev(rbt_hip *h) { return h ? h->expert_counts : nullptr; }
+const int32_t *rbt_hip_expert_counts_dev(rbt_hip *h) { return h ? h->grouped.counts : nullptr; }
+
+int rbt_hip_tile_rows(rbt_hip *h, int *rows) {
+    if (!h || !rows) return fail(h, "tile_rows: NULL argument");
+    *rows = h->grouped.rows;
+    if (!h->grouped.choice) return 1;
+    if (!set_device(h)) return 0;
+    int32_t choice = 0;
+    HIP_OK(h, hipMemcpyAsync(&choice, h->grouped.choice, sizeof choice, hipMemcpyDeviceToHost, h->stream));
+    HIP_OK(h, hipStreamSynchronize(h->stream));
+    *rows = choice & 1 ? 128 : 64;
+    return 1;
+}
 
 // Staging regions between these sizes are copied by kernels.
 constexpr uint64_t kSeamKernelMin = 24u << 10, kSeamKernelBytes = 5u << 18;

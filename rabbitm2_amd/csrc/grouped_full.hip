@@ -479,7 +479,7 @@ hipError_t launch_dense_full(const Launch &L, int dtype, const float *x, int T, 
 hipError_t launch_grouped_full(const Launch &Ld, const Launch &Lg, const Launch &Lw, const Launch &Lc, int dtype,
                                const void *experts, uint64_t stride, const float *xb, int T, int E, int K, int D, int H,
                                const int32_t *routing, const float *weights, float *hbuf, void *ws, float *x_inout,
-                               float *moe_out, int32_t **counts_out) {
+                               float *moe_out, GroupedCall *call_out) {
     if (T <= 0 || K <= 0) return hipErrorInvalidValue;
     const int P = T * K;
     uint8_t *w = static_cast<uint8_t *>(ws);
@@ -496,10 +496,10 @@ hipError_t launch_grouped_full(const Launch &Ld, const Launch &Lg, const Launch 
     int32_t *perm = reinterpret_cast<int32_t *>(carve(4 * (size_t)P));
     int32_t *pos_of = reinterpret_cast<int32_t *>(carve(4 * (size_t)P));
     float *y = reinterpret_cast<float *>(carve(4 * (size_t)P * D));
-    if (counts_out) *counts_out = counts;
     const int rg = P <= kFullShortLists * E ? 2 : 4;
+    if (call_out) *call_out = GroupedCall{counts, 16 * rg, nullptr};
     hipError_t e = launch_dispatch(Ld, routing, P, E, counts, offsets, perm, pos_of, m_off, 16 * rg, m_off128,
-                                   choice, 2, 0, reinterpret_cast<int32_t *>(y));
+                                   choice, 2, PlanShape{}, reinterpret_cast<int32_t *>(y));
     if (e != hipSuccess) return e;
     const int max_mtiles = (P + 16 * rg - 1) / (16 * rg) + E;  // >= sum over experts of ceil(count / (16 rg))
     const uint64_t mat = (uint64_t)H * D * (dtype == RBT_DT_BF16 ? 2 : 4);

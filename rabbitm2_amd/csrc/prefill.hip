@@ -39,22 +39,74 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// Relative time of a wide 128-row tile and of a 64-row tile half as wide, for the plan that dispatch_kernel
-// makes: gate/up, dim 2048, rounds of 256 tiles take 108-120 and 38-42 us (from the second round on; one
-// round of wide tiles, 93-123 us, is never beaten). 64 experts, us per gate/up with wide / 64-row tiles:
-// evenly routed 900 tokens (280 wide tiles, 1040 of 64 rows) 211 / 191, 1024 tokens 224 / 202, 1300 tokens
-// 239 / 230, 2048 tokens 332 / 335; +2 on eight experts' logits 400 tokens (320, 768) 153 / 133, 777 tokens
-// (384, 1024) 216 / 162, 1500 tokens (512, 1600) 229 / 264.
-constexpr int kWideTileCost = 29, kShortTileCost = 10;
-constexpr int kDispRegs = 4;  // 64-pair steps per wave kept in registers by dispatch_kernel (4096 pairs)
+// The plan between wide 128-row tiles and 64-row tiles half as wide (grouped_gemm_wide_kernel), by their times in
+// hundredths of a round of 64-row tiles on the chip's 256 CUs (dim 2048 gate/up 38 us, both in proportion to the
+// reduction length). full: a round of wide tiles of 8 row groups; empty2: less, in halves, per empty row group.
+// Where some list is longer than 4x the mean, the slots run column-major, short lists' tiles end early all over
+// the chip, and a second round of few tiles starts behind those: it then costs second + second_kd / reduction
+// length + per_group for each row group past the third of the tiles that it starts behind (`behind` more than it
+// has), for up to part_max tiles. A tiled copy makes the wide tiles faster, so it has its own figures.
+// us per gate/up + down, wide tiles / wide tiles on a copy / 64-row tiles (dim 2048, 64 experts, top-8, hidden
+// 1024): even 777 tokens (one round) 195 / 184 / 264, 1000 tokens 333 / 310 / 300, 1500 tokens 371 / 359 / 427;
+// +2 on eight experts' logits 400 tokens 226 / 195 / 201, 512 tokens 232 / 197 / 239, 777 tokens 324 / 298 / 249,
+// 1500 tokens 368 / 345 / 436; +1 on 16 experts 400 tokens 322 / 298 / 200. Over 708 histograms at five shapes
+// (dims 512 to 4096, 16 to 128 experts) the pick is at most 6% slower than always wide without a copy (-5% on
+// average) and 13% with one (-3%; 128 experts of ~48 rows, where both are bound by the weights' bytes).
+struct TileCosts {
+    int full, empty2, second, second_kd, per_group, behind, part_max;
+};
+constexpr TileCosts kBlobCosts{290, 15, 80, 40960, 50, 96, 64}, kCopyCosts{260, 5, 60, 20480, 20, 32, 256};
 
+// One wave, experts' totals in c[4] per lane, m128 / m64 row tiles of the two heights: whether the 64-row tiles
+// are the faster ones.
+__device__ __forceinline__ bool short_tiles_pay(const int (&c)[4], int m128, int m64, bool skewed, PlanShape s) {
+    if (m128 * (s.H / 256) <= 256) return false;  // one round of wide tiles
+    const TileCosts k = s.copy ? kCopyCosts : kBlobCosts;
+    int groups = 0;
+    uint64_t rem[2] = {0, 0};  // the lists' last tiles by row groups 1 .. 8, 16 bits each (full tiles not among them)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        groups += (c[i] + 15) / 16;
+        const int q = ((c[i] & 127) + 15) / 16;
+        if (q) rem[(q - 1) >> 2] += 1ull << (16 * ((q - 1) & 3));
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        groups += __shfl_xor(groups, d, 64);
+        rem[0] += __shfl_xor((unsigned long long)rem[0], d, 64);
+        rem[1] += __shfl_xor((unsigned long long)rem[1], d, 64);
+    }
+    const int round = k.full - k.empty2 * (8 * m128 - groups) / (2 * m128);
+    long long wide = 0, shorter = 0;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        const int nt = g ? s.D / 512 : s.H / 256, kd = g ? s.H : s.D;  // wide column tiles, reduction length
+        const int rounds = (m128 * nt + 255) / 256, part = m128 * nt - (rounds - 1) * 256;
+        int cost = rounds * round;
+        if (skewed && rounds == 2 && part <= k.part_max) {
+            const int need = (part + k.behind + nt - 1) / nt;
+            int q = 1, have = (int)(rem[0] & 0xFFFF);
+            while (q < 8 && have < need) {
+                have += (int)(rem[q >> 2] >> (16 * (q & 3))) & 0xFFFF;
+                ++q;
+            }
+            cost = min(cost, round + k.second + k.second_kd / kd + k.per_group * max(0, q - 3) +
+                                 (part > 64 ? 40 + (part - 64) * 5 / 8 : 0));
+        }
+        wide += (long long)cost * kd;
+        shorter += (long long)((m64 * 2 * nt + 255) / 256) * 100 * kd;
+    }
+    return shorter < wide;
+}
+
+constexpr int kDispRegs = 4;  // 64-pair steps per wave kept in registers by dispatch_kernel (4096 pairs)
 
 // One wave: the experts' totals s_tot become their first list positions; with write, also the outputs of the
 // dispatch that follow from the totals (see dispatch_kernel).
 __device__ __forceinline__ void dispatch_scan(int *s_tot, int P, int E, bool write, int32_t *__restrict__ counts,
                                               int32_t *__restrict__ offsets, int32_t *__restrict__ m_off, int mt_rows,
                                               int32_t *__restrict__ m_off2, int32_t *__restrict__ choice, int tall,
-                                              int wide_nt) {
+                                              PlanShape plan) {
     const int lane = threadIdx.x & 63;
     int c[4], mt[4], mt2[4];
 #pragma unroll
@@ -84,6 +136,9 @@ __device__ __forceinline__ void dispatch_scan(int *s_tot, int P, int E, bool wri
             im2 += um2;
         }
     }
+    bool shorter = tall == 1;
+    if (write && !shorter && plan.H)
+        shorter = short_tiles_pay(c, __builtin_amdgcn_readlane(im2, 63), __builtin_amdgcn_readlane(im, 63), skewed, plan);
     int oc = ic - sc, om = im - sm, om2 = im2 - sm2;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -102,10 +157,6 @@ __device__ __forceinline__ void dispatch_scan(int *s_tot, int P, int E, bool wri
             m_off[E] = om + mt[i];
             if (m_off2) {
                 m_off2[E] = om2 + mt2[i];
-                // wide tiles cost kWideTileCost / kShortTileCost of a 64-row one, and a round of 256
-                // ends with its last tile
-                const int rw = ((om2 + mt2[i]) * wide_nt + 255) / 256, rs = ((om + mt[i]) * 2 * wide_nt + 255) / 256;
-                const bool shorter = tall == 1 || (wide_nt && rw > 1 && rs * kShortTileCost < rw * kWideTileCost);
                 choice[0] = shorter ? 0 : (1 | (skewed ? 2 : 0));  // 64-row tiles: expert-major
                 choice[1] = shorter ? om + mt[i] : om2 + mt2[i];    // the plan's row tiles
             }
@@ -137,8 +188,8 @@ __device__ __forceinline__ int rank_pairs(int *row, int e, bool valid, uint64_t 
 // perm[P]: pair ids grouped by expert, increasing within an expert; pos_of[P]: inverse of perm;
 // m_off[E+1]: exclusive prefix of ceil(counts / mt_rows) (the grouped GEMMs' row tiles per expert);
 // with m_off2 given, also m_off2[E+1] for 128-row tiles and choice[2], the grouped GEMMs' plan (and its row
-// tiles): bit 0 the tile height (1: 128 rows, 0: mt_rows; tall = 1 forces mt_rows; else 128, unless wide_nt > 0
-// and the rounds of tiles are cheaper with 64 rows, see kWideTileCost), bit 1 the slot order of the 128-row
+// tiles): bit 0 the tile height (1: 128 rows, 0: mt_rows; tall = 1 forces mt_rows; else 128, unless plan.H > 0
+// and the 64-row tiles are faster, see short_tiles_pay), bit 1 the slot order of the 128-row
 // tiles (column-major when some list is longer than 4x the mean, else expert-major; see tile_of). Without wide
 // tiles, at 512 tokens of the OLMoE layer, 128-row tiles beat 64-row ones with uniform routing (209 against
 // 262 us per call) and, in column-major order, with +2 on 8 experts' logits (247 against 255 us) and +4 on 4
@@ -155,7 +206,7 @@ __global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t *__restric
                                                         int32_t *__restrict__ perm, int32_t *__restrict__ pos_of,
                                                         int32_t *__restrict__ m_off, int mt_rows,
                                                         int32_t *__restrict__ m_off2, int32_t *__restrict__ choice,
-                                                        int tall, int wide_nt) {
+                                                        int tall, PlanShape plan) {
     constexpr int NW = 16;
     __shared__ int s_w[NW][kDispatchMaxE];  // A: running counts per wave; B: each wave's base positions
     __shared__ int s_tot[kDispatchMaxE];    // B: each expert's total, then its first list position
@@ -200,7 +251,7 @@ __global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t *__restric
     }
     __syncthreads();
     if (wv == 0)
-        dispatch_scan(s_tot, P, E, true, counts, offsets, m_off, mt_rows, m_off2, choice, tall, wide_nt);
+        dispatch_scan(s_tot, P, E, true, counts, offsets, m_off, mt_rows, m_off2, choice, tall, plan);
     __syncthreads();
     // B3: each wave's first position for each expert
 #pragma unroll
@@ -278,7 +329,7 @@ __global__ __launch_bounds__(1024) void dispatch_place_kernel(const int32_t *__r
                                                               int32_t *__restrict__ perm, int32_t *__restrict__ pos_of,
                                                               int32_t *__restrict__ m_off, int mt_rows,
                                                               int32_t *__restrict__ m_off2, int32_t *__restrict__ choice,
-                                                              int tall, int wide_nt) {
+                                                              int tall, PlanShape plan) {
     __shared__ int s_tot[kDispatchMaxE], s_base[kDispatchMaxE];
     const int tid = threadIdx.x, nb = gridDim.x, blk = blockIdx.x;
     if (tid < E) {
@@ -293,7 +344,7 @@ __global__ __launch_bounds__(1024) void dispatch_place_kernel(const int32_t *__r
         s_base[tid] = before;
     }
     __syncthreads();
-    if (tid < 64) dispatch_scan(s_tot, P, E, blk == 0, counts, offsets, m_off, mt_rows, m_off2, choice, tall, wide_nt);
+    if (tid < 64) dispatch_scan(s_tot, P, E, blk == 0, counts, offsets, m_off, mt_rows, m_off2, choice, tall, plan);
     __syncthreads();
     for (int p = blk * S + tid; p < min(P, (blk + 1) * S); p += 1024) {
         const int e = min(max(routing[p], 0), E - 1), pos = s_tot[e] + s_base[e] + pos_of[p];
@@ -1343,7 +1394,7 @@ void prefill_x_planes(void *ws, int T, int E, int K, int D, uint16_t **x_hi, uin
 
 hipError_t launch_dispatch(const Launch &L, const int32_t *routing, int P, int E, int32_t *counts, int32_t *offsets,
                            int32_t *perm, int32_t *pos_of, int32_t *m_off, int mt_rows, int32_t *m_off2, int32_t *choice,
-                           int tall, int wide_nt, int32_t *bcnt) {
+                           int tall, PlanShape plan, int32_t *bcnt) {
     if (P < 1 || E < 1 || E > kDispatchMaxE) return hipErrorInvalidValue;
     if (bcnt && P > kDispOneBlockPairs) {
         int per = (P + kDispBlocks - 1) / kDispBlocks;
@@ -1355,10 +1406,10 @@ hipError_t launch_dispatch(const Launch &L, const int32_t *routing, int P, int E
         const hipError_t e = launch(L1, dispatch_count_kernel, g, b, 0, routing, P, E, per, bcnt, pos_of);
         if (e != hipSuccess) return e;
         return launch(L2, dispatch_place_kernel, g, b, 0, routing, P, E, per, (const int32_t *)bcnt, counts, offsets, perm,
-                      pos_of, m_off, mt_rows, m_off2, choice, tall, wide_nt);
+                      pos_of, m_off, mt_rows, m_off2, choice, tall, plan);
     }
     return launch(L, dispatch_kernel, dim3(1), dim3(1024), 0, routing, P, E, counts, offsets, perm, pos_of, m_off,
-                  mt_rows, m_off2, choice, tall, wide_nt);
+                  mt_rows, m_off2, choice, tall, plan);
 }
 
 hipError_t launch_combine(const Launch &Lc, const float *y, const int32_t *pos_of, const float *weights, int T, int K,
@@ -1374,7 +1425,7 @@ hipError_t launch_combine(const Launch &Lc, const float *y, const int32_t *pos_o
 hipError_t launch_prefill(const Launch &Ld, const Launch &Lg, const Launch &Lw, const Launch &Lc, const void *experts,
                           uint64_t stride, const float *xb, int T, int E, int K, int D, int H, const int32_t *routing,
                           const float *weights, float *hbuf, void *ws, float *x_inout, float *moe_out,
-                          int32_t **counts_out, bool x_split_done, bool combine, int tile_rows, const void *tiled,
+                          GroupedCall *call_out, bool x_split_done, bool combine, int tile_rows, const void *tiled,
                           bool wide_ok) {
     if (tile_rows != 0 && tile_rows != 32 && tile_rows != 64 && tile_rows != 128) return hipErrorInvalidValue;
     if (T <= 0 || K <= 0) return hipErrorInvalidValue;  // the dispatch reads at least one pair
@@ -1385,7 +1436,6 @@ hipError_t launch_prefill(const Launch &Ld, const Launch &Lg, const Launch &Lw, 
     uint16_t *x_hi = r.x_hi, *x_lo = r.x_lo;
     // the h planes (bf16 hi, lo; [P][H] each) take the f32 [P][H] h buffer
     uint16_t *h_hi = reinterpret_cast<uint16_t *>(hbuf), *h_lo = h_hi + (size_t)P * H;
-    if (counts_out) *counts_out = counts;
     // activation split (unless the router kernel wrote the planes), then the dispatch: one timed
     // interval (first start .. dispatch end)
     hipError_t e = hipSuccess;
@@ -1410,10 +1460,12 @@ hipError_t launch_prefill(const Launch &Ld, const Launch &Lg, const Launch &Lw, 
     const int mt_rows = small ? 32 : 64;
     const int tall = !tall_ok || small || tile_rows == 64 ? 1 : 2;
     const bool sel = !small && tall_ok;
+    if (call_out) *call_out = GroupedCall{counts, sel ? 0 : mt_rows, sel ? r.choice : nullptr};
     // the wide kernel where the shape has it; it takes 64-row tiles where the dispatch finds them faster
     const bool wide = sel && tall == 2 && wide_ok && gemm_wide_supported(2, H, D) && gemm_wide_supported(1, D, H);
     e = launch_dispatch(Ldd, routing, P, E, counts, offsets, perm, pos_of, m_off, mt_rows, sel ? r.m_off128 : nullptr,
-                        r.choice, tall, wide && tile_rows == 0 ? H / 256 : 0, reinterpret_cast<int32_t *>(y));
+                        r.choice, tall, wide && tile_rows == 0 ? PlanShape{H, D, tiled != nullptr} : PlanShape{},
+                        reinterpret_cast<int32_t *>(y));
     if (e != hipSuccess) return e;
     const uint8_t *ex = static_cast<const uint8_t *>(experts);
     const int max_mtiles = (P + mt_rows - 1) / mt_rows + E;  // >= sum over experts of ceil(count / mt_rows)

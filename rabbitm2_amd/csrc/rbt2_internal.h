@@ -211,6 +211,14 @@ hipError_t launch_experts_decode(const Launch &Lg, const Launch &Ld, int dtype, 
 // fills routing/weights; otherwise it reads routing written by the top-k kernel.
 constexpr int kTopkInGateupMaxE = 64;
 
+// What a grouped call leaves behind for rbt_hip_expert_counts_dev and rbt_hip_tile_rows: the histogram, and
+// the list rows per tile, fixed by the host or (rows 0) chosen on the device (bit 0 of *choice: 128, else 64).
+struct GroupedCall {
+    const int32_t *counts = nullptr;
+    int rows = 0;
+    const int32_t *choice = nullptr;
+};
+
 // Grouped form for many tokens (bf16 weights): dispatch of the (token, slot) pairs into per-expert
 // lists, gate/up and down as grouped GEMMs on MFMA (every expert's weights read once per call), and
 // the combine in selection order. hbuf [T*K][H]; ws holds prefill_workspace_bytes(). *counts_out
@@ -226,7 +234,7 @@ size_t prefill_workspace_bytes(int T, int E, int K, int D);
 hipError_t launch_prefill(const Launch &Ld, const Launch &Lg, const Launch &Lw, const Launch &Lc, const void *experts,
                           uint64_t stride, const float *xb, int T, int E, int K, int D, int H, const int32_t *routing,
                           const float *weights, float *hbuf, void *ws, float *x_inout, float *moe_out,
-                          int32_t **counts_out, bool x_split_done,
+                          GroupedCall *call_out, bool x_split_done,
                           bool combine = true, int tile_rows = 0, const void *tiled = nullptr, bool wide_ok = true);
 // The tiled copy of a layer's bf16 experts that the 128-row grouped GEMMs stream contiguously (same
 // bytes as the blobs, in tile order): whether the shape has one, its size, and the re-layout launch
@@ -249,9 +257,14 @@ hipError_t launch_combine_rmsnorm(const Launch &L, const float *y, const int32_t
 // choice may be NULL together (one tile height, expert-major slots). bcnt: 64 x E ints of scratch that are
 // free until the dispatch is done (the down GEMM's output buffer), for the form of many pairs.
 constexpr int kDispatchMaxE = 256;
+// What the dispatch picks between the wide kernel's two tile heights from (H 0: no choice): the layer's dims and
+// whether the wide tiles read a tiled copy.
+struct PlanShape {
+    int H = 0, D = 0, copy = 0;
+};
 hipError_t launch_dispatch(const Launch &L, const int32_t *routing, int P, int E, int32_t *counts, int32_t *offsets,
                            int32_t *perm, int32_t *pos_of, int32_t *m_off, int mt_rows, int32_t *m_off2, int32_t *choice,
-                           int tall, int wide_nt = 0, int32_t *bcnt = nullptr);
+                           int tall, PlanShape plan = PlanShape{}, int32_t *bcnt = nullptr);
 hipError_t launch_combine(const Launch &L, const float *y, const int32_t *pos_of, const float *weights, int T, int K,
                           int D, float *x_inout, float *moe_out);
 
@@ -266,7 +279,7 @@ size_t full_workspace_bytes(int T, int E, int K, int D);
 hipError_t launch_grouped_full(const Launch &Ld, const Launch &Lg, const Launch &Lw, const Launch &Lc, int dtype,
                                const void *experts, uint64_t stride, const float *xb, int T, int E, int K, int D, int H,
                                const int32_t *routing, const float *weights, float *hbuf, void *ws, float *x_inout,
-                               float *moe_out, int32_t **counts_out);
+                               float *moe_out, GroupedCall *call_out);
 
 // Rows of T tokens through up to three dense matrices on the same kernel (full f32 activation precision):
 // out_s [T][rows_s] = x W_s^T, or with resid != NULL resid [T][rows_0] += (one matrix).

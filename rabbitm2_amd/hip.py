@@ -25,6 +25,7 @@ EXPORTS = (
     "rbt_hip_forward_batch", "rbt_hip_generate_batch", "rbt_hip_set_sampling", "rbt_hip_file_info",
     "rbt_hip_generate_stream", "rbt_hip_routing_history", "rbt_hip_expert_cache_replay",
     "rbt_hip_moe_dev_noalloc", "rbt_hip_prefill_layout", "rbt_hip_prefill_layout_drop", "rbt_hip_profiler_attached",
+    "rbt_hip_tile_rows",
 )
 
 TOKEN_FN = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_int32)
@@ -71,6 +72,7 @@ def lib():
         L.rbt_hip_prefill_layout.argtypes = [vp, C.POINTER(MoeLayer)]
         L.rbt_hip_prefill_layout_drop.argtypes = [vp, C.POINTER(MoeLayer)]
         L.rbt_hip_expert_counts_dev.argtypes, L.rbt_hip_expert_counts_dev.restype = [vp], vp
+        L.rbt_hip_tile_rows.argtypes = [vp, C.POINTER(C.c_int)]
         L.rbt_hip_matvec.argtypes = [vp, vp, u64, vp, i32, i32]
         L.rbt_hip_matvec_dev.argtypes = [vp, vp, vp, i32, vp, i32, i32]
         L.rbt_hip_malloc.argtypes = [vp, C.POINTER(vp), u64]
@@ -361,6 +363,11 @@ class Device:
         out = np.empty(n_experts, np.int32)
         self._check(self.L.rbt_hip_d2h(self.h, _p(out), C.c_void_p(p), out.nbytes))
         return out
+
+    def tile_rows(self):
+        rows = C.c_int()
+        self._check(self.L.rbt_hip_tile_rows(self.h, C.byref(rows)))
+        return rows.value
 
     def matvec_dev(self, out, W, dtype, x, rows, cols):
         self._check(self.L.rbt_hip_matvec_dev(self.h, out.p, W if isinstance(W, C.c_void_p) else W.p, dtype, x.p,
