@@ -81,7 +81,9 @@ __global__ __launch_bounds__(256) void prompt_rope_kernel(float *__restrict__ q,
 // Bound: the serial chain of a wave's key groups (products 128 x 32 clocks per group); 16 queries per
 // block, its keys split over four waves, keep the longest chain at a quarter of the keys and fill the chip
 // (16 heads, 400 positions: 400 blocks, 25.5 us; with the kernel below 16 layers take 1.4 ms longer).
+// A position's output depends on the rows up to its own only, whatever the later ones hold.
 constexpr int kPaQ = 16, kPaKeys = 32, kPaHd = 128;
+constexpr uint32_t kInfBits = 0x7F800000u;
 __global__ __launch_bounds__(256) void prompt_attn_kernel(const float *__restrict__ q, int n_heads, int n_kv, int p0,
                                                           int T, const float *__restrict__ kc,
                                                           const float *__restrict__ vc, float *__restrict__ ao) {
@@ -144,18 +146,41 @@ __global__ __launch_bounds__(256) void prompt_attn_kernel(const float *__restric
         l *= alpha;
 #pragma unroll
         for (int d = 0; d < 8; ++d) o[d] *= alpha;
+        // A key behind a query has weight 0 there, but 0 times an infinity or NaN is NaN, so values that are not
+        // finite stay out of the products and are added below, to the queries that may see them.
+        uint32_t top = 0;
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float p = expf(sc[b][i] - ref);
-                l += p;
-                // keys past this query carry weight 0, whatever their (clamped) row holds
-                const bool none = j0 + 16 * b + 4 * g + i >= n;
+                sc[b][i] = expf(sc[b][i] - ref);
+                l += sc[b][i];
+                const bool none = j0 + 16 * b + 4 * g + i >= n;  // (clamped) rows past the block's keys
 #pragma unroll
-                for (int d = 0; d < 8; ++d)
-                    o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(none ? 0.0f : vr[b][i][d >> 2][d & 3], p, o[d], 0, 0, 0);
+                for (int d = 0; d < 8; ++d) {
+                    const float v = vr[b][i][d >> 2][d & 3];
+                    const uint32_t mag = none ? 0u : __float_as_uint(v) & 0x7FFFFFFFu;
+                    top = max(top, mag);
+                    o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(none || mag >= kInfBits ? 0.0f : v, sc[b][i], o[d], 0,
+                                                                0, 0);
+                }
             }
+        if (__any(top >= kInfBits)) {  // key by key; the weights change lanes through this wave's s_o
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s_o[wv][c][16 * b + 4 * g + i] = sc[b][i];
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            for (int k = 0; k < kPaKeys && j0 + k < n; ++k) {
+                if (j0 + k > last) continue;
+                const float p = s_o[wv][c][k], *vp = vb + (size_t)(j0 + k) * kvd + 32 * g;
+#pragma unroll
+                for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+                    for (int d = 0; d < 8; ++d)
+                        if (!__builtin_isfinite(vp[8 * ii + d])) o[d][ii] += p * vp[8 * ii + d];
+            }
+        }
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);

@@ -81,3 +81,36 @@ def test_block_prompt_matches_steps(history, shape):
     print(f"hd{hd} n{n}: logits {rel:.2e} from the steps'", flush=True)
     assert np.array_equal(got_h, want_h) and np.array_equal(got_r, want_r)
     assert rel <= 1e-4
+
+
+@pytest.mark.parametrize("hd", [128, 64])
+@pytest.mark.parametrize("bad", [0, 5, 21, 31, 32, 38])
+def test_block_prompt_keeps_positions_before_a_nonfinite_one(history, hd, bad):
+    """A token whose embedding holds an infinity makes its own and every later position NaN, and none before it:
+    routing and logits of the earlier ones are the per-token path's, within its own bar above, and so is all
+    routing (NaN logits select experts 0 .. K - 1)."""
+    dev, n = history, 40
+    cfg = po.Config(vocab=96, dim=132, n_layers=2, n_heads=2, n_kv_heads=1, head_dim=hd, n_experts=8, top_k=2,
+                    expert_hidden=72, max_seq=64, dtype=po.DT_BF16, qk_norm=1, norm_topk=1, rope_theta=10000.0,
+                    rms_eps=1e-5)
+    model = po.build_model(cfg, po.GenParams(seed=43, w_scale=1.0, fan_in_scale=1, emb_scale=0.5, norm_jitter=0.1))
+    dev.upload(model)
+    emb, _ = dev.tensor("tok_emb")
+    model[emb + 95 * 2 * cfg.dim:][:2] = (0x80, 0x7F)  # token 95's first element: infinity
+    dev.upload(model)
+    dev.set_router_order(po.ORDER_AVX2)
+    tokens = np.random.default_rng(44).integers(0, 95, n).astype(np.int32)
+    tokens[bad] = 95
+    dev.state_init(64)
+    want = [dev.forward(int(tok), pos, cfg.vocab, cfg.n_layers, cfg.top_k)[0] for pos, tok in enumerate(tokens)]
+    want_h = dev.routing_history(0, 0, n, cfg.n_layers, cfg.top_k)
+    dev.state_init(64)
+    dev.generate(tokens, 0)
+    assert np.array_equal(dev.routing_history(0, 0, n - 1, cfg.n_layers, cfg.top_k), want_h[:n - 1])
+    for pos in sorted({max(bad - 1, 0), max(bad - 15, 0), bad, n - 1}):  # steps back over the block's cache rows
+        got, _ = dev.forward(int(tokens[pos]), pos, cfg.vocab, cfg.n_layers, cfg.top_k)
+        assert np.isnan(want[pos]).all() == (pos >= bad)
+        if pos >= bad:
+            assert np.isnan(got).all()
+        else:
+            assert np.linalg.norm(got - want[pos]) <= 1e-4 * np.linalg.norm(want[pos])
