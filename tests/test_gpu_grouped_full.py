@@ -98,6 +98,53 @@ def test_full_grouped_nonfinite_rows_stay_apart(dev):
         layer.close()
 
 
+@pytest.mark.parametrize("dt", [po.DT_F32, po.DT_BF16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("what", ["inf in w3", "inf in w2", "inf in w1", "overflow in w3", "overflow in w2", "inf in x"])
+@pytest.mark.parametrize("shape", [(68, 36), (512, 132)], ids=["D68", "D512"])
+def test_full_grouped_infinities_are_the_gemvs(dev, what, dt, shape):
+    """Where a weight is infinite or a sum of finite products overflows, the infinities (and their signs) and
+    the NaN are those of the per-pair GEMVs. Activations of one bf16 part, whose other parts are zeros."""
+    D, H = shape
+    layer = SynthLayer(dev, D, 4, 2, H, dt, 0, seed=39, w_scale=1.0, fan_in=True)
+    dev.set_router_order(po.ORDER_AVX2)
+    try:
+        big = 2e19 if "overflow" in what else np.inf
+        enc = np.array([big], np.float32)
+        enc = enc.view(np.uint16)[1:] if dt == po.DT_BF16 else enc
+        mat = D * H
+        first = {"w1": 0, "w3": mat, "w2": 2 * mat}[what[-2:]] if what != "inf in x" else None
+        xb = layer.make_x(16, seed=40)
+        if first is not None:  # one row of the first expert's matrix: every product of it, or its last
+            n = H if what.endswith("w2") else D
+            row = np.repeat(enc, n if "overflow" in what else 1)
+            at = first + 3 * n + (0 if "overflow" in what else n - 1)
+            dev.h2d(layer.experts_dev, row, offset=at * layer.esz)
+        if what == "overflow in w3":
+            xb[3] = 1e19  # products 2e38: any two of them overflow
+        elif what == "overflow in w2":
+            xb[3] = 1e10
+            raw = np.repeat(np.array([1e10], np.float32).view(np.uint16)[1:] if dt == po.DT_BF16
+                            else np.array([1e10], np.float32), 2 * mat)
+            dev.h2d(layer.experts_dev, raw, offset=0)  # gate and up 1e20 D, h past the largest float
+        elif what == "inf in x":
+            xb[3, D - 1] = np.inf
+        dev.set_option("prefill_min_tokens", 65536)
+        want = layer.run_gpu(xb)["moe"]
+        dev.set_option("prefill_min_tokens", 2)
+        got = layer.run_gpu(xb)
+        assert dev.expert_counts(4) is not None and dev.expert_counts(4).sum() == 32
+        got = got["moe"]
+        assert not np.isfinite(want).all()
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+        fin = np.isfinite(want)
+        g64, w64 = got[fin].astype(np.float64), want[fin].astype(np.float64)
+        assert np.linalg.norm(g64 - w64) <= 4e-6 * np.linalg.norm(w64)  # sums of at most 512 f32 products
+    finally:
+        dev.set_option("prefill_min_tokens", 12)
+        layer.close()
+
+
 def test_full_grouped_scratch_limit(dev):
     """rbt_hip_moe_dev_noalloc takes the per-pair GEMVs where the grouped buffers pass its scratch array, so
     the calls that fitted without them still run."""
