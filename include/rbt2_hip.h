@@ -80,10 +80,12 @@ int rbt_hip_set_router_order(rbt_hip *h, int order);
  *                         weights: (token, slot) pairs dispatched into per-expert lists and the
  *                         expert FFN run as grouped GEMMs on the matrix cores, each expert's weights
  *                         read once per call. Smaller T runs one GEMV per pair. Routing is the same
- *                         either way; outputs agree within the parity tolerance. f32 weights, and bf16
- *                         weights whose dims the bf16 tiles do not divide, have a grouped form of their
- *                         own at full f32 activation precision; it is taken where it is faster (by
- *                         size), or from this many tokens (and at least 2) on once the option is set.
+ *                         either way; outputs agree within the parity tolerance.
+ *   "full_min_tokens"     f32 weights, and bf16 weights whose dims the bf16 tiles do not divide or of
+ *                         fewer tokens, have a grouped form of their own at full f32 activation
+ *                         precision, which prompt blocks take too. 0 (default): taken where it is
+ *                         faster, by the size of the call; 1..65536: from that many tokens (and at
+ *                         least 2) on.
  *   "prefill_layout"      1 (default): the grouped GEMMs read a layer's tiled expert copy where the
  *                         caller made one with rbt_hip_prefill_layout (none exists otherwise: by
  *                         default every kernel reads the .rbt2 blobs); 0: the blobs only.

@@ -142,7 +142,7 @@ struct rbt_hip {
     Sampling sampling;     // rbt_hip_set_sampling: how rbt_hip_generate* pick tokens
     uint64_t seed = 0;
     int prefill_min_tokens = kPrefillMinTokensDefault;  // option "prefill_min_tokens"
-    bool prefill_min_set = false;                        // the caller chose it
+    int full_min_tokens = 0;                             // option "full_min_tokens" (0: by size)
     int prefill_tile_rows = 0;  // option "prefill_tile_rows": rows per grouped-GEMM tile, 0 = by batch
     bool prefill_wide = true;   // option "prefill_wide": 128-row tiles 512 weight rows wide
     int gen_timed_from = 1;     // option "generate_timed_from": first generated step of ms_out[1]
@@ -894,11 +894,11 @@ int capture_step(rbt_hip *h, bool final, hipGraphExec_t *exec) {
     return 1;
 }
 
-// Whether T tokens take the full-precision grouped form by size: where it beats the per-pair GEMVs, or from
-// the caller's own "prefill_min_tokens" on.
+// Whether T tokens take the full-precision grouped form: where it beats the per-pair GEMVs, or from the caller's
+// own "full_min_tokens" on.
 bool full_from(const rbt_hip *h, int dtype, int T, int E, int K, int D, int H, const void *experts, uint64_t stride,
                const float *xb) {
-    if (h->prefill_min_set) return T >= h->prefill_min_tokens;
+    if (h->full_min_tokens) return T >= h->full_min_tokens;
     return full_pays(experts_decode_supported(dtype, T, K, D, H, experts, stride, xb, xb), dtype, T, E, K, D, H);
 }
 
@@ -1659,7 +1659,9 @@ int rbt_hip_set_option(rbt_hip *h, const char *name, int64_t value) {
     } else if (strcmp(name, "prefill_min_tokens") == 0) {
         if (value < 1 || value > 65536) return fail(h, "set_option: prefill_min_tokens must be in [1, 65536]");
         h->prefill_min_tokens = (int)value;
-        h->prefill_min_set = true;
+    } else if (strcmp(name, "full_min_tokens") == 0) {
+        if (value < 0 || value > 65536) return fail(h, "set_option: full_min_tokens must be in [0, 65536]");
+        h->full_min_tokens = (int)value;
     } else if (strcmp(name, "prefill_tile_rows") == 0) {
         if (value != 0 && value != 32 && value != 64 && value != 128)
             return fail(h, "set_option: prefill_tile_rows must be 0, 32, 64 or 128");

@@ -31,6 +31,7 @@ def test_rows_are_the_single_tokens_rows(dev, case):
     bias = np.array([float(b)] + [0.0] * (E - 1), np.float32) if b else None
     layer = SynthLayer(dev, D, E, K, H, dt, 1, seed=51, w_scale=1.0, fan_in=True, bias=bias)
     dev.set_option("prefill_min_tokens", 1000)  # the GEMVs at every T here
+    dev.set_option("full_min_tokens", 1000)
     try:
         dev.set_router_order(po.ORDER_AVX2)
         xb, x = layer.make_x(T, seed=52, bf16=False), layer.make_x(T, seed=53)
@@ -41,4 +42,5 @@ def test_rows_are_the_single_tokens_rows(dev, case):
                 assert got[k][t].tobytes() == one[k][0].tobytes(), (t, k)
     finally:
         dev.set_option("prefill_min_tokens", 12)
+        dev.set_option("full_min_tokens", 0)
         layer.close()

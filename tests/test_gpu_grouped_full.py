@@ -1,5 +1,5 @@
 """The full-precision grouped form (rabbitm2_amd/csrc/grouped_full.hip): f32 weights, and bf16 weights of
-dims that the bf16 tiles do not divide, from "prefill_min_tokens" tokens on.
+dims that the bf16 tiles do not divide, where it is faster or from "full_min_tokens" tokens on.
 
 Each output is held to its value in 64 bits within the worst case of its own sums: a sum of n f32 products
 in blocks of 64 columns and then over the blocks is off by at most gamma = (64 + n / 32 + 16) * 2^-24 of the
@@ -14,6 +14,14 @@ from oracle import pyoracle as po
 from tests.common import SynthLayer, routing_check
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def by_size(dev):
+    """Every test leaves the choice of the form to the size of the call again."""
+    yield
+    dev.set_option("full_min_tokens", 0)
+
 
 SHAPES = [
     # (D, E, K, H, dtype, T, bias on expert 0)
@@ -59,7 +67,7 @@ def reference(layer, xb, routing, weights):
 def test_full_grouped_shapes(dev, shape):
     D, E, K, H, dt, T, b = shape
     bias = np.array([float(b)] + [0.0] * (E - 1), np.float32) if b else None
-    dev.set_option("prefill_min_tokens", 12)  # from 12 tokens on whatever the sizes
+    dev.set_option("full_min_tokens", 12)  # from 12 tokens on whatever the sizes
     layer = SynthLayer(dev, D, E, K, H, dt, 1, seed=31, w_scale=1.0, fan_in=True, bias=bias)
     try:
         dev.set_router_order(po.ORDER_AVX2)
@@ -82,7 +90,7 @@ def test_full_grouped_shapes(dev, shape):
 
 def test_full_grouped_nonfinite_rows_stay_apart(dev):
     """A token with infinities and NaN leaves the other tokens' rows as they are without it."""
-    dev.set_option("prefill_min_tokens", 12)
+    dev.set_option("full_min_tokens", 12)
     layer = SynthLayer(dev, 68, 4, 4, 36, po.DT_BF16, 0, seed=35, w_scale=1.0, fan_in=True)
     try:
         dev.set_router_order(po.ORDER_AVX2)
@@ -128,9 +136,9 @@ def test_full_grouped_infinities_are_the_gemvs(dev, what, dt, shape):
             dev.h2d(layer.experts_dev, raw, offset=0)  # gate and up 1e20 D, h past the largest float
         elif what == "inf in x":
             xb[3, D - 1] = np.inf
-        dev.set_option("prefill_min_tokens", 65536)
+        dev.set_option("full_min_tokens", 65536)
         want = layer.run_gpu(xb)["moe"]
-        dev.set_option("prefill_min_tokens", 2)
+        dev.set_option("full_min_tokens", 2)
         got = layer.run_gpu(xb)
         assert dev.expert_counts(4) is not None and dev.expert_counts(4).sum() == 32
         got = got["moe"]
@@ -141,7 +149,6 @@ def test_full_grouped_infinities_are_the_gemvs(dev, what, dt, shape):
         g64, w64 = got[fin].astype(np.float64), want[fin].astype(np.float64)
         assert np.linalg.norm(g64 - w64) <= 4e-6 * np.linalg.norm(w64)  # sums of at most 512 f32 products
     finally:
-        dev.set_option("prefill_min_tokens", 12)
         layer.close()
 
 
@@ -149,7 +156,7 @@ def test_full_grouped_scratch_limit(dev):
     """rbt_hip_moe_dev_noalloc takes the per-pair GEMVs where the grouped buffers pass its scratch array, so
     the calls that fitted without them still run."""
     D, E, K, H, T = 2048, 8, 8, 64, 1200  # y alone is 75 MiB; the GEMVs need 2.4 MiB
-    dev.set_option("prefill_min_tokens", 12)
+    dev.set_option("full_min_tokens", 12)
     layer = SynthLayer(dev, D, E, K, H, po.DT_F32, 1, seed=37, w_scale=1.0, fan_in=True)
     xb = layer.make_x(T, seed=38)
     xd, moe = dev.upload_array(xb), dev.malloc(4 * T * D)
@@ -163,3 +170,49 @@ def test_full_grouped_scratch_limit(dev):
         dev.free(xd)
         dev.free(moe)
         layer.close()
+
+
+# (D, E, K, H, dtype) around the number of tokens from which the grouped form is taken. The lines:
+# 100e6 expected saved bytes, 450e6 for the shapes of the specialised GEMVs, 1000e6 where their gate/up reads an
+# expert once.
+LINES = [(1600, 40, 6, 800, po.DT_BF16), (1000, 20, 3, 330, po.DT_BF16), (260, 6, 2, 132, po.DT_F32),
+         (512, 8, 2, 512, po.DT_F32), (2048, 64, 8, 1024, po.DT_F32)]
+
+
+@pytest.mark.parametrize("shape", LINES, ids=["D%dE%dK%dH%ddt%d" % s for s in LINES])
+def test_full_grouped_is_taken_by_size(shape):
+    """A handle whose options nobody set: on either side of the line the call's bits are those of the form it is
+    expected to take, and not the other's; setting "prefill_min_tokens" changes nothing of it, and
+    "full_min_tokens" 0 brings the size back."""
+    from rabbitm2_amd.hip import Device
+    D, E, K, H, dt = shape
+    esz = po.ELEM[dt]
+    fast = (D * esz) % 1024 == 0 and (H * esz) % 1024 == 0  # the specialised GEMVs' rows, in whole wave-steps
+
+    def takes_grouped(T):
+        p, sel = T * K, E * (1.0 - (1.0 - K / E) ** T)
+        once = p <= 128 and D * esz <= 1024 * (4 if dt == po.DT_BF16 else 8) and (p - sel) * 2.0 * H * D * esz >= 60e6
+        return (p - sel) * 3.0 * H * D * esz >= (100e6 if not fast else 1000e6 if once else 450e6)
+
+    edge = next(T for T in range(2, 2000) if takes_grouped(T))
+    with Device(0) as dev:
+        layer = SynthLayer(dev, D, E, K, H, dt, 1, seed=45, w_scale=1.0, fan_in=True)
+        try:
+            dev.set_router_order(po.ORDER_AVX2)
+            for T in (edge - 1, edge):
+                xb = layer.make_x(T, seed=46, bf16=False)
+                got = layer.run_gpu(xb)["moe"].tobytes()
+                dev.set_option("prefill_min_tokens", 12)
+                dev.set_option("full_min_tokens", 65536)
+                gemvs = layer.run_gpu(xb)["moe"].tobytes()
+                dev.set_option("full_min_tokens", 2)
+                grouped = layer.run_gpu(xb)["moe"].tobytes()
+                dev.set_option("full_min_tokens", 0)
+                assert layer.run_gpu(xb)["moe"].tobytes() == got
+                assert gemvs != grouped
+                assert got == (grouped if T == edge else gemvs), T
+            for bad in (-1, 65537):
+                with pytest.raises(Exception):
+                    dev.set_option("full_min_tokens", bad)
+        finally:
+            layer.close()

@@ -136,8 +136,9 @@ def test_grouped_deterministic(dev, grouped_from):
 
 
 def test_grouped_not_taken_for_f32(dev, grouped_from):
-    """f32 weights stay on the GEMV path (the MFMA path multiplies bf16 weights); results still meet
-    the bar."""
+    """f32 weights never take the bf16 tiles, whatever "prefill_min_tokens" is: a call this small runs the
+    per-pair GEMVs, bit for bit, as it does when the full-precision grouped form is put out of reach; results
+    meet the bar."""
     grouped_from(1)
     layer = SynthLayer(dev, 256, 8, 2, 256, po.DT_F32, 1, seed=4, w_scale=1.0, fan_in=True)
     try:
@@ -147,7 +148,12 @@ def test_grouped_not_taken_for_f32(dev, grouped_from):
         got = layer.run_gpu(xb)
         assert routing_check(got["routing"], want["routing"], want["probs"])[1] == 0
         assert normwise_err(got["moe"], want["moe"]) <= MOE_RTOL
+        dev.set_option("full_min_tokens", 65536)
+        assert layer.run_gpu(xb)["moe"].tobytes() == got["moe"].tobytes()
+        dev.set_option("full_min_tokens", 2)
+        assert layer.run_gpu(xb)["moe"].tobytes() != got["moe"].tobytes()
     finally:
+        dev.set_option("full_min_tokens", 0)
         layer.close()
 
 

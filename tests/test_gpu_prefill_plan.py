@@ -141,7 +141,7 @@ def test_dispatch_of_many_pairs(dev, E, K, T):
     the token alone gives within the two forms' rounding, and the histogram is the routing's."""
     layer = SynthLayer(dev, 64, E, K, 32, po.DT_BF16, 0, seed=62, w_scale=1.0, fan_in=True)
     try:
-        dev.set_option("prefill_min_tokens", 12)
+        dev.set_option("full_min_tokens", 12)
         dev.set_router_order(po.ORDER_AVX2)
         xb = layer.make_x(T, seed=63)
         got = layer.run_gpu(xb)
@@ -151,4 +151,5 @@ def test_dispatch_of_many_pairs(dev, E, K, T):
         rel = np.linalg.norm(got["moe"][pick] - want["moe"], axis=1) / np.linalg.norm(want["moe"], axis=1)
         assert rel.max() <= 1e-5  # sums of at most 64 f32 products in other orders
     finally:
+        dev.set_option("full_min_tokens", 0)
         layer.close()

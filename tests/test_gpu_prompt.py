@@ -29,6 +29,7 @@ def history(dev):
     dev.set_option("routing_history", 1)
     yield dev
     dev.set_option("routing_history", 0)
+    dev.set_option("full_min_tokens", 0)
 
 
 @pytest.mark.parametrize("tag", sorted(ORDERS))
@@ -59,9 +60,11 @@ BLOCKS = [
 ]
 
 
+@pytest.mark.parametrize("form", ["gemvs", "grouped"])
 @pytest.mark.parametrize("shape", BLOCKS, ids=["hd%dh%dkv%ddt%dn%d" % b for b in BLOCKS])
-def test_block_prompt_matches_steps(history, shape):
+def test_block_prompt_matches_steps(history, shape, form):
     dev = history
+    dev.set_option("full_min_tokens", 2 if form == "grouped" else 65536)  # the blocks' MoE form
     hd, heads, kv, dt, n = shape
     cfg = po.Config(vocab=96, dim=132, n_layers=2, n_heads=heads, n_kv_heads=kv, head_dim=hd, n_experts=8, top_k=2,
                     expert_hidden=72, max_seq=700, dtype=dt, qk_norm=1, norm_topk=1, rope_theta=10000.0, rms_eps=1e-5)
