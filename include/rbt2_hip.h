@@ -156,7 +156,9 @@ int rbt_hip_moe(rbt_hip *h, int layer, const float *xb, int T, float *x_inout, i
  *   routing_dev [T][top_k]  int32 expert ids, selection order
  *   weights_dev [T][top_k]  combine weights (after norm_topk renormalisation, rabbit2.c:539)
  * Workspace is taken from the handle; it grows (hipMalloc) only when T exceeds every earlier
- * call's T, so call rbt_hip_reserve() first to keep allocation off the per-token path. */
+ * call's T, so call rbt_hip_reserve() first to keep allocation off the per-token path. Where the buffers
+ * of the full-precision grouped form (option "full_min_tokens") cannot be allocated, or not while the
+ * stream is being captured, the per-pair GEMVs run instead. */
 int rbt_hip_moe_dev(rbt_hip *h, const rbt_moe_layer *L, const float *xb_dev, int T, float *x_dev, float *moe_dev,
                     int32_t *routing_dev, float *weights_dev);
 int rbt_hip_reserve(rbt_hip *h, const rbt_moe_layer *L, int max_tokens);

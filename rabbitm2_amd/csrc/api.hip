@@ -407,6 +407,27 @@ int pre_reserve(rbt_hip *h, size_t bytes) {
     return 1;
 }
 
+// The same for the full-precision grouped form, which no call depends on: 0 where the memory cannot be had, or
+// not now because the stream is being captured (the per-pair GEMVs run instead); -1 where the stream fails.
+int full_reserve(rbt_hip *h, size_t bytes) {
+    Workspace &w = h->ws;
+    if (bytes <= w.pre_bytes) return 1;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(h->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return 0;
+    if (HIP_TRY(hipStreamSynchronize(h->stream)) != hipSuccess) return -1;
+    (void)hipFree(w.pre);
+    w.pre = nullptr;
+    w.pre_bytes = 0;
+    h->grouped = GroupedCall{};
+    if (HIP_TRY(hipMalloc(&w.pre, bytes)) != hipSuccess) {
+        (void)hipGetLastError();
+        w.pre = nullptr;
+        return 0;
+    }
+    w.pre_bytes = bytes;
+    return 1;
+}
+
 int stage_reserve(rbt_hip *h, uint64_t bytes) {
     if (bytes <= h->stage_bytes) return 1;
     HIP_OK(h, hipStreamSynchronize(h->stream));
@@ -1437,9 +1458,11 @@ int rbt_hip_reserve(rbt_hip *h, const rbt_moe_layer *L, int max_tokens) {
     const int T = max_tokens > 0 ? max_tokens : 1;
     if (!ws_reserve(h, T, L->n_experts, L->top_k, L->expert_hidden)) return 0;
     // the larger of the two grouped forms' (it adds the activation planes), for any alignment of the rows
-    if (T >= h->prefill_min_tokens ||
-        full_from(h, L->dtype, T, L->n_experts, L->top_k, L->dim, L->expert_hidden, L->experts, 1, nullptr))
-        return pre_reserve(h, prefill_workspace_bytes(T, L->n_experts, L->top_k, L->dim));
+    const size_t pre = prefill_workspace_bytes(T, L->n_experts, L->top_k, L->dim);
+    if (T >= h->prefill_min_tokens) return pre_reserve(h, pre);
+    if (full_from(h, L->dtype, T, L->n_experts, L->top_k, L->dim, L->expert_hidden, L->experts, 1, nullptr) &&
+        full_reserve(h, pre) < 0)
+        return fail(h, "reserve: %s failed", failed_call());
     return 1;
 }
 
@@ -1452,8 +1475,15 @@ int rbt_hip_moe_dev(rbt_hip *h, const rbt_moe_layer *L, const float *xb_dev, int
     if (!xb_dev) return fail(h, "moe: xb is NULL");
     if (!set_device(h)) return 0;
     if (!ws_reserve(h, T, L->n_experts, L->top_k, L->expert_hidden)) return 0;
-    const MoeForm form = moe_form(h, L, T, xb_dev);
-    if (!pre_reserve(h, pre_bytes_of(form, T, L->n_experts, L->top_k, L->dim))) return 0;
+    MoeForm form = moe_form(h, L, T, xb_dev);
+    const size_t pre = pre_bytes_of(form, T, L->n_experts, L->top_k, L->dim);
+    if (form == kMoeGroupedFull) {
+        const int room = full_reserve(h, pre);
+        if (room < 0) return fail(h, "moe: %s failed", failed_call());
+        if (room == 0) form = kMoeGeneral;
+    } else if (!pre_reserve(h, pre)) {
+        return 0;
+    }
     return moe_block(h, L, xb_dev, T, x_dev, moe_dev, routing_dev, weights_dev, h->ws, form, true);
 }
 

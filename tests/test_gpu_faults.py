@@ -131,3 +131,32 @@ def test_cli_exits_1_with_the_message(tmp_path):
         assert res.returncode == 1 and what in res.stderr, (fault, res.returncode, res.stderr)
     res = subprocess.run([CLI, str(path), "--gen", "4"] + toks, capture_output=True, text=True, timeout=120)
     assert res.returncode == 0 and [int(t) for t in res.stdout.split()] == fx["gen_scalar"][:4].tolist()
+
+
+CHILD_LAYER = r"""
+import sys
+import numpy as np
+sys.path.insert(0, sys.argv[1])
+from oracle import pyoracle as po
+from rabbitm2_amd.hip import Device
+from tests.common import SynthLayer
+with Device(0) as dev:
+    dev.set_router_order(po.ORDER_AVX2)
+    layer = SynthLayer(dev, 1600, 40, 6, 800, po.DT_BF16, 1, seed=7, w_scale=1.0, fan_in=True)
+    xb = layer.make_x(60, seed=8, bf16=False)
+    first, second = (layer.run_gpu(xb)["moe"].tobytes() for _ in range(2))
+    dev.set_option("full_min_tokens", 65536)
+    gemvs = layer.run_gpu(xb)["moe"].tobytes()
+    print("RESULT", first == gemvs, second == gemvs, flush=True)
+"""
+
+
+def test_no_memory_for_the_grouped_buffers_runs_the_gemvs():
+    """A call that the full-precision grouped form would take, whose buffers cannot be allocated (the 11th
+    allocation: the layer's two, four of the first call's arguments, four of the workspace, then theirs): the per-pair
+    GEMVs run, and the next call takes the grouped form."""
+    res = subprocess.run([sys.executable, "-c", CHILD_LAYER, ROOT], capture_output=True, text=True, timeout=300,
+                         env=dict(os.environ, RBT_HIP_FAULT="malloc:11"))
+    assert res.returncode == 0, res.stderr[-3000:]
+    assert "injecting a failure into hipMalloc(&w.pre" in res.stderr, res.stderr
+    assert [ln for ln in res.stdout.splitlines() if ln.startswith("RESULT")] == ["RESULT True False"]

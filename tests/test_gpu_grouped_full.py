@@ -216,3 +216,47 @@ def test_full_grouped_is_taken_by_size(shape):
                     dev.set_option("full_min_tokens", bad)
         finally:
             layer.close()
+
+
+def test_full_grouped_under_capture():
+    """A captured call allocates nothing: where the workspace was not reserved for the grouped form, the per-pair
+    GEMVs are captured, and after an eager call the grouped form is. Each replay gives the eager call's bits."""
+    import ctypes as C
+
+    from rabbitm2_amd.hip import Device
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+    hip.hipGraphInstantiate.argtypes = [C.POINTER(C.c_void_p), C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
+    hip.hipGraphLaunch.argtypes = [C.c_void_p, C.c_void_p]
+    hip.hipGraphExecDestroy.argtypes = hip.hipGraphDestroy.argtypes = [C.c_void_p]
+    D, T = 100, 40
+    with Device(0) as dev:
+        layer = SynthLayer(dev, D, 7, 3, 33, po.DT_BF16, 1, seed=47, w_scale=1.0, fan_in=True)
+        xb = layer.make_x(T, seed=48, bf16=False)
+        xd, moe = dev.upload_array(xb), dev.malloc(4 * T * D)
+        dev.set_router_order(po.ORDER_AVX2)
+        dev.moe_dev(layer.desc(), xd, T, moe=moe)  # by size: the GEMVs
+        dev.synchronize()
+        gemvs = dev.d2h(moe, (T, D), np.float32).tobytes()
+        dev.set_option("full_min_tokens", 2)
+        grouped = None
+        for reserved in (False, True):
+            if reserved:
+                dev.moe_dev(layer.desc(), xd, T, moe=moe)
+                dev.synchronize()
+                grouped = dev.d2h(moe, (T, D), np.float32).tobytes()
+                assert grouped != gemvs
+            graph, gexec = C.c_void_p(), C.c_void_p()
+            assert hip.hipStreamBeginCapture(dev.stream, 2) == 0
+            dev.moe_dev(layer.desc(), xd, T, moe=moe)
+            assert hip.hipStreamEndCapture(dev.stream, C.byref(graph)) == 0
+            assert hip.hipGraphInstantiate(C.byref(gexec), graph, None, None, 0) == 0
+            for _ in range(3):
+                dev.memset(moe, 0)
+                assert hip.hipGraphLaunch(gexec, dev.stream) == 0
+                dev.synchronize()
+                assert dev.d2h(moe, (T, D), np.float32).tobytes() == (grouped if reserved else gemvs)
+            hip.hipGraphExecDestroy(gexec)
+            hip.hipGraphDestroy(graph)
+        layer.close()
