@@ -1133,10 +1133,7 @@ int prompt_reserve(rbt_hip *h, int n) {
     return n;
 }
 
-// forward() (rabbit2.c:453-542, without the final norm and lm_head) of positions p0 .. p0 + T - 1 of the
-// single sequence, whose tokens are in seq[] and whose earlier positions are in the cache. Everything is
-// enqueued on the handle stream.
-int prompt_block(rbt_hip *h, int p0, int T) {
+int prompt_layers(rbt_hip *h, int p0, int T) {
     const rbt_config &c = h->cfg;
     const DecodeState &ds = h->ds;
     const PromptBuf &p = h->prompt;
@@ -1144,7 +1141,6 @@ int prompt_block(rbt_hip *h, int p0, int T) {
     Launch L;
     L.s = h->stream;
     auto vec = [&](uint64_t off) { return reinterpret_cast<const float *>(h->model + off); };
-    const GroupedCall user_call = h->grouped;  // rbt_hip_expert_counts_dev is about the caller's calls
     HIP_OK(h, launch_prompt_embed(L, c.dtype, h->model + h->tok_emb, D, c.vocab, ds.seq + p0, T, p.x));
     for (int l = 0; l < c.n_layers; l++) {
         const LayerOff &ly = h->layers[(size_t)l];
@@ -1169,8 +1165,18 @@ int prompt_block(rbt_hip *h, int p0, int T) {
         if (h->rhist)
             HIP_OK(h, launch_prompt_record(L, w.routing, l, c.n_layers, c.top_k, p0, T, h->rhist));
     }
-    h->grouped = user_call;
     return 1;
+}
+
+// forward() (rabbit2.c:453-542, without the final norm and lm_head) of positions p0 .. p0 + T - 1 of the
+// single sequence, whose tokens are in seq[] and whose earlier positions are in the cache. Everything is
+// enqueued on the handle stream.
+int prompt_block(rbt_hip *h, int p0, int T) {
+    // rbt_hip_expert_counts_dev is about the caller's calls, and this buffer goes with the decode state
+    const GroupedCall user_call = h->grouped;
+    const int ok = prompt_layers(h, p0, T);
+    h->grouped = user_call;
+    return ok;
 }
 
 }  // namespace

@@ -160,3 +160,55 @@ def test_no_memory_for_the_grouped_buffers_runs_the_gemvs():
     assert res.returncode == 0, res.stderr[-3000:]
     assert "injecting a failure into hipMalloc(&w.pre" in res.stderr, res.stderr
     assert [ln for ln in res.stdout.splitlines() if ln.startswith("RESULT")] == ["RESULT True False"]
+
+
+CHILD_PROMPT = r"""
+import json, sys
+import numpy as np
+sys.path.insert(0, sys.argv[1])
+from oracle import pyoracle as po
+from rabbitm2_amd.hip import Device, HipError
+cfg = po.Config(vocab=96, dim=132, n_layers=2, n_heads=2, n_kv_heads=1, head_dim=64, n_experts=8, top_k=2,
+                expert_hidden=72, max_seq=128, dtype=po.DT_BF16, qk_norm=1, norm_topk=1, rope_theta=10000.0,
+                rms_eps=1e-5)
+model = po.build_model(cfg, po.GenParams(seed=41, w_scale=1.0, fan_in_scale=1, emb_scale=0.5, norm_jitter=0.1))
+rng = np.random.default_rng(42)
+tokens = rng.integers(0, cfg.vocab, 100).astype(np.int32)
+with Device(0) as dev:
+    dev.set_router_order(po.ORDER_AVX2)
+    dev.upload(model)
+    dev.state_init(0)
+    exec(sys.argv[2])
+"""
+
+
+def prompt_child(body, fault=None):
+    env = dict(os.environ, **({"RBT_HIP_FAULT": fault} if fault else {}))
+    res = subprocess.run([sys.executable, "-c", CHILD_PROMPT, ROOT, body], capture_output=True, text=True, timeout=300,
+                         env=env)
+    assert res.returncode == 0, res.stderr[-3000:]
+    return json.loads([ln for ln in res.stdout.splitlines() if ln.startswith("RESULT ")][-1][7:]), res.stderr
+
+
+def test_failed_prompt_block_keeps_the_callers_histogram():
+    """A prompt block that fails in its second layer (the 13th launch: two of the caller's own MoE call, the
+    embedding, eight of the first layer, then its second launch) leaves rbt_hip_expert_counts_dev at the caller's
+    last call, not at the block's buffer, which the next state_init frees."""
+    body = """
+dev.set_option("full_min_tokens", 2)
+xb, moe = dev.upload_array(rng.standard_normal((5, 132)).astype(np.float32)), dev.malloc(5 * 132 * 4)
+dev.moe_dev(dev.layer(0), xb, 5, moe=moe)
+before = dev.expert_counts(8).tolist()
+try:
+    dev.generate(tokens[:40], 0)
+    failed = ""
+except HipError as e:
+    failed = str(e)
+after = dev.expert_counts(8).tolist()
+dev.state_init(0)
+dev.generate(tokens[:40], 0)
+print("RESULT " + json.dumps([failed, before, after, dev.expert_counts(8).tolist()]), flush=True)
+"""
+    (failed, before, after, later), _ = prompt_child(body, "launch:13")
+    assert "launch_dense_full" in failed and sum(before) == 10
+    assert after == before and later == before
