@@ -94,7 +94,7 @@ struct DecodeState {
 };
 
 // Buffers of a prompt block (prompt_block): one allocation for `tokens` positions, made by the first prompt
-// long enough, freed with the decode state.
+// long enough and again by one that needs more, freed with the decode state.
 struct PromptBuf {
     int tokens = 0;
     uint8_t *block = nullptr;
@@ -1071,7 +1071,7 @@ int moe_block(rbt_hip *h, const rbt_moe_layer *L, const float *xb_dev, int T, fl
 }
 
 // ---- a prompt in blocks of positions (rabbit2.c:703-714 token by token)
-constexpr int kPromptBlock = 512;  // positions per block at most
+constexpr int kPromptBlock = 512;  // positions per block at most, a power of two times kPromptMinTokens
 // Positions from which a block beats the per-token steps (16 layers of the dim-2048 model): 4 positions 2.9
 // against 3.5 ms, 23 positions 3.5 against 16.2 ms, 399 positions 7.4 against 270 ms.
 constexpr int kPromptMinTokens = 4;
@@ -1088,49 +1088,54 @@ MoeForm prompt_form(const rbt_hip *h, const rbt_moe_layer *L, int T) {
 }
 
 // How many of n leading prompt positions of the single sequence are to be run in blocks (0: none, token by
-// token), with the buffers for them in place. Where they cannot be had, the tokens run one by one; -1 where
-// the stream itself fails.
+// token), with the buffers for blocks of h->prompt.tokens in place. They have room for a power of two of
+// positions, so that prompts that grow call by call seldom allocate anew. Where that cannot be had, the blocks
+// are shorter, down to none; -1 where the stream itself fails.
 int prompt_reserve(rbt_hip *h, int n) {
     const rbt_config &c = h->cfg;
-    const int qd = c.n_heads * c.head_dim, kvd = c.n_kv_heads * c.head_dim, T = std::min(n, kPromptBlock);
-    if (n < kPromptMinTokens || !dense_full_supported(c.dtype, T, c.dim, std::max(qd, kvd), nullptr) ||
-        !dense_full_supported(c.dtype, T, qd, c.dim, nullptr))
+    const int qd = c.n_heads * c.head_dim, kvd = c.n_kv_heads * c.head_dim, want = std::min(n, kPromptBlock);
+    if (n < kPromptMinTokens || !dense_full_supported(c.dtype, want, c.dim, std::max(qd, kvd), nullptr) ||
+        !dense_full_supported(c.dtype, want, qd, c.dim, nullptr))
         return 0;
     PromptBuf &p = h->prompt;
-    if (T <= p.tokens) return n;
-    rbt_moe_layer ml;
-    if (!rbt_hip_layer(h, 0, &ml)) return 0;
-    size_t off = 0;
-    auto carve = [&](size_t floats) {
-        const size_t at = off;
-        off += up256(4 * floats);
-        return at;
-    };
-    const size_t t = (size_t)T, ox = carve(t * c.dim), oxb = carve(t * c.dim), oq = carve(t * qd), ok = carve(t * kvd),
-                 ov = carve(t * kvd), oa = carve(t * qd), om = off;
-    // room for either form at any block length up to T
-    off += std::max(moe_scratch_bytes(T, c.n_experts, c.top_k, c.expert_hidden, c.dim, kMoeGroupedFull),
-                    moe_scratch_bytes(T, c.n_experts, c.top_k, c.expert_hidden, c.dim, kMoeGeneral));
-    uint8_t *b = nullptr;
+    if (want <= p.tokens) return n;
     if (p.block) {  // smaller ones, which earlier work on the stream may still use
         if (HIP_TRY(hipStreamSynchronize(h->stream)) != hipSuccess) return -1;
         (void)hipFree(p.block);
         p = PromptBuf{};
     }
-    if (HIP_TRY(hipMalloc(&b, off)) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
+    int room = kPromptMinTokens;
+    while (room < want) room *= 2;
+    for (; room >= kPromptMinTokens; room /= 2) {
+        const size_t t = (size_t)std::min(room, h->ds.ctx - 1);  // no prompt has more positions before its last
+        size_t off = 0;
+        auto carve = [&](size_t floats) {
+            const size_t at = off;
+            off += up256(4 * floats);
+            return at;
+        };
+        const size_t ox = carve(t * c.dim), oxb = carve(t * c.dim), oq = carve(t * qd), ok = carve(t * kvd),
+                     ov = carve(t * kvd), oa = carve(t * qd), om = off;
+        // for either form at any block length up to t
+        off += std::max(moe_scratch_bytes((int)t, c.n_experts, c.top_k, c.expert_hidden, c.dim, kMoeGroupedFull),
+                        moe_scratch_bytes((int)t, c.n_experts, c.top_k, c.expert_hidden, c.dim, kMoeGeneral));
+        uint8_t *b = nullptr;
+        if (HIP_TRY(hipMalloc(&b, off)) != hipSuccess) {
+            (void)hipGetLastError();
+            continue;
+        }
+        p.block = b;
+        p.tokens = (int)t;
+        p.x = reinterpret_cast<float *>(b + ox);
+        p.xb = reinterpret_cast<float *>(b + oxb);
+        p.q = reinterpret_cast<float *>(b + oq);
+        p.k = reinterpret_cast<float *>(b + ok);
+        p.v = reinterpret_cast<float *>(b + ov);
+        p.ao = reinterpret_cast<float *>(b + oa);
+        p.moe = b + om;
+        return n;
     }
-    p.block = b;
-    p.tokens = T;
-    p.x = reinterpret_cast<float *>(b + ox);
-    p.xb = reinterpret_cast<float *>(b + oxb);
-    p.q = reinterpret_cast<float *>(b + oq);
-    p.k = reinterpret_cast<float *>(b + ok);
-    p.v = reinterpret_cast<float *>(b + ov);
-    p.ao = reinterpret_cast<float *>(b + oa);
-    p.moe = b + om;
-    return n;
+    return 0;
 }
 
 int prompt_layers(rbt_hip *h, int p0, int T) {
@@ -1958,8 +1963,8 @@ int rbt_hip_generate_stream(rbt_hip *h, const int32_t *prompt, int n_prompt, int
     for (int i = 0; i < 4 && e == hipSuccess; i++) e = HIP_TRY(hipEventCreate(&ev[i]));
     if (e == hipSuccess) e = HIP_TRY(hipEventRecord(ev[0], h->stream));
     // the prompt: n_prompt forwards, the last one with lm_head + argmax (the first generated token)
-    for (int p = 0; p < blocked && e == hipSuccess; p += kPromptBlock)
-        if (!prompt_block(h, p, std::min(kPromptBlock, blocked - p))) {
+    for (int p = 0; p < blocked && e == hipSuccess; p += h->prompt.tokens)
+        if (!prompt_block(h, p, std::min(h->prompt.tokens, blocked - p))) {
             cleanup();
             return 0;
         }

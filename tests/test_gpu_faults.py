@@ -212,3 +212,25 @@ print("RESULT " + json.dumps([failed, before, after, dev.expert_counts(8).tolist
     (failed, before, after, later), _ = prompt_child(body, "launch:13")
     assert "launch_dense_full" in failed and sum(before) == 10
     assert after == before and later == before
+
+
+PROMPT_BODY = """
+out = []
+for n in (34, 60, 64):
+    dev.generate(tokens[:n], 0)
+    logits, _ = dev.forward(int(tokens[n - 1]), n - 1, cfg.vocab, cfg.n_layers, cfg.top_k)
+    out.append(logits.tolist())
+print("RESULT " + json.dumps(out), flush=True)
+"""
+
+
+@pytest.mark.parametrize("nth,injected", [(7, True), (8, False)], ids=["smaller", "no-second"])
+def test_prompt_buffers(nth, injected):
+    """The 7th allocation (the model, the decode state and the workspace's four come first) is the first prompt's
+    buffer, for 64 positions: where it fails, the prompt runs in blocks of 32, with logits within the bar of
+    tests/test_gpu_prompt.py. Without that, longer prompts up to 65 tokens allocate nothing more."""
+    want, _ = prompt_child(PROMPT_BODY)
+    got, err = prompt_child(PROMPT_BODY, f"malloc:{nth}")
+    assert ("injecting a failure into hipMalloc(&b, off)" in err) == injected, err
+    for g, w in zip(got, want):
+        assert np.linalg.norm(np.subtract(g, w)) <= (1e-4 if injected else 0.0) * np.linalg.norm(w)
