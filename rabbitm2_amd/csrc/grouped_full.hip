@@ -245,7 +245,7 @@ __global__ __launch_bounds__(64 * kFullWaves * KS, 2) void grouped_full_kernel(c
     // (kFullAhead steps ahead): the LDS store waits for activations issued AS - 1 steps ago and not for
     // the weights behind them. Every load is issued in every step, past the last one too (no branches, so the
     // waits stay exact, and one copy of the steps: the code of a second, branching set for the last steps
-    // was fetched anew by every block, GUARDNEW).
+    // was fetched anew by every block).
     auto step = [&](auto jc, int c) {
         constexpr int J = decltype(jc)::value;
         store_a(aset[(J + 1) % AS], (c + 1) & 1, J & 1 ? 0u : kNegate);  // the buffer that step c - 1 read

@@ -1092,11 +1092,12 @@ inline bool batch_ok(int T, int D, int dtype, const void *W, const float *xb) {
            (D * esz) % 16 == 0 && D % 4 == 0;
 }
 
-// Tokens up to which a block per (token, row pair) beats the batch kernels (dim 2048, 64 experts, us):
-// f32 scalar order 32 tokens 8.8, 256 tokens 33.7 (batch kernel: 300 tokens 33.6); f32 AVX2 order 32 tokens
-// 5.1, 256 tokens 17.9 (batch kernel: 27.4 and 26); bf16 scalar order 32 tokens 9.5, 256 tokens 30.8 (batch
-// kernel: 300 tokens 34.0). Before either: f32 scalar 200 tokens 36.1, bf16 scalar 512 tokens 43.7, 2000
-// tokens 155 (now 43.7).
+// Tokens up to which a block per (token, row pair) is taken before the batch kernels (dim 2048, 64 experts, us:
+// this at T tokens / the batch kernel at 257 / the general kernel, which both orders' calls ran on before or
+// would): f32 scalar 32 tokens 8.4 / - / 34.1, 256 tokens 29.1 / 31.5 / 37.0; f32 AVX2 32 tokens 4.3, 256
+// tokens 15.4 / 24.2 (its crossover lies higher); bf16 scalar 32 tokens 7.0 / - / 17.5, 160 tokens 19.1 / - /
+// 20.1, 256 tokens 26.5 / 31.9 / 23.2 (the general kernel, one round of blocks, is the faster one from ~170
+// tokens to 256; at 512 tokens 32.2 against its 42.8, at 2000 36.1 against 156).
 constexpr int kFewMaxTokens = 256;
 
 // The logits by the kernels above where they apply (else hipErrorNotSupported).
